@@ -525,16 +525,12 @@ template <typename T> constexpr int kPanelTiles = ScalarTraits<T>::is_complex ? 
 // Factor one diagonal tile in LDS (S: in G, out R; Xo: out R^{-1}) by wave 0.
 // Returns the bad pivot (0 = fine), uniform over the workgroup.
 template <typename T>
-__device__ inline int factor_diag(T (*S)[33], T (*Xo)[33], T* rowbuf) {
+__device__ inline int factor_diag(T (*S)[33], T (*Xo)[33]) {
   __shared__ int bad_s;
   if (threadIdx.x == 0) bad_s = 0;
   __syncthreads();
   if (threadIdx.x < 64) {
-    // complex tiles: the 2 x 2-blocked in-wave factorisation (the single-pass
-    // elimination needs more registers than a wave has)
-    int b;
-    if constexpr (ScalarTraits<T>::is_complex) b = wave_chol_inv32<T>(S, Xo);
-    else b = wave_chol_aug32<T>(S, Xo, rowbuf);
+    const int b = wave_chol_inv32<T>(S, Xo);
     if (threadIdx.x == 0) bad_s = b;
   }
   __syncthreads();
@@ -692,7 +688,7 @@ __device__ inline void y_task(const CholTileArgs& a, int K, int r, int half, T* 
 // lands in tA .. tC; complex data reuses the block's tiles and tF, and the
 // roles rotate every iteration).
 template <typename T>
-__device__ void chol_panel(const CholTileArgs& a, T (*lds)[TB][33], T* rowbuf) {
+__device__ void chol_panel(const CholTileArgs& a, T (*lds)[TB][33]) {
   T* G = reinterpret_cast<T*>(a.G);
   T* X = reinterpret_cast<T*>(a.X);
   const int nt = a.nt;
@@ -737,7 +733,7 @@ __device__ void chol_panel(const CholTileArgs& a, T (*lds)[TB][33], T* rowbuf) {
         mm32<T>(tC, tB, true, tB, false, -1.0, true);
       }
       stamp(K, 3 + h);
-      const int bad = factor_diag<T>(h ? tC : tA, h ? tD : tX, rowbuf);
+      const int bad = factor_diag<T>(h ? tC : tA, h ? tD : tX);
       if (bad != 0) {
         report_bad<T>(a, c0 + h, bad);
         return;
@@ -895,10 +891,9 @@ __global__ void __launch_bounds__(256) chol_tile_kernel(CholTileArgs a) {
   T(*tD)[33] = lds[3];
   T(*tE)[33] = lds[4];
   T(*tX)[33] = lds[5];
-  __shared__ __align__(16) T rowbuf[2 * TB];
   __shared__ int task_s;
   if (blockIdx.x == 0) {
-    chol_panel<T>(a, lds, rowbuf);
+    chol_panel<T>(a, lds);
     return;
   }
   T* G = reinterpret_cast<T*>(a.G);

@@ -117,58 +117,12 @@ __device__ __forceinline__ int step_lane(int c) {
   asm volatile("" : "+v"(c));
   return c;
 }
+__device__ __forceinline__ void order_after(zd& v, double dep) { asm volatile("" : "+v"(v.x), "+v"(v.y) : "v"(dep)); }
 __device__ __forceinline__ void order_after(zd& v, const zd& dep) {
   asm volatile("" : "+v"(v.x), "+v"(v.y) : "v"(dep.x));
 }
-// An index (zero) that appears to depend on `dep`: a load through it cannot
-// be issued before `dep` is computed.
-__device__ __forceinline__ void index_after(int& z, double dep) { asm volatile("" : "+v"(z) : "v"(dep)); }
-__device__ __forceinline__ void index_after(int& z, const zd& dep) {
-  asm volatile("" : "+v"(z) : "v"(dep.x), "v"(dep.y));
-}
-
-// Cholesky with inverse of a 32 x 32 Hermitian positive definite block, by
-// ONE wave (no workgroup barrier, no LDS traffic inside the factorisation):
-//   S (LDS, 32 x 33) holds the upper triangle on entry (rows/columns beyond the
-//   active size padded with the identity by the caller); on exit S = W (upper,
-//   zero below) with S_in = W^H W, and Y = W^{-1} (upper, zero below).
-//   Returns 0, or j + 1 for the first pivot j that is not positive (uniform
-//   over the wave; S and Y are then unspecified).
-// Lane c (c = lane % 32; lanes 32..63 mirror lanes 0..31) keeps column c of W
-// and of Y in registers; row entries of other columns come from lane
-// broadcasts (v_readlane), four at a time.  Cholesky step j: W(j, c) =
-// S(j, c) / d_j, then S(r, c) -= conj(W(j, r)) W(j, c) for r > j (entries
-// below the diagonal only receive the mirrored update and are ignored).
-// `dinv` of lane j receives 1 / W(j, j).
-template <typename T, int N, int J>
-__device__ __forceinline__ void cholN_step(T (&s)[N], int c0, int& bad, T& dinv) {
-  const int c = step_lane(c0);
-  const double d2 = s_re(rdl(s[J], J));
-  if (!bad && !(d2 > 0.0)) bad = J + 1;
-  const double rd = (d2 > 0.0) ? rsqrt_nr(d2) : 0.0;
-  const double d = d2 * rd;
-  dinv = sel(c == J, s_from_real<T>(rd), dinv);
-  const T w = sel(c > J, s_scale(s[J], rd), sel(c == J, s_from_real<T>(d), s_zero(T())));
-  s[J] = w;
-  T src = w;
-#pragma unroll
-  for (int r0 = J + 1; r0 < N; r0 += kBc<T>) {
-    T b[kBc<T>];
-#pragma unroll
-    for (int u = 0; u < kBc<T>; ++u) b[u] = (r0 + u < N) ? rdl(src, r0 + u) : s_zero(T());
-#pragma unroll
-    for (int u = 0; u < kBc<T>; ++u)
-      if (r0 + u < N) s[r0 + u] = s_sub(s[r0 + u], s_mul(s_conj(b[u]), w));
-    order_after(src, s[r0]);
-  }
-}
-template <typename T, int N, int... Js>
-__device__ __forceinline__ void cholN_steps(T (&s)[N], int c, int& bad, T& dinv, std::integer_sequence<int, Js...>) {
-  (cholN_step<T, N, Js>(s, c, bad, dinv), ...);
-}
-
-// Inverse Y of an upper triangular N x N block U held by lanes as above
-// (lane c: s[r] = U(r, c)), `dinv` of lane r = 1 / U(r, r).  Rows from the
+// Inverse Y of an upper triangular N x N block U, lane c holding column c
+// (s[r] = U(r, c)), `dinv` of lane r = 1 / U(r, r).  Rows from the
 // bottom: Y(r, c) = (delta_rc - sum_{k > r} U(r, k) Y(k, c)) / U(r, r).
 template <typename T, int N, int I>
 __device__ __forceinline__ void trinvN_row(T (&y)[N], const T (&s)[N], const T& dinv, int c0) {
@@ -199,12 +153,6 @@ __device__ __forceinline__ void trinvN_rows(T (&y)[N], const T (&s)[N], const T&
                                             std::integer_sequence<int, Is...>) {
   (trinvN_row<T, N, Is>(y, s, dinv, c), ...);
 }
-template <typename T, int... Is>
-__device__ __forceinline__ void trinv32_rows(T (&y)[32], const T (&s)[32], const T& dinv, int c,
-                                             std::integer_sequence<int, Is...> seq) {
-  trinvN_rows<T, 32>(y, s, dinv, c, seq);
-}
-
 // Inverse Z of a unit lower triangular N x N block L (lane c: s[r] = L(r, c)
 // for r > c), rows from the top: Z(r, c) = delta_rc - sum_{c <= k < r} L(r, k) Z(k, c).
 template <typename T, int N, int R>
@@ -275,146 +223,249 @@ __device__ __forceinline__ void wave_mm16(T (*D)[33], const T (*A)[33], const T 
   }
 }
 
-// Cholesky with inverse of a 16 x 16 diagonal block (rows / columns r0..r0+15
-// of S and Y) by one wave, lane c (c = lane % 16) holding column c; W and
-// W^{-1} (upper, zero below) replace the block of S and fill the block of Y.
-template <typename T>
-__device__ __forceinline__ int wave_chol_inv16(T (*S)[33], T (*Y)[33], int r0) {
-  const int l = lane_id();
-  const int c = l & 15;
-  const bool writer = l < 16;
-  T s[16];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const T v = S[r0 + r][r0 + c];
-    s[r] = sel(r <= c, v, s_zero(T()));
+// ---------------------------------------------------------------------------
+// One-wave elimination of [s | x] by 16 pivots.  A 16-lane row of the wave is
+// one DPP row, so the pivot row's entry r (held by lane r) reaches all its
+// lanes as the DPP source of the multiply-add itself (row_newbcast, the one
+// DPP control that 64-bit operations take): no LDS round trip, no readlane.
+// ---------------------------------------------------------------------------
+
+// v of lane K of each 16-lane row, in all lanes of that row.
+template <int K> __device__ __forceinline__ double row_bcast(double v) {
+  const long u = __builtin_bit_cast(long, v), z = 0;
+  const long r = __builtin_amdgcn_update_dpp(z, u, 0x150 + K, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, r);
+}
+
+// s -= conj(b_R) ws, x -= conj(b_R) wx with b_R = b of lane R of the row.  A
+// VGPR may be a DPP source from two instructions after its write: ws depends
+// on the reciprocal of b's pivot (elim16_step), so b was written earlier than
+// that and the asm needs no wait of its own.
+template <int R>
+__device__ __forceinline__ void elim_row(double& s, double& x, double b, double ws, double wx) {
+  asm("v_fmac_f64_dpp %0, -%2, %3 row_newbcast:%c5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, -%2, %4 row_newbcast:%c5 row_mask:0xf bank_mask:0xf"
+      : "+v"(s), "+v"(x)
+      : "v"(b), "v"(ws), "v"(wx), "n"(R));
+}
+template <int R>
+__device__ __forceinline__ void elim_row(zd& s, zd& x, const zd& b, const zd& ws, const zd& wx) {
+  asm("v_fmac_f64_dpp %0, -%4, %6 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, -%4, %7 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %2, -%4, %8 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %3, -%4, %9 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, -%5, %7 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %5, %6 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %2, -%5, %9 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %3, %5, %8 row_newbcast:%c10 row_mask:0xf bank_mask:0xf"
+      : "+v"(s.x), "+v"(s.y), "+v"(x.x), "+v"(x.y)
+      : "v"(b.x), "v"(b.y), "v"(ws.x), "v"(ws.y), "v"(wx.x), "v"(wx.y), "n"(R));
+}
+// Step K: with the pivot d = s[K] of lane K and the pivot row b = s[K],
+//   s[r] -= conj(b_r) s[K] / d,  x[r] -= conj(b_r) x[K] / d   (r > K).
+// 1 / d is v_rcp_f64's y with its third-order correction, y (1 + e + e^2) with
+// e = 1 - d y (|e| about 2^-23, so the cubic remainder is far below one ulp).
+// Row K + 1, which holds the next pivot, is updated first, and the next
+// pivot's reciprocal is formed between the other rows' updates (order_after
+// keeps it there), so that the serial chain runs under them.
+struct ElimPivot {
+  double d, y, e, t, inv;
+};
+template <typename T, int K, int R0, int R1>
+__device__ __forceinline__ void elim16_rows(T (&s)[16], T (&x)[16], const T& b, const T& ws, const T& wx) {
+  if constexpr (R0 < R1) {
+    elim_row<R0>(s[R0], x[R0], b, ws, wx);
+    elim16_rows<T, K, R0 + 1, R1>(s, x, b, ws, wx);
   }
-  int bad = 0;
-  T dinv = s_zero(T());
-  cholN_steps<T, 16>(s, c, bad, dinv, std::make_integer_sequence<int, 16>{});
-#pragma unroll
-  for (int r = 0; r < 16; ++r)
-    if (writer) S[r0 + r][r0 + c] = (r <= c) ? s[r] : s_zero(T());
-  T y[16];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) y[r] = s_zero(T());
-  trinvN_rows<T, 16>(y, s, dinv, c, std::make_integer_sequence<int, 16>{});
-#pragma unroll
-  for (int r = 0; r < 16; ++r)
-    if (writer) Y[r0 + r][r0 + c] = y[r];
-  return bad;
+}
+template <typename T, int K>
+__device__ __forceinline__ void elim16_step(T (&s)[16], T (&x)[16], int c0, double& piv, ElimPivot& p) {
+  const T b = s[K];
+  T ws = s_scale(b, p.inv);
+  const T wx = s_scale(x[K], p.inv);
+  piv = sel(step_lane(c0) == K, p.d, piv);
+  if constexpr (K < 15) {
+    constexpr int n = 14 - K, R0 = K + 2, R1 = R0 + (n + 1) / 2, R2 = R1 + (16 - R1 + 2) / 3,
+                  R3 = R2 + (16 - R2 + 1) / 2;
+    elim_row<K + 1>(s[K + 1], x[K + 1], b, ws, wx);
+    p.d = row_bcast<K + 1>(s_re(s[K + 1]));
+    p.y = __builtin_amdgcn_rcp(p.d);
+    order_after(ws, p.y);
+    elim16_rows<T, K, R0, R1>(s, x, b, ws, wx);
+    p.e = fma(-p.d, p.y, 1.0);
+    order_after(ws, p.e);
+    elim16_rows<T, K, R1, R2>(s, x, b, ws, wx);
+    p.t = fma(p.e, p.e, p.e);
+    order_after(ws, p.t);
+    elim16_rows<T, K, R2, R3>(s, x, b, ws, wx);
+    p.inv = fma(p.y, p.t, p.y);
+    order_after(ws, p.inv);
+    elim16_rows<T, K, R3, 16>(s, x, b, ws, wx);
+  }
+}
+template <typename T, int... Ks>
+__device__ __forceinline__ void elim16_steps(T (&s)[16], T (&x)[16], int c, double& piv,
+                                             std::integer_sequence<int, Ks...>) {
+  ElimPivot p;
+  p.d = row_bcast<0>(s_re(s[0]));
+  p.y = __builtin_amdgcn_rcp(p.d);
+  p.e = fma(-p.d, p.y, 1.0);
+  p.t = fma(p.e, p.e, p.e);
+  p.inv = fma(p.y, p.t, p.y);
+  (elim16_step<T, Ks>(s, x, c, piv, p), ...);
+}
+template <typename T, int... Ks>
+__device__ __forceinline__ void elim16_scale(T (&x)[16], double rs, std::integer_sequence<int, Ks...>) {
+  ((x[Ks] = s_scale(x[Ks], row_bcast<Ks>(rs))), ...);
+}
+
+// Lane c of every 16-lane row holds column c of the Hermitian block A in s
+// (rows r <= c; the others hold anything: they only reach their own lane's
+// s) and a column of any right-hand side B in x; on exit x = R^{-H} B with
+// A = R^H R (B = A's upper triangle gives R, and B = I gives R^{-H}).
+// Returns 0, or k + 1 for the first pivot k that is not positive (uniform;
+// x is then unspecified).
+template <typename T> __device__ __forceinline__ int wave_elim16(T (&s)[16], T (&x)[16], int c) {
+  double piv = 1.0;
+  elim16_steps<T>(s, x, c, piv, std::make_integer_sequence<int, 16>{});
+  const unsigned m = (unsigned)__ballot(!(piv > 0.0)) & 0xffffu;
+  elim16_scale<T>(x, rsqrt_nr(piv), std::make_integer_sequence<int, 16>{});
+  return m ? __builtin_ctz(m) + 1 : 0;
 }
 
 // Cholesky with inverse of a 32 x 32 Hermitian positive definite block, by
 // ONE wave (no workgroup barrier):
 //   S (LDS, 32 x 33) holds the upper triangle on entry (rows/columns beyond the
 //   active size padded with the identity by the caller); on exit S = W (upper,
-//   zero below) with S_in = W^H W, and Y = W^{-1} (upper, zero below).
+//   zero below) with S_in = W^H W, and Y = W^{-1} (upper, zero below).  The
+//   padding column of S (index 32) is used as scratch.
 //   Returns 0, or j + 1 for the first pivot j that is not positive (uniform
 //   over the wave; S and Y are then unspecified).
-// 2 x 2 blocks of 16: W11, Y11 in-wave; W12 = Y11^H S12; S22 -= W12^H W12;
-// W22, Y22 in-wave; Y12 = -Y11 (W12 Y22) -- the off-diagonal products on MFMA.
-template <typename T>
-__device__ __forceinline__ int wave_chol_inv32(T (*S)[33], T (*Y)[33]) {
-  auto blk = [](T (*M)[33], int r0, int c0) { return reinterpret_cast<T (*)[33]>(&M[r0][c0]); };
-  int bad = wave_chol_inv16<T>(S, Y, 0);
-  wave_mm16<T, true>(blk(S, 0, 16), blk(Y, 0, 0), blk(S, 0, 16), 1.0, false);     // W12 = Y11^H S12
-  wave_mm16<T, true>(blk(S, 16, 16), blk(S, 0, 16), blk(S, 0, 16), -1.0, true);   // S22 -= W12^H W12
-  const int b2 = wave_chol_inv16<T>(S, Y, 16);
-  if (bad == 0 && b2 != 0) bad = 16 + b2;
-  wave_mm16<T, false>(blk(Y, 0, 16), blk(S, 0, 16), blk(Y, 16, 16), 1.0, false);  // P = W12 Y22
-  wave_mm16<T, false>(blk(Y, 0, 16), blk(Y, 0, 0), blk(Y, 0, 16), -1.0, false);   // Y12 = -Y11 P
-  const int l = lane_id();
-  for (int e = l; e < 256; e += 64) {
-    const int i = e & 15, j = e >> 4;
-    S[16 + i][j] = s_zero(T());
-    Y[16 + i][j] = s_zero(T());
+// Two eliminations by 16 pivots; all four 16-lane rows of the wave keep the
+// diagonal block in s and eliminate a right-hand side each in x:
+//   of S11:  I -> W11^{-H} = Y11^H,  S12 -> W12,  S11 -> W11,  0
+//   then on MFMA  S22 -= W12^H W12,  H = W12^H Y11^H
+//   of S22:  I -> Y22^H,  -H -> Y12^H,  S22 -> W22,  0
+// (W^{-H} = [Y11^H 0; -Y22^H H, Y22^H]).  The zeros become the lower left
+// blocks of W and Y, and the columns of I are read from the padding column of
+// S, so that every lane loads and stores through one pointer without selects:
+// one wave issues an instruction about every five cycles, and their number is
+// what this costs.  Measured (one wave alone): 7.6e3 cycles Float64, 17.7e3
+// ComplexF64 (of which the two eliminations 4.1e3 and 11e3), against 15.4e3 for
+// an elimination of the whole [S | I] with its pivot rows through LDS
+// (Float64) and 40.5e3 for 16 x 16 factorisations with readlane broadcasts
+// (ComplexF64).
+template <typename T> __device__ __forceinline__ int wave_chol_inv32(T (*S)[33], T (*Y)[33]) {
+  const int l = lane_id(), c = l & 15, q = l >> 4;
+  // loads of one array are issued together (left alone, the scheduler waits
+  // for each before the next)
+  auto pin = [](T (&a)[16]) {
+    double* p = reinterpret_cast<double*>(&a[0]);
+    constexpr int ND = 16 * sizeof(T) / sizeof(double);
+#pragma unroll
+    for (int h = 0; h < ND; h += 8)
+      asm volatile("" : "+v"(p[h]), "+v"(p[h + 1]), "+v"(p[h + 2]), "+v"(p[h + 3]), "+v"(p[h + 4]), "+v"(p[h + 5]),
+                        "+v"(p[h + 6]), "+v"(p[h + 7]));
+  };
+  // zeros below the diagonal of W's 16 x 16 block at D: the columns left of
+  // the diagonal in row c, four per 16-lane row; the others write to the
+  // padding column of Y.  A complex factor's diagonal is made exactly real.
+  auto clear_lower = [&](T* D) {
+    if constexpr (ScalarTraits<T>::is_complex)
+      if (q == 0) D[34 * c].y = 0.0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = 4 * q + u;
+      T* p = j < c ? D + 33 * c + j : &Y[c][32];
+      *p = s_zero(T());
+    }
+  };
+  if (l < 32) S[l][32] = l == 15 ? s_one(T()) : s_zero(T());
+  wave_lds_sync();
+  const T* eye = &S[15 - c][32];   // rows 0 .. 15: column c of I
+  const T* none = &S[16][32];      // zeros
+  T s[16], x[16];
+  {
+    const T* px = q == 0 ? eye : q == 1 ? &S[0][16 + c] : q == 2 ? &S[0][c] : none;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = S[r][c];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) x[r] = px[33 * r];
+    pin(s);
+    pin(x);
+  }
+  int bad = wave_elim16<T>(s, x, c);
+  if (q == 0) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) Y[c][r] = s_conj(x[r]);
+  } else {
+    T* p = q == 1 ? &S[0][16 + c] : q == 2 ? &S[0][c] : &S[16][c];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) p[33 * r] = x[r];
   }
   wave_lds_sync();
-  return bad;
-}
-
-// Cholesky factorisation with inverse of a 32 x 32 Hermitian positive definite
-// tile by ONE wave, eliminating [G | I] in a single pass:
-//   S (LDS, 32 x 33): upper triangle of G on entry (strict lower part not
-//   read); on exit R (upper, zero below) with G = R^H R.
-//   Y (LDS, 32 x 33): on exit X = R^{-1} (upper, zero below).
-//   row: LDS scratch of 64 elements, 16-byte aligned (two pivot-row buffers).
-// Lane c < 32 keeps column c of G, lane 32 + c column c of the identity (that
-// becomes M = R^{-H}, lower).  Step k, with the pivot d = G'(k, k) read from
-// lane k and the raw pivot row G'(k, r) in LDS:
-//   x[r] -= conj(G'(k, r)) x[k] / d  (r > k),   x[k] <- x[k] / sqrt(d)
-// is the same instruction stream for both halves: the Cholesky update
-// G'(r, c) -= conj(R(k, r)) R(k, c) and the forward elimination of the
-// identity Z(r, c) -= conj(R(k, r)) M(k, c).
-// Software pipelined: the update of row k + 1 and its publication as the next
-// pivot row (the dependency chain: one LDS round trip, the pivot reciprocal
-// and two FMAs per column) are issued before the bulk of the step's updates,
-// which then overlap the next round trip; the pivot rows alternate between
-// two buffers so the bulk reads of step k never race the write of step k + 1.
-// Returns 0, or k + 1 for the first pivot k that is not positive (S and Y are
-// then unspecified).
-template <typename T>
-__device__ __forceinline__ int wave_chol_aug32(T (*S)[33], T (*Y)[33], T* row) {
-  const int l = lane_id();
-  const int c = l & 31;
-  const bool lo = l < 32;
-  T x[32];
+  {
+    // the accumulators start from S22 and 0 and subtract the products, the last four rows first
+    v4d gr, hr = {0.0, 0.0, 0.0, 0.0}, gi = {0.0, 0.0, 0.0, 0.0}, hi = {0.0, 0.0, 0.0, 0.0};
+    T w[4], h[4];
 #pragma unroll
-  for (int r = 0; r < 32; ++r) {
-    const T v = S[r][c];
-    x[r] = lo ? (r <= c ? v : s_zero(T())) : (r == c ? s_one(T()) : s_zero(T()));
-  }
-  // `row` is read at wave-uniform addresses; an index offset the compiler
-  // cannot see is zero keeps those values in vector registers (as uniform
-  // values they would be moved to scalar registers and hoisted, and spill).
-  int zoff = 0;
-  asm volatile("" : "+v"(zoff));
-  if (lo) row[c] = x[0];
-  int bad = 0;
+    for (int u = 0; u < 4; ++u) {
+      w[u] = S[4 * u + q][16 + c];
+      h[u] = Y[c][4 * u + q];
+      const T old = S[16 + 4 * u + q][16 + c];
+      gr[u] = s_re(old);
+      if constexpr (ScalarTraits<T>::is_complex) gi[u] = s_im(old);
+    }
+    clear_lower(&S[0][0]);
 #pragma unroll
-  for (int k = 0; k < 32; ++k) {
-    T* cur = row + (k & 1) * 32;
-    T* nxt = row + ((k + 1) & 1) * 32;
-    wave_lds_sync();  // the pivot row of step k is visible
-    // the whole pivot row in one burst of 16-byte reads (issued together, so
-    // their latency is paid once per step; read one at a time, as the
-    // scheduler otherwise does, they cost most of the step)
-    T rv[32];
-    {
-      using V2 = typename ScalarTraits<T>::vec2;
-      const V2* cv = reinterpret_cast<const V2*>(cur + zoff);
-#pragma unroll
-      for (int r = (k + 1) & ~1; r < 32; r += 2) {
-        const V2 v = cv[r / 2];
-        rv[r] = ScalarTraits<T>::lo(v);
-        rv[r + 1] = ScalarTraits<T>::hi(v);
+    for (int u = 3; u >= 0; --u) {
+      gr = mfma_f64(-s_re(w[u]), s_re(w[u]), gr);
+      hr = mfma_f64(-s_re(w[u]), s_re(h[u]), hr);
+      if constexpr (ScalarTraits<T>::is_complex) {
+        // - conj(w) w and - conj(w) conj(h)
+        gi = mfma_f64(-s_re(w[u]), s_im(w[u]), gi);
+        hi = mfma_f64(s_re(w[u]), s_im(h[u]), hi);
+        gr = mfma_f64(-s_im(w[u]), s_im(w[u]), gr);
+        hr = mfma_f64(s_im(w[u]), s_im(h[u]), hr);
+        gi = mfma_f64(s_im(w[u]), s_re(w[u]), gi);
+        hi = mfma_f64(s_im(w[u]), s_re(h[u]), hi);
       }
     }
-    const T raw = x[k];
-    const double d = s_re(rdl(raw, k));
-    bad = bad ? bad : (d > 0.0 ? 0 : k + 1);
-    const double dd = (d > 0.0) ? d : 1.0;
-    const double inv = recip_nr(dd);
-    const T w = s_scale(raw, inv);
-    if (k < 31) {
-      // the chain: row k + 1, published as the next pivot row
-      x[k + 1] = s_sub(x[k + 1], s_mul(s_conj(rv[k + 1]), w));
-      if (lo) nxt[c] = x[k + 1];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if constexpr (ScalarTraits<T>::is_complex) {
+        S[16 + 4 * u + q][16 + c] = mkz(gr[u], gi[u]);
+        Y[4 * u + q][16 + c] = mkz(hr[u], hi[u]);
+      } else {
+        S[16 + 4 * u + q][16 + c] = gr[u];
+        Y[4 * u + q][16 + c] = hr[u];
+      }
     }
-#pragma unroll
-    for (int r = k + 2; r < 32; ++r) x[r] = s_sub(x[r], s_mul(s_conj(rv[r]), w));
-    // one step of overlap at most: step k + 1's chain may run ahead of this
-    // bulk, but row k + 3 (the chain of step k + 2) waits for all of it
-#pragma unroll
-    for (int r = k + 4; r < 32; ++r) order_after(x[k + 3], x[r]);
-    x[k] = s_scale(raw, rsqrt_nr(dd));
   }
+  wave_lds_sync();
+  {
+    const T* px = q == 0 ? eye : q == 1 ? &Y[0][16 + c] : q == 2 ? &S[16][16 + c] : none;
 #pragma unroll
-  for (int r = 0; r < 32; ++r) {
-    if (lo) S[r][c] = (r <= c) ? x[r] : s_zero(T());
-    else Y[c][r] = (r >= c) ? s_conj(x[r]) : s_zero(T());
+    for (int r = 0; r < 16; ++r) s[r] = S[16 + r][16 + c];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) x[r] = px[33 * r];
+    pin(s);
+    pin(x);
   }
+  wave_lds_sync();
+  const int b2 = wave_elim16<T>(s, x, c);
+  if (bad == 0 && b2 != 0) bad = 16 + b2;
+  if (q < 2) {
+    T* p = q == 0 ? &Y[16 + c][16] : &Y[c][16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) p[r] = s_conj(x[r]);
+  } else {
+    T* p = q == 2 ? &S[16][16 + c] : &Y[16][c];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) p[33 * r] = x[r];
+  }
+  wave_lds_sync();
+  clear_lower(&S[16][16]);
   wave_lds_sync();
   return bad;
 }
