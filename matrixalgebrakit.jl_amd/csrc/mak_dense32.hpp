@@ -237,10 +237,16 @@ template <int K> __device__ __forceinline__ double row_bcast(double v) {
   return __builtin_bit_cast(double, r);
 }
 
+template <int K> __device__ __forceinline__ zd row_bcast(const zd& v) {
+  return mkz(row_bcast<K>(v.x), row_bcast<K>(v.y));
+}
+
 // s -= conj(b_R) ws, x -= conj(b_R) wx with b_R = b of lane R of the row.  A
-// VGPR may be a DPP source from two instructions after its write: ws depends
-// on the reciprocal of b's pivot (elim16_step), so b was written earlier than
-// that and the asm needs no wait of its own.
+// VGPR may be a DPP source from two instructions after its write.  b is the
+// step's pivot row, last written by the previous step's first update, and ws
+// depends on the reciprocal of its pivot, so no wait is needed here (one
+// s_nop per row costs a sixth of the whole factorisation); elim16_step fixes
+// b in its registers behind a wait of its own.
 template <int R>
 __device__ __forceinline__ void elim_row(double& s, double& x, double b, double ws, double wx) {
   asm("v_fmac_f64_dpp %0, -%2, %3 row_newbcast:%c5 row_mask:0xf bank_mask:0xf\n\t"
@@ -268,6 +274,8 @@ __device__ __forceinline__ void elim_row(zd& s, zd& x, const zd& b, const zd& ws
 // Row K + 1, which holds the next pivot, is updated first, and the next
 // pivot's reciprocal is formed between the other rows' updates (order_after
 // keeps it there), so that the serial chain runs under them.
+__device__ __forceinline__ void dpp_source(double& b) { asm("s_nop 1" : "+v"(b)); }
+__device__ __forceinline__ void dpp_source(zd& b) { asm("s_nop 1" : "+v"(b.x), "+v"(b.y)); }
 struct ElimPivot {
   double d, y, e, t, inv;
 };
@@ -280,7 +288,8 @@ __device__ __forceinline__ void elim16_rows(T (&s)[16], T (&x)[16], const T& b, 
 }
 template <typename T, int K>
 __device__ __forceinline__ void elim16_step(T (&s)[16], T (&x)[16], int c0, double& piv, ElimPivot& p) {
-  const T b = s[K];
+  T b = s[K];
+  dpp_source(b);
   T ws = s_scale(b, p.inv);
   const T wx = s_scale(x[K], p.inv);
   piv = sel(step_lane(c0) == K, p.d, piv);
