@@ -55,22 +55,67 @@ constexpr double kBf16CorrMaxE = 5e-14;
 
 struct CQ2Layout {
   size_t offQ1, offG, offE, offX, offU, offW, offT, offSl, offFlags, offPart, offSt, offXc, bytes;
-  int ks;    // split-K slices of the Gram products
+  int ks;    // split-K slices reserved for the Gram products
+  int kcap;  // slices that fit from offX on
   int ldxc;  // leading dimension of the Cholesky's copy of X1
 };
 
-// Split-K slices of an upper-triangle n x n Gram over m rows on 128 x 128
-// tiles: two workgroups per CU (about 512; one per CU leaves the MFMA waiting
-// on loads), slices of at least 256 rows.  At n = 1024, m = 8192: 36 tiles x
-// 14 slices, 190 us (45 TF/s on the upper-triangle count) against 300 us for
-// 64 x 64 tiles or one workgroup per CU.
-constexpr int kGramTile = 128;
+// Split-K slices that the workspace reserves for an upper-triangle n x n Gram
+// over m rows (about 512 workgroups of 128 x 128 tiles, slices of at least 256
+// rows); the Grams may use more where n x n buffers that are free then adjoin
+// them (gram_plan).
 int gram_slices(int m, int n) {
-  const int t = cdiv(n, kGramTile);
+  const int t = cdiv(n, 128);
   const int upper = t * (t + 1) / 2;
   int ks = (512 + upper / 2) / std::max(upper, 1);
   ks = std::min(ks, std::max(1, m / 256));
   return std::max(1, std::min(ks, 32));
+}
+
+// Tile and slice count of the Gram (slices: at most `cap`, of at least 64 rows,
+// since the slice sum reads them all).  A workgroup alone on its CU is bound by
+// the latency of its 16-deep steps (0.56, 0.97 and 2.7 us each on 32, 64 and
+// 128 tiles, against 0.11, 0.43 and 1.7 us of MFMA), so it takes many of them,
+// and small problems want short slices of small tiles.  Measured on Float64,
+// us, the best slice count of each tile (32 / 64 / 128):  n = 128, m = 1024:
+// 5 / 6 / 12;  256 x 2048: 9 / 11 / 18;  512 x 1024: 14 / 14 / 17;  512 x 8192:
+// 65 / 58 / 70;  768 x 1536: 32 / 28 / 32;  2048 x 2048: 212 / 177 / 189.  So 32
+// up to n = 256, 64 beyond, and about 3072 workgroups (2048 x 2048: 256 us with
+// 528, 181 with 2112, 177 with 3696).  A wide matrix that exceeds the L2 caches
+// (32 MB) is read n / tile times from beyond them: 128 tiles are faster there
+// inside a factorisation (1024 x 8192: 195 us against 221), two workgroups per
+// CU, the slice count that fills rounds of 512 best (2048 x 8192: 677 us with 7
+// slices, 930 with 4).
+struct GramPlan {
+  int tile, ks;
+};
+template <typename T> GramPlan gram_plan(int m, int n, int cap) {
+  GramPlan p;
+  cap = std::max(1, std::min(std::min(cap, 32), m / 64));
+  if (ScalarTraits<T>::is_complex) {  // 64 x 64 (or 32 x 32) by the dispatcher, two workgroups per CU
+    const int t = cdiv(n, 64);
+    p.tile = 0;
+    p.ks = std::min(std::max(gram_slices(m, n), 1024 / (t * (t + 1) / 2)), cap);
+    return p;
+  }
+  if (n > 768 && (size_t)m * n * sizeof(T) > ((size_t)32 << 20)) {
+    const int t = cdiv(n, 128), upper = t * (t + 1) / 2;
+    p.tile = 128;
+    p.ks = 1;
+    double best = cdiv(upper, 512);
+    for (int ks = 2; ks <= std::min(cap, 16); ++ks) {
+      const double r = (double)cdiv(upper * ks, 512) / ks;
+      if (r < 0.95 * best) {
+        best = r;
+        p.ks = ks;
+      }
+    }
+    return p;
+  }
+  p.tile = n <= 256 ? 32 : 64;
+  const int t = cdiv(n, p.tile);
+  p.ks = std::max(1, std::min(3072 / (t * (t + 1) / 2), cap));
+  return p;
 }
 
 template <typename T> CQ2Layout cq2_layout(int m, int n) {
@@ -82,13 +127,14 @@ template <typename T> CQ2Layout cq2_layout(int m, int n) {
   L.offQ1 = take((size_t)m * n * sizeof(T));
   L.offG = take(nn);
   L.offE = take(nn);
-  L.offX = take(nn);
   L.offU = take(nn);
+  L.offX = take(nn);  // X .. T are free while a Gram runs: its slices start here
   L.offW = take(nn);
   L.offT = take(nn);
-  // the Gram slices; later the packed operands of the BF16 / FP32 correction
+  // the rest of the Gram slices; later the packed operands of the BF16 / FP32 correction
   L.offSl = take(std::max(nn * L.ks, ScalarTraits<T>::is_complex ? gemm_lo_complex_workspace_bytes(m, n, n)
                                                                     : gemm_prec_workspace_bytes(m, n, n)));
+  L.kcap = (int)std::min<size_t>(64, (off - L.offX) / std::max<size_t>(nn, 1));
   L.offFlags = take(chol_tile_flag_ints(n) * sizeof(int));
   L.offPart = take(kRedWgs * sizeof(double));
   L.offSt = take(64 * sizeof(int));
@@ -111,8 +157,6 @@ template <typename T> GemmArgs gq(int M, int N, int K, const T* A, int64_t lda, 
   return g;
 }
 
-// G (n x n, upper triangle; the strict lower part is left unspecified) =
-// X^H X for X m x n: split-K slices then their sum.
 // G[upper] = sum of the ks slices (n x n each, upper triangles only).
 template <typename T>
 __global__ void __launch_bounds__(256) sum_upper_slices_kernel(const T* P, int ks, int n, T* G) {
@@ -134,12 +178,13 @@ __global__ void __launch_bounds__(256) sum_upper_slices_kernel(const T* P, int k
   }
 }
 
-// The split-K slices of the upper Gram X^H X; returns their count.
-template <typename T> int gram_upper_slices(const T* X, int64_t ldx, int m, int n, T* slices, int ks, hipStream_t s) {
+// The split-K slices (at most cap) of the upper Gram X^H X; returns their count.
+template <typename T> int gram_upper_slices(const T* X, int64_t ldx, int m, int n, T* slices, int cap, hipStream_t s) {
+  const GramPlan p = gram_plan<T>(m, n, cap);
   GemmArgs g = gq<T>(n, n, m, X, ldx, X, ldx, slices, n, 1.0, 0.0, 0);
   g.upperC = 1;
-  if (!ScalarTraits<T>::is_complex) g.tile = kGramTile;
-  g.kchunk = cdiv(cdiv(m, ks), 16) * 16;
+  if (!ScalarTraits<T>::is_complex) g.tile = p.tile;
+  g.kchunk = cdiv(cdiv(m, p.ks), 16) * 16;
   g.ksplit = cdiv(m, g.kchunk);
   g.splitStride = (int64_t)n * n;
   gemm<T>(OP_C, OP_N, g, s);
@@ -147,8 +192,8 @@ template <typename T> int gram_upper_slices(const T* X, int64_t ldx, int m, int 
 }
 
 template <typename T>
-void gram_upper(const T* X, int64_t ldx, int m, int n, T* G, T* slices, int ks, hipStream_t s) {
-  const int nsl = gram_upper_slices<T>(X, ldx, m, n, slices, ks, s);
+void gram_upper(const T* X, int64_t ldx, int m, int n, T* G, T* slices, int cap, hipStream_t s) {
+  const int nsl = gram_upper_slices<T>(X, ldx, m, n, slices, cap, s);
   const int64_t tot = (int64_t)n * (n + 1) / 2;
   hipLaunchKernelGGL((sum_upper_slices_kernel<T>), dim3((unsigned)std::min<int64_t>(cdiv64(tot, 256), 2048)), dim3(256),
                      0, s, slices, nsl, n, G);
@@ -312,15 +357,15 @@ void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q,
   zero_ints(st, 8, s);  // st[2]: the Cholesky's info
   // pass 1: Q1 = A X1 inside the Cholesky launch, column block by column
   // block as X1 becomes final
-  gram_upper<T>(A, lda, m, n, G, Sl, L.ks, s);
+  gram_upper<T>(A, lda, m, n, G, X, L.kcap, s);
   {
     const CholRightProduct rp{A, lda, Q1, m, m, ws + L.offXc, L.ldxc};
     chol_tile_factor<T>(G, n, n, X, n, flags, st + 2, 0, s, 0, nullptr, &rp);
   }
   // pass 2: G2 = I + E (slices summed with U1 = up(E) and ||E||_F in one
   // sweep), the decision, and W2, W2^{-1} in closed form
-  const int ks2 = gram_upper_slices<T>(Q1, m, m, n, Sl, L.ks, s);
-  hipLaunchKernelGGL((cq2_sum_up_kernel<T>), dim3(kRedWgs), dim3(256), 0, s, Sl, ks2, n, E, U, part);
+  const int ks2 = gram_upper_slices<T>(Q1, m, m, n, X, L.kcap, s);
+  hipLaunchKernelGGL((cq2_sum_up_kernel<T>), dim3(kRedWgs), dim3(256), 0, s, X, ks2, n, E, U, part);
   hipLaunchKernelGGL(cq2_decide_kernel, dim3(1), dim3(256), 0, s, part, kRedWgs, st + 2, 1, st);
   // second order (st[1] == 1): U = up(E - U1^H U1), U2 = U U
   {
