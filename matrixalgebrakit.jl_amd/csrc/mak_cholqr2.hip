@@ -428,6 +428,12 @@ template <typename T> T* cholqr2_scratch(char* ws, int m, int n) {
   return reinterpret_cast<T*>(ws + cq2_layout<T>(m, n).offQ1);
 }
 
+template <typename T> Cholqr2Buffers<T> cholqr2_buffers(char* ws, int m, int n) {
+  const CQ2Layout L = cq2_layout<T>(m, n);
+  auto at = [&](size_t off) { return reinterpret_cast<T*>(ws + off); };
+  return Cholqr2Buffers<T>{at(L.offQ1), {at(L.offE), at(L.offU), at(L.offX), at(L.offW), at(L.offT)}};
+}
+
 template size_t cholqr2_workspace_bytes<double>(int, int);
 template size_t cholqr2_workspace_bytes<zd>(int, int);
 template void cholqr2_enqueue<double>(hipStream_t, int, int, const double*, int64_t, double*, int64_t, double*,
@@ -435,6 +441,8 @@ template void cholqr2_enqueue<double>(hipStream_t, int, int, const double*, int6
 template void cholqr2_enqueue<zd>(hipStream_t, int, int, const zd*, int64_t, zd*, int64_t, zd*, int64_t, char*);
 template int* cholqr2_status<double>(char*, int, int);
 template int* cholqr2_status<zd>(char*, int, int);
+template Cholqr2Buffers<double> cholqr2_buffers<double>(char*, int, int);
+template Cholqr2Buffers<zd> cholqr2_buffers<zd>(char*, int, int);
 template double* cholqr2_scratch<double>(char*, int, int);
 template zd* cholqr2_scratch<zd>(char*, int, int);
 

@@ -70,6 +70,19 @@ void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q,
                      char* ws);
 template <typename T> int* cholqr2_status(char* ws, int m, int n);
 template <typename T> T* cholqr2_scratch(char* ws, int m, int n);
+// Workspace of a cholqr2_enqueue call that is free once its launches are
+// enqueued (later launches of the same stream may overwrite it).
+template <typename T> struct Cholqr2Buffers {
+  T* mn;     // m x n
+  T* nn[5];  // n x n each
+};
+template <typename T> Cholqr2Buffers<T> cholqr2_buffers(char* ws, int m, int n);
+
+// The Householder QR's signs and trailing columns from the CholeskyQR2
+// factors (mak_qtrail.hip), enqueued after cholqr2_enqueue with its workspace.
+template <typename T>
+void qr_trailing_enqueue(hipStream_t s, int m, int n, T* Q, int64_t ldq, T* R, int64_t ldr, int full, int positive,
+                         char* cw);
 
 template <typename T> size_t polar_workspace_bytes(int m, int n);
 template <typename T>

@@ -70,6 +70,8 @@ template <typename T> TreePlan plan_tree(int H, int nbc, size_t base) {
 
 // Panels at least this tall go through the CholeskyQR2 path first.
 constexpr int kCholQrMinRows = 64;
+// Columns from which the whole-matrix CholeskyQR2 path is tried first.
+constexpr int kCholQr2MinN = 64;
 
 template <typename T> struct QrLayout {
   size_t offTpanels = 0;  // NB*NB per panel
@@ -158,7 +160,7 @@ template <typename T> QrLayout<T> qr_layout(int m, int n, int qcols) {
   }
   L.offQs = off;
   off += align256((size_t)m * minmn * sizeof(T));
-  if (qcols == minmn && cholqr2_eligible(m, n)) {
+  if (cholqr2_eligible(m, n) && (qcols == minmn || n >= kCholQr2MinN)) {
     L.offCq2 = off;
     off += align256(cholqr2_workspace_bytes<T>(m, n));
   }
@@ -395,9 +397,6 @@ void geqrf_blocked(T* A, int64_t lda, int m, int n, char* ws, size_t qcols, hipS
   if (geqrf_enqueue<T>(A, lda, m, n, ws, qcols, s)) geqrf_finish<T>(A, lda, m, n, ws, qcols, s);
 }
 
-// Columns from which the whole-matrix CholeskyQR2 path is tried first.
-constexpr int kCholQr2MinN = 64;
-
 // out (kg x N, ld kg) = V^H X for V = Vc (rows x kg, ld ldv): split-K
 // product into the Wp slices, then their sum.
 template <typename T>
@@ -607,19 +606,31 @@ int qr_driver(hipStream_t s, int full, int m, int n, T* A, int64_t lda, T* Q, in
   }
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &cs) != hipSuccess) cs = hipStreamCaptureStatusActive;
-  // qr_compact!(positive = true): whole-matrix CholeskyQR2 first (A is only
-  // read; a rejected input goes on to the Householder path below)
-  if (L.offCq2 && positive && !inplace && Tout == nullptr && n >= kCholQr2MinN && cs == hipStreamCaptureStatusNone) {
+  // Whole-matrix CholeskyQR2 first (A is only read; a rejected input goes on
+  // to the Householder path below); the trailing columns of qr_full! and the
+  // Householder signs of positive = false follow from its Q.  The signs are
+  // those of the panel path: for a square matrix the last column's reflector
+  // is the identity there, and for complex data its last panels (under
+  // kCholQrMinRows rows) take real signs, so those forms stay on it.
+  const bool signs = !positive || (full && m > n);
+  T* Qd = inplace ? reinterpret_cast<T*>(ws + L.offQs) : Q;
+  const int64_t ldqd = inplace ? m : ldq;
+  const bool whole = L.offCq2 && Tout == nullptr && n >= kCholQr2MinN &&
+                     cs == hipStreamCaptureStatusNone &&
+                     (!signs || (m > n && (!ScalarTraits<T>::is_complex || m - (n - 1) / NB * NB >= kCholQrMinRows)));
+  if (whole) {
     char* cw = ws + L.offCq2;
-    cholqr2_enqueue<T>(s, m, n, A, lda, Q, ldq, R, ldr, cw);
+    cholqr2_enqueue<T>(s, m, n, A, lda, Qd, ldqd, R, ldr, cw);
+    if (signs) qr_trailing_enqueue<T>(s, m, n, Qd, ldqd, R, ldr, full, positive, cw);
     int st = 0;
     if (hipMemcpyAsync(&st, cholqr2_status<T>(cw, m, n), sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
       return 1;
-    if (st == 1) return hipGetLastError() == hipSuccess ? 0 : 1;
+    if (st == 1) {
+      if (inplace) copy_mat<T>(m, qcols, Qd, ldqd, Q, ldq, s);
+      return hipGetLastError() == hipSuccess ? 0 : 1;
+    }
   }
-  T* Qd = inplace ? reinterpret_cast<T*>(ws + L.offQs) : Q;
-  const int64_t ldqd = inplace ? m : ldq;
   // Q, R and the tape are formed before the CholeskyQR2 flag is read, so the
   // one synchronisation does not leave the GPU waiting for the host; they are
   // formed again in the (rare) case that a panel was refactored.  In the
