@@ -21,7 +21,8 @@
  *       mak_*_polar_*      once for ||A||_F, then once per QDWH iteration
  *                          (convergence and the Cholesky status) and once
  *                          more per QR-based iteration (the closed-form test);
- *       mak_*_pullback_*   once (the rank / convergence counters);
+ *       mak_*_pullback_*   a few times (the conditioning and convergence values
+ *                          of the polar rule's solver, the rank counters);
  *       mak_qr_batched_execute is fully asynchronous (one graph launch).
  *   - Calls are reentrant: all state lives in the caller's workspace (the
  *     batched plans own their graph and stream; the polar's blocked Cholesky,
@@ -294,11 +295,13 @@ int mak_qr_full_cotangent_z(void* stream, int batch, int m, int n, int p, const 
 
 /* left_polar_pullback!(dA, A, (W, P), (dW, dP)) for `batch` equally sized
  * matrices (m >= n), accumulating into dA.  The Sylvester equation
- * P C + C P = M - M^H is solved by preconditioned conjugate gradients
- * (maxiter <= 0: 200, tol <= 0: 1e-14 relative residual); when CG has not
- * converged after 48 steps (ill-conditioned P), the batch is solved exactly
- * through the eigendecomposition of P (rocSOLVER, opened at first use),
- * which also gives P^{-1}.  iters receives the CG step count (may be NULL).
+ * P C + C P = M - M^H is solved to full precision by a doubling iteration
+ * when dW is given and P is well conditioned (maxiter >= 48, tol >= 1e-15);
+ * else by preconditioned conjugate gradients (maxiter <= 0: 200, tol <= 0:
+ * 1e-14 relative residual); when CG has not converged after 48 steps
+ * (ill-conditioned P), the batch is solved exactly through the
+ * eigendecomposition of P (rocSOLVER, opened at first use), which also gives
+ * P^{-1}.  iters receives the doubling or CG step count (may be NULL).
  * Returns 6 when CG did not reach tol and rocSOLVER is not available, 2 when
  * P is not positive definite.
  * Replaces left_polar_pullback! (src/pullbacks/polar.jl:7-29). */
