@@ -257,8 +257,8 @@ int mak_right_polar_pushforward_z(void* stream, int m, int n, const void* Wh, in
 int mak_pullback_workspace_size(int kind, int dtype, int batch, int m, int n, size_t* bytes);
 
 /* qr_pullback!(dA, A, (Q, R), (dQ, dR)) for `batch` equally sized matrices
- * (matrix b at pointer + b * stride), accumulating into dA (dA += ...).  Q is
- * re-formed from the compact WY factors (A_wy, T) kept by
+ * (matrix b at pointer + b * stride), accumulating into dA (dA += ...).  Q
+ * enters through the compact WY factors (A_wy, T) kept by
  * mak_qr_compact_wy_*, with the gauge signs when `positive` matches the
  * primal's positive = true; R is the primal's R (min(m,n) x n, only its upper
  * triangle is read); p is the rank (qr_rank, src/pullbacks/qr.jl:1-2).

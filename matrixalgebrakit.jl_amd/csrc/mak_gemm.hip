@@ -603,7 +603,7 @@ static void gemm_shape(const GemmArgs& g, hipStream_t s) {
   } else if (!cplx && g.K <= 128 && wgs(64, 64) >= 512) {
     // short-K updates stream C: smaller tiles keep more loads in flight
     launch_gemm_tile<64, 64, 16, 2, 2, OPA, OPB, T>(g, s);
-  } else if (!cplx && wgs(128, 128) >= 192) {
+  } else if (!cplx && wgs(128, 128) >= 192 && std::min(g.M, g.N) > 64) {  // (else half of each 128 tile is padding)
     if constexpr (!cplx) launch_gemm_tile<128, 128, 16, 2, 2, OPA, OPB, T>(g, s);
   } else if (wgs(64, 64) >= 128) {
     launch_gemm_tile<64, 64, 16, 2, 2, OPA, OPB, T>(g, s);

@@ -2,12 +2,18 @@
 // equally sized matrices (strided storage, every product a batched MFMA GEMM).
 //
 // qr_pullback! (MatrixAlgebraKit src/pullbacks/qr.jl:73-120), rank p:
-//   Q is re-formed from the compact WY factors kept by the primal
-//   (V strictly below the diagonal of A_wy, one 32x32 T per panel), with the
-//   positive gauge of R;
 //   dQ1 -= Q1 (dR12 R12^H), dA2 += Q1 dR12                    (n > p)
 //   M = triu(dR11) R11^H - Q1^H dQ1 ; M <- copyltu(M) (real diagonal)
 //   dA1 += (dQ1 + Q1 M) R11^{-H}
+// with Q1 = ([I; 0] - V T V_1^H) D from the compact WY factors kept by the
+// primal (V strictly below the diagonal of A_wy, one 32x32 T per panel, merged
+// here; D the gauge signs).  Q1 itself is never formed: with N = dR12 R12^H,
+//   Z = V^H dQ1,  Q1^H dQ1 = D^H (dQ1_top - V_1 T^H Z)
+//   B = D [(M - N) R11^{-H}, dR12],  G = T V_1^H B
+//   dA += dQ1 [R11^{-H}, 0] + [B; 0] - V G
+// Four products with m rows (V^H V, V^H dQ, dQ R^{-H}, V G) and a dozen n x n
+// ones, where forming Q1 panel by panel took a pass over all of it per 32
+// columns and three more products: 256 x (2048 x 256) Float64 10.0 -> 7.0 ms.
 // left_polar_pullback! (src/pullbacks/polar.jl:7-29):
 //   dP <- herm(dP) ; M = W^H dW - dP P ; solve P C + C P = M - M^H
 //   dA += W (C + dP) + (dW - W W^H dW) P^{-1}
@@ -86,15 +92,6 @@ __global__ void btriu_kernel(int m, int n, const T* X, int64_t ldx, int64_t sx, 
   const int r = (int)(idx % m), c = (int)(idx / m);
   Y[blockIdx.z * sy + r + c * ldy] = (r <= c) ? X[blockIdx.z * sx + r + c * ldx] : s_zero(T());
 }
-// M <- copyltu(M): lower part <- conj(upper part), real diagonal
-template <typename T> __global__ void bcopyltu_kernel(int n, T* M, int64_t ldm, int64_t sm) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (int64_t)n * n) return;
-  const int r = (int)(idx % n), c = (int)(idx / n);
-  T* Mb = M + blockIdx.z * sm;
-  if (r > c) Mb[r + c * ldm] = s_conj(Mb[c + r * ldm]);
-  else if (r == c) Mb[r + c * ldm] = s_from_real<T>(s_re(Mb[r + c * ldm]));
-}
 // Y = (X + X^H) / 2
 template <typename T>
 __global__ void bherm_kernel(int n, const T* X, int64_t ldx, int64_t sx, T* Y, int64_t ldy, int64_t sy) {
@@ -123,49 +120,128 @@ __global__ void baxpy_kernel(int m, int n, double a, const T* X, int64_t ldx, in
   T* y = Y + blockIdx.z * sy + r + c * ldy;
   *y = s_add(*y, s_scale(X[blockIdx.z * sx + r + c * ldx], a));
 }
-// Q[:, j] *= sign_safe(Awy[j, j])  (positive gauge of the re-formed Q)
+// V1 (p x p) = the unit lower top of V; T (p x p) = the panels' T blocks on the
+// diagonal, zero elsewhere.
 template <typename T>
-__global__ void bgauge_kernel(int m, int k, const T* A, int64_t lda, int64_t sa, T* Q, int64_t ldq, int64_t sq) {
+__global__ void __launch_bounds__(256) bwy_tops_kernel(int p, const T* A, int64_t lda, int64_t sa, const T* Tp,
+                                                       int64_t st, T* V1, T* Tm) {
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x, pp = (int64_t)p * p;
+  if (idx >= pp) return;
+  const int r = (int)(idx % p), c = (int)(idx / p);
+  const int64_t o = blockIdx.z * pp + idx;
+  V1[o] = r > c ? A[blockIdx.z * sa + r + (int64_t)c * lda] : (r == c ? s_one(T()) : s_zero(T()));
+  Tm[o] = r / NB == c / NB ? Tp[blockIdx.z * st + (int64_t)(c / NB) * NB * NB + r % NB + (c % NB) * NB] : s_zero(T());
+}
+// M - N with M = copyltu(A0 + N - D^H (dQ_top - Y)) (the upper part mirrored,
+// real diagonal), by pairs of mirrored 32 x 32 tiles; A0, N, dQ may be null
+// (zero).  sgn: d_i = sign_safe(A(i, i)) when sgn is 1, else 1.
+template <typename T>
+__global__ void __launch_bounds__(256) bqr_m_kernel(int p, const T* A0, const T* N, const T* dQ, int64_t lddq,
+                                                    int64_t sdq, const T* Y, const T* A, int64_t lda, int64_t sa,
+                                                    int sgn, T* Out) {
+  __shared__ T tile[32][33];
+  if (blockIdx.x > blockIdx.y) return;
+  const int r0 = blockIdx.x * 32, c0 = blockIdx.y * 32;
+  const int64_t o = (int64_t)blockIdx.z * p * p;
+  for (int e = threadIdx.x; e < 1024; e += 256) {
+    const int i = r0 + e % 32, j = c0 + e / 32;
+    T v = s_zero(T());
+    if (i < p && j < p && i <= j) {
+      const int64_t x = o + i + (int64_t)j * p;
+      const T n = N != nullptr ? N[x] : s_zero(T());
+      if (A0 != nullptr) v = A0[x];
+      v = s_add(v, n);
+      if (dQ != nullptr) {
+        T q = s_sub(dQ[blockIdx.z * sdq + i + (int64_t)j * lddq], Y[x]);
+        if (sgn) q = s_mul(s_conj(sign_safe(A[blockIdx.z * sa + i + (int64_t)i * lda])), q);
+        v = s_sub(v, q);
+      }
+      if (i == j) v = s_from_real<T>(s_re(v));
+      Out[x] = s_sub(v, n);
+    }
+    tile[e % 32][e / 32] = v;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < 1024; e += 256) {
+    const int i = c0 + e % 32, j = r0 + e / 32;  // the mirrored entry, i > j
+    if (i < p && j < p && i > j) {
+      const int64_t x = o + i + (int64_t)j * p;
+      T v = s_conj(tile[e / 32][e % 32]);
+      if (N != nullptr) v = s_sub(v, N[x]);
+      Out[x] = v;
+    }
+  }
+}
+// B (p x n, packed) = D [E, dR12] (dR12 null: zero) and dA_top += B.
+template <typename T>
+__global__ void __launch_bounds__(256) bqr_b_kernel(int p, int n, const T* E, const T* dR, int64_t lddr, int64_t sdr,
+                                                    const T* A, int64_t lda, int64_t sa, int sgn, T* B, T* dA,
+                                                    int64_t ldda, int64_t sda) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (int64_t)m * k) return;
-  const int r = (int)(idx % m), c = (int)(idx / m);
-  T* q = Q + blockIdx.z * sq + r + c * ldq;
-  *q = s_mul(*q, sign_safe(A[blockIdx.z * sa + c + c * lda]));
+  if (idx >= (int64_t)p * n) return;
+  const int r = (int)(idx % p), c = (int)(idx / p);
+  T v = s_zero(T());
+  if (c < p) v = E[(int64_t)blockIdx.z * p * p + idx];
+  else if (dR != nullptr) v = dR[blockIdx.z * sdr + r + (int64_t)c * lddr];
+  if (sgn) v = s_mul(sign_safe(A[blockIdx.z * sa + r + (int64_t)r * lda]), v);
+  B[(int64_t)blockIdx.z * p * n + idx] = v;
+  T* y = dA + blockIdx.z * sda + r + (int64_t)c * ldda;
+  *y = s_add(*y, v);
 }
 
-// Inverse of a kb x kb (kb <= 64) upper-triangular diagonal block of U into Y
-// (rank-1 steps in LDS).  Block b of the grid's z dimension handles matrix b;
-// the grid's x dimension enumerates the diagonal blocks.
+// Inverse of a kb x kb (kb <= 64) upper-triangular diagonal block of U into Y.
+// Block b of the grid's z dimension handles matrix b; the grid's x dimension
+// enumerates the diagonal blocks.  Two waves invert the 32 x 32 halves by back
+// substitution (lane c: column c, the rows of U read from LDS at uniform
+// addresses), the off-diagonal part is -Y11 U12 Y22 on MFMA: 242 us (256
+// matrices of four blocks, rank-1 steps with a barrier each) -> 36 us.
 template <typename T>
 __global__ void __launch_bounds__(256) btrtri_diag_kernel(int n, const T* U, int64_t ldu, int64_t su, T* Y,
                                                           int64_t ldy, int64_t sy) {
-  __shared__ T Ul[DBK][DBK + 1];
-  __shared__ T S[DBK][DBK + 1];
+  __shared__ T Ul[3][32][33];  // U11, U22 (identity-padded), U12
+  __shared__ T Yl[2][32][33];
   const int tid = threadIdx.x;
   const int k0 = blockIdx.x * DBK;
   const int kb = min(DBK, n - k0);
   const T* Ub = U + blockIdx.z * su + k0 + (int64_t)k0 * ldu;
   T* Yb = Y + blockIdx.z * sy + k0 + (int64_t)k0 * ldy;
-  for (int i = tid; i < DBK * DBK; i += 256) {
-    const int r = i % DBK, c = i / DBK;
-    Ul[r][c] = (r <= c && c < kb) ? Ub[r + c * ldu] : s_zero(T());
+  for (int e = tid; e < 3 * 1024; e += 256) {
+    const int h = e >> 10, i = e & 31, j = (e >> 5) & 31;
+    const int r = (h == 1 ? 32 : 0) + i, c = (h == 0 ? 0 : 32) + j;
+    T v = s_zero(T());
+    if (r < kb && c < kb && r <= c) v = Ub[r + (int64_t)c * ldu];
+    else if (r == c) v = s_one(T());
+    Ul[h][i][j] = v;
   }
   __syncthreads();
-  for (int i = tid; i < DBK * DBK; i += 256) {
-    const int r = i % DBK, c = i / DBK;
-    S[r][c] = (r == c && r < kb) ? s_div(s_one(T()), Ul[r][r]) : s_zero(T());
-  }
-  __syncthreads();
-  for (int jj = kb - 1; jj > 0; --jj) {
-    for (int i = tid; i < DBK * DBK; i += 256) {
-      const int r = i % DBK, c = i / DBK;
-      if (r < jj && c >= jj && c < kb) S[r][c] = s_sub(S[r][c], s_mul(s_div(Ul[r][jj], Ul[r][r]), S[jj][c]));
+  const int w = tid >> 6, c = tid & 63;
+  if (w < 2 && c < 32) {
+    T y[32];
+#pragma unroll
+    for (int r = 31; r >= 0; --r) {
+      T acc0 = r == c ? s_one(T()) : s_zero(T()), acc1 = s_zero(T());
+#pragma unroll
+      for (int k = r + 1; k < 32; ++k) {
+        const T u = s_neg(Ul[w][r][k]);
+        if (k & 1) acc1 = s_fma(u, y[k], acc1);
+        else acc0 = s_fma(u, y[k], acc0);
+      }
+      y[r] = s_div(s_add(acc0, acc1), Ul[w][r][r]);
     }
-    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 32; ++r) Yl[w][r][c] = r <= c ? y[r] : s_zero(T());
   }
-  for (int i = tid; i < DBK * DBK; i += 256) {
-    const int r = i % DBK, c = i / DBK;
-    if (r < kb && c < kb) Yb[r + c * ldy] = (r <= c) ? S[r][c] : s_zero(T());
+  __syncthreads();
+  mm32<T>(Ul[2], Ul[2], false, Yl[1], false, 1.0, false);
+  mm32<T>(Ul[2], Yl[0], false, Ul[2], false, -1.0, false);
+  for (int e = tid; e < DBK * DBK; e += 256) {
+    const int r = e % DBK, cc = e / DBK;
+    if (r < kb && cc < kb) {
+      T v = s_zero(T());
+      if (r < 32 && cc >= 32) v = Ul[2][r][cc - 32];
+      else if (r / 32 == cc / 32) v = Yl[r / 32][r % 32][cc % 32];
+      Yb[r + (int64_t)cc * ldy] = v;
+    }
   }
 }
 
@@ -270,33 +346,6 @@ void bpotrf_upper(int batch, int n, T* Z, int64_t ldz, int64_t sz, T* Ydiag, int
       gemm<T>(OP_C, OP_N, bga<T>(batch, rest, rest, kb, Zrow, ldz, sz, Zrow, ldz, sz, Z22, ldz, sz, -1.0, 1.0), s);
     }
   }
-}
-
-// Batched Q re-formation from compact WY (qr_compact shape, Q m x k).
-template <typename T>
-void borgqr(int batch, int m, int n, const T* A, int64_t lda, int64_t sa, const T* Tp, int64_t st, T* Q, int64_t ldq,
-            int64_t sq, T* Wb, T* W2b, int positive, hipStream_t s) {
-  const int k = std::min(m, n);
-  hipLaunchKernelGGL((bfill_kernel<T>), egrid((int64_t)m * k, batch), dim3(256), 0, s, m, k, Q, ldq, sq, 1);
-  const int npan = cdiv(k, NB);
-  const int64_t sw = (int64_t)NB * k;
-  for (int p = npan - 1; p >= 0; --p) {
-    const int j0 = p * NB, nbc = std::min(NB, k - j0), rows = m - j0, ncols = k - j0;
-    const T* Vp = A + j0 + (int64_t)j0 * lda;
-    T* C = Q + j0 + (int64_t)j0 * ldq;
-    // W = V^H C ; W2 = T W ; C -= V W2
-    GemmArgs g1 = bga<T>(batch, nbc, ncols, rows, Vp, lda, sa, C, ldq, sq, Wb, nbc, sw, 1.0, 0.0);
-    g1.unitLowerA = 1;
-    gemm<T>(OP_C, OP_N, g1, s);
-    gemm<T>(OP_N, OP_N, bga<T>(batch, nbc, ncols, nbc, Tp + (int64_t)p * NB * NB, NB, st, Wb, nbc, sw, W2b, nbc, sw,
-                               1.0, 0.0), s);
-    GemmArgs g3 = bga<T>(batch, rows, ncols, nbc, Vp, lda, sa, W2b, nbc, sw, C, ldq, sq, -1.0, 1.0);
-    g3.unitLowerA = 1;
-    gemm<T>(OP_N, OP_N, g3, s);
-  }
-  if (positive)
-    hipLaunchKernelGGL((bgauge_kernel<T>), egrid((int64_t)m * k, batch), dim3(256), 0, s, m, k, A, lda, sa, Q, ldq,
-                       sq);
 }
 
 // ---- batched reductions for CG: out[b] = Re sum conj(X_b) Y_b
@@ -590,14 +639,9 @@ int polar_pullback_doubling(hipStream_t s, int batch, int m, int n, const T* W, 
 // workspace layouts
 // ---------------------------------------------------------------------------
 template <typename T> size_t qr_pullback_ws(int batch, int m, int n) {
-  const int k = std::min(m, n);
-  size_t b = 0;
-  b += al256((size_t)batch * m * k * sizeof(T));      // Q
-  b += al256((size_t)batch * m * k * sizeof(T));      // X = dQ1 (+ Q M)
-  b += al256((size_t)batch * k * k * sizeof(T)) * 3;  // M, Rinv, triu(dR11)
-  b += al256((size_t)batch * NB * k * sizeof(T)) * 2; // WY scratch
-  b += al256((size_t)batch * k * k * sizeof(T));      // triu(R11)
-  return b;
+  const size_t k = std::min(m, n);
+  return al256((size_t)batch * k * k * sizeof(T)) * 10     // V1, S, T, triu(R11), R11^{-1}, N, A0, M, two scratch
+         + al256((size_t)batch * k * n * sizeof(T)) * 2;   // B, G
 }
 // out[b] = max(out[b], max |X_ij|) over a rows x cols block of matrix b
 // (upper = 1: only i <= j), by a grid-stride loop per batch member and an
@@ -691,48 +735,80 @@ int qr_pullback(hipStream_t s, int batch, int m, int n, int p, int positive, con
   }
   if (batch == 0 || p == 0) return 0;
   char* w = reinterpret_cast<char*>(work);
-  auto take = [&](size_t bytes) { char* q = w; w += al256(bytes); return reinterpret_cast<T*>(q); };
-  const int64_t smk = (int64_t)m * k, skk = (int64_t)k * k;
-  T* Q = take((size_t)batch * smk * sizeof(T));
-  T* X = take((size_t)batch * smk * sizeof(T));
-  T* M = take((size_t)batch * skk * sizeof(T));
-  T* Rinv = take((size_t)batch * skk * sizeof(T));
-  T* dR11u = take((size_t)batch * skk * sizeof(T));
-  T* Wb = take((size_t)batch * NB * k * sizeof(T));
-  T* W2b = take((size_t)batch * NB * k * sizeof(T));
-  T* Rt = take((size_t)batch * skk * sizeof(T));
-  // Q = orgqr(V, T) (times the gauge signs when the primal used positive = true)
-  borgqr<T>(batch, m, n, A, lda, sa, Tp, st, Q, m, smk, Wb, W2b, positive, s);
-  // Rt = triu(R11): only the upper triangle of R is read (UpperTriangular(R11), src/pullbacks/qr.jl:92)
-  hipLaunchKernelGGL((btriu_kernel<T>), egrid((int64_t)p * p, batch), dim3(256), 0, s, p, p, R, ldr, sr, Rt,
-                     (int64_t)k, skk);
-  // X = dQ1
-  if (dQ) hipLaunchKernelGGL((bcopy_kernel<T>), egrid((int64_t)m * p, batch), dim3(256), 0, s, m, p, dQ, lddq, sdq, X,
-                             (int64_t)m, smk);
-  else hipLaunchKernelGGL((bfill_kernel<T>), egrid((int64_t)m * p, batch), dim3(256), 0, s, m, p, X, (int64_t)m, smk, 0);
-  if (dR && n > p) {
-    // X -= Q1 (dR12 R12^H) ; dA2 += Q1 dR12
-    gemm<T>(OP_N, OP_C, bga<T>(batch, p, p, n - p, dR + (int64_t)p * lddr, lddr, sdr, R + (int64_t)p * ldr, ldr, sr,
-                               M, k, skk, 1.0, 0.0), s);
-    gemm<T>(OP_N, OP_N, bga<T>(batch, m, p, p, Q, m, smk, M, k, skk, X, m, smk, -1.0, 1.0), s);
-    gemm<T>(OP_N, OP_N, bga<T>(batch, m, n - p, p, Q, m, smk, dR + (int64_t)p * lddr, lddr, sdr,
-                               dA + (int64_t)p * ldda, ldda, sda, 1.0, 1.0), s);
+  auto take = [&](size_t elems) { char* q = w; w += al256(elems * sizeof(T)); return reinterpret_cast<T*>(q); };
+  const int64_t pp = (int64_t)p * p;
+  const size_t bk = (size_t)batch * k * k;
+  T *V1 = take(bk), *S = take(bk), *Tm = take(bk), *Ru = take(bk), *Rinv = take(bk), *N = take(bk), *A0 = take(bk),
+    *M = take(bk), *X1 = take(bk), *X2 = take(bk);
+  T *B = take((size_t)batch * k * n), *G = take((size_t)batch * k * n);
+  const dim3 gpp = egrid(pp, batch);
+  auto prod = [&](int opA, int opB, const T* X, const T* Y, T* C, double alpha, double beta, int tri) {
+    GemmArgs g = bga<T>(batch, p, p, p, X, p, pp, Y, p, pp, C, p, pp, alpha, beta);
+    g.tri = tri;
+    gemm<T>(opA, opB, g, s);
+  };
+  // V_1, S = V^H V (upper) and the merged T: T(0:j, b) = -T(0:j, 0:j) S(0:j, b) T_b
+  hipLaunchKernelGGL((bwy_tops_kernel<T>), gpp, dim3(256), 0, s, p, A, lda, sa, Tp, st, V1, Tm);
+  if (p > NB) {
+    GemmArgs g = bga<T>(batch, p, p, m - p, A + p, lda, sa, A + p, lda, sa, S, p, pp, 1.0, 0.0);
+    g.upperC = 1;
+    gemm<T>(OP_C, OP_N, g, s);
+    g = bga<T>(batch, p, p, p, V1, p, pp, V1, p, pp, S, p, pp, 1.0, 1.0);
+    g.upperC = 1;
+    gemm<T>(OP_C, OP_N, g, s);
   }
-  // M = triu(dR11) R11^H - Q1^H X
-  if (dR) {
-    hipLaunchKernelGGL((btriu_kernel<T>), egrid((int64_t)p * p, batch), dim3(256), 0, s, p, p, dR, lddr, sdr, dR11u,
-                       (int64_t)k, skk);
-    gemm<T>(OP_N, OP_C, bga<T>(batch, p, p, p, dR11u, k, skk, Rt, k, skk, M, k, skk, 1.0, 0.0), s);
-    gemm<T>(OP_C, OP_N, bga<T>(batch, p, p, m, Q, m, smk, X, m, smk, M, k, skk, -1.0, 1.0), s);
-  } else {
-    gemm<T>(OP_C, OP_N, bga<T>(batch, p, p, m, Q, m, smk, X, m, smk, M, k, skk, -1.0, 0.0), s);
+  for (int j = NB; j < p; j += NB) {
+    const int nb = std::min(NB, p - j);
+    gemm<T>(OP_N, OP_N, bga<T>(batch, j, nb, nb, S + (int64_t)j * p, p, pp, Tm + j + (int64_t)j * p, p, pp, X1, p, pp,
+                               1.0, 0.0), s);
+    gemm<T>(OP_N, OP_N, bga<T>(batch, j, nb, j, Tm, p, pp, X1, p, pp, Tm + (int64_t)j * p, p, pp, -1.0, 0.0), s);
   }
-  hipLaunchKernelGGL((bcopyltu_kernel<T>), egrid((int64_t)p * p, batch), dim3(256), 0, s, p, M, (int64_t)k, skk);
-  // X += Q1 M
-  gemm<T>(OP_N, OP_N, bga<T>(batch, m, p, p, Q, m, smk, M, k, skk, X, m, smk, 1.0, 1.0), s);
-  // dA1 += X R11^{-H}
-  btrtri_upper<T>(batch, p, Rt, k, skk, Rinv, k, skk, s);
-  gemm<T>(OP_N, OP_C, bga<T>(batch, m, p, p, X, m, smk, Rinv, k, skk, dA, ldda, sda, 1.0, 1.0), s);
+  // R11^{-1}: only the upper triangle of R is read (UpperTriangular(R11), src/pullbacks/qr.jl:92)
+  btrtri_upper<T>(batch, p, R, ldr, sr, Rinv, p, pp, s);
+  const bool wide = dR != nullptr && n > p;
+  if (dR) {  // A0 = triu(dR11) R11^H ; N = dR12 R12^H
+    hipLaunchKernelGGL((btriu_kernel<T>), gpp, dim3(256), 0, s, p, p, dR, lddr, sdr, X1, (int64_t)p, pp);
+    hipLaunchKernelGGL((btriu_kernel<T>), gpp, dim3(256), 0, s, p, p, R, ldr, sr, Ru, (int64_t)p, pp);
+    prod(OP_N, OP_C, X1, Ru, A0, 1.0, 0.0, TRI_A_UPPER | TRI_B_LOWER);
+    if (wide)
+      gemm<T>(OP_N, OP_C, bga<T>(batch, p, p, n - p, dR + (int64_t)p * lddr, lddr, sdr, R + (int64_t)p * ldr, ldr, sr,
+                                 N, p, pp, 1.0, 0.0), s);
+  }
+  if (dQ) {  // X2 = V_1 T^H (V^H dQ1)
+    GemmArgs g = bga<T>(batch, p, p, m, A, lda, sa, dQ, lddq, sdq, X1, p, pp, 1.0, 0.0);
+    g.unitLowerA = 1;
+    gemm<T>(OP_C, OP_N, g, s);
+    prod(OP_C, OP_N, Tm, X1, S, 1.0, 0.0, TRI_A_LOWER);
+    prod(OP_N, OP_N, V1, S, X2, 1.0, 0.0, TRI_A_LOWER);
+  }
+  hipLaunchKernelGGL((bqr_m_kernel<T>), dim3(cdiv(p, 32), cdiv(p, 32), batch), dim3(256), 0, s, p,
+                     dR ? (const T*)A0 : nullptr, wide ? (const T*)N : nullptr, dQ, lddq, sdq, (const T*)X2, A, lda, sa,
+                     positive, M);
+  // B = D [(M - N) R11^{-H}, dR12], dA_top += B, G = T V_1^H B
+  prod(OP_N, OP_C, M, Rinv, X1, 1.0, 0.0, TRI_B_LOWER);
+  const int nc = wide ? n : p;
+  hipLaunchKernelGGL((bqr_b_kernel<T>), egrid((int64_t)p * nc, batch), dim3(256), 0, s, p, nc, (const T*)X1, dR, lddr,
+                     sdr, A, lda, sa, positive, B, dA, ldda, sda);
+  const int64_t pc = (int64_t)p * nc;
+  {
+    GemmArgs g = bga<T>(batch, p, nc, p, V1, p, pp, B, p, pc, G, p, pc, 1.0, 0.0);
+    g.tri = TRI_A_UPPER;
+    gemm<T>(OP_C, OP_N, g, s);
+    g = bga<T>(batch, p, nc, p, Tm, p, pp, G, p, pc, B, p, pc, 1.0, 0.0);
+    g.tri = TRI_A_UPPER;
+    gemm<T>(OP_N, OP_N, g, s);
+  }
+  // dA += dQ1 [R11^{-H}, 0] - V G
+  if (dQ) {
+    GemmArgs g = bga<T>(batch, m, p, p, dQ, lddq, sdq, Rinv, p, pp, dA, ldda, sda, 1.0, 1.0);
+    g.tri = TRI_B_LOWER;
+    gemm<T>(OP_N, OP_C, g, s);
+  }
+  {
+    GemmArgs g = bga<T>(batch, m, nc, p, A, lda, sa, B, p, pc, dA, ldda, sda, -1.0, 1.0);
+    g.unitLowerA = 1;
+    gemm<T>(OP_N, OP_N, g, s);
+  }
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
