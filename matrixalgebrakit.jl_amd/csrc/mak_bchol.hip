@@ -1,0 +1,679 @@
+// CholeskyQR2 of whole blocks, many unevenly sized blocks per launch (the
+// batched qr_compact! plan, mak_batched.hip):
+//   G = A^H A = R1^H R1,  Q1 = A R1^{-1},  E = Q1^H Q1 - I,
+//   U = the upper half of E (half of its diagonal),
+//   Q = Q1 (I - U),  R = (I + U) R1.
+// E is what the condition of G left of the rounding of R1; with
+// ||E||_F <= 1e-8 (condition numbers to about 2e4) the terms of second order in
+// U are below rounding, so that the second factorisation is U itself.  With
+// ||E||_F <= 0.1 (to about 1e7) a second pass comes between: Q1 with one step
+// of refinement (its residual A - Q1 R1 would grow with the condition of R1's
+// diagonal tiles), the Cholesky factor R2 of Q1^H Q1, Q1 <- Q1 R2^{-1},
+// R1 <- R2 R1.  A block whose Gram matrix has a pivot that is not positive, or
+// whose E is larger, is rejected: left to the gated Householder launches.  A is
+// only read.
+//
+// Every product runs on 64 x 64 tiles, one workgroup of four waves (32 x 32
+// each) per task, over task lists of all blocks:
+//   Gram      upper tiles of G, K = all rows
+//   factor    block column by block column (64 wide, left-looking): step k
+//             forms the tiles R_kj, and the task of tile (k, k+1) goes on to
+//             factor diagonal tile k+1, so that a step is one launch
+//   solve     64-row strips, block column by block column:
+//             Q1_j = (A_j - sum_i Q1_i R_ij) R_jj^{-1}.  Substitution and not
+//             a product with R1^{-1}: its residual does not grow with the
+//             condition number of R1
+//   Gram      E, and its tiles' norms
+//   correct   Q1 - Q1 U in place, strips from the last block column to the
+//             first; the tiles of R
+// 4 m n^2 flops a block, as many as blocked Householder with its orgqr, but
+// with inner dimensions of up to m or n instead of 32: the panel schedule read
+// and wrote the trailing matrix once per 32 columns.
+// Tasks are listed so that a block stays on one XCD (workgroup b runs on XCD
+// b mod 8), whose L2 then serves the operands that its tiles share.
+#include <algorithm>
+
+#include "mak_common.hpp"
+#include "mak_dense32.hpp"
+#include "mak_kernels.hpp"
+
+namespace mak {
+
+namespace {
+
+constexpr int BT = kBCholTile;  // 64
+constexpr double kBCholMaxE = 1e-8, kBCholMaxE2 = 0.1;
+
+// LDS of one stage of a tile product: KB inner indices of the two operands.
+// The pitches keep the fragment reads (16 rows x 4 k of a wave) off each
+// other's banks; KB = 8 for ComplexF64 keeps two stages at 37 KB (four
+// workgroups a CU).
+template <typename T> struct BcCfg;
+template <> struct BcCfg<double> {
+  static constexpr int KB = 16, PK = 17, PR = 80;
+  static constexpr int L = 16 * PR, R = 64 * PK, STAGE = L + R;
+  static constexpr int OCC_GRAM = 4, OCC = 3;  // waves per SIMD
+  static constexpr int POOL = 2 * STAGE;
+};
+template <> struct BcCfg<zd> {
+  static constexpr int KB = 8, PK = 9, PR = 65;
+  static constexpr int L = 64 * PK, R = 64 * PK, STAGE = L + R;
+  static constexpr int OCC_GRAM = 2, OCC = 2;
+  static constexpr int POOL = 2 * STAGE;
+};
+constexpr int KX = 16;  // inner indices of one stage of the product with a 64 x 64 inverse
+template <typename T> struct BcX;
+template <> struct BcX<double> { static constexpr int PK = 17, PR = 80; };
+template <> struct BcX<zd> { static constexpr int PK = 17, PR = 65; };
+static_assert(KX * BcX<double>::PR + 64 * BcX<double>::PK <= BcCfg<double>::POOL, "stage of the inverse");
+static_assert(KX * BcX<zd>::PR + 64 * BcX<zd>::PK <= BcCfg<zd>::POOL, "stage of the inverse");
+
+// 32 x 32 accumulators of a wave: row 16 i + lane % 16, column 16 j + 4 u + lane / 16
+template <typename T> struct BcAcc;
+template <> struct BcAcc<double> {
+  v4d r[2][2];
+  __device__ __forceinline__ void zero() {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) r[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+  }
+  __device__ __forceinline__ double get(int i, int j, int u) const { return r[i][j][u]; }
+  template <bool CL>
+  __device__ __forceinline__ void step(const double (&a)[2], const double (&b)[2]) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) r[i][j] = mfma_f64(b[j], a[i], r[i][j]);
+  }
+};
+// three real products (Gauss): re = p - q, im = s - p - q
+template <> struct BcAcc<zd> {
+  v4d p[2][2], q[2][2], s[2][2];
+  __device__ __forceinline__ void zero() {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) p[i][j] = q[i][j] = s[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+  }
+  __device__ __forceinline__ zd get(int i, int j, int u) const {
+    return mkz(p[i][j][u] - q[i][j][u], s[i][j][u] - p[i][j][u] - q[i][j][u]);
+  }
+  template <bool CL>
+  __device__ __forceinline__ void step(const zd (&a)[2], const zd (&b)[2]) {
+    double ai[2], as[2], bs[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      ai[i] = CL ? -a[i].y : a[i].y;
+      as[i] = a[i].x + ai[i];
+      bs[i] = b[i].x + b[i].y;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        p[i][j] = mfma_f64(b[j].x, a[i].x, p[i][j]);
+        q[i][j] = mfma_f64(b[j].y, ai[i], q[i][j]);
+        s[i][j] = mfma_f64(bs[j], as[i], s[i][j]);
+      }
+  }
+};
+
+// acc += op(L) R over K inner indices, for a 64 x 64 tile:
+//   KL:  op(L)(i, k) = conj(L[k + i ldl]);  otherwise L[i + k ldl];
+//   R(k, j) = R[k + j ldr].
+// Rows i >= nl and columns j >= nr repeat the last valid one (the caller drops
+// them); 64 ldl and 64 ldr elements stay below 2 GB.  Two LDS stages, one
+// barrier per stage, and the values of two more on their way in registers.  The
+// caller leaves the pool free; it is free again on return.
+template <typename T, bool KL>
+__device__ __forceinline__ void bc_product(BcAcc<T>& acc, T* pool, const T* L, int64_t ldl, int nl, const T* R,
+                                           int64_t ldr, int nr, int K) {
+  using C = BcCfg<T>;
+  constexpr int KB = C::KB, NQ = BT * KB / 256;
+  if (K <= 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int lr = lane & 15, lq = lane >> 4;
+  const int wm = w & 1, wn = w >> 1;
+  // byte offsets of this thread's elements from bases that advance uniformly
+  unsigned ol[NQ], orr[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const int e = tid + 256 * q;
+    orr[q] = (unsigned)((e % KB + min(e / KB, nr - 1) * (int)ldr) * (int)sizeof(T));
+    ol[q] = (unsigned)((KL ? e % KB + min(e / KB, nl - 1) * (int)ldl : min(e % BT, nl - 1) + (e / BT) * (int)ldl) *
+                       (int)sizeof(T));
+  }
+  struct Regs {
+    T l[NQ], r[NQ];
+  };
+  Regs v0, v1;
+  auto load = [&](Regs& v, int k0) {
+    const char* bl = reinterpret_cast<const char*>(L + (KL ? (int64_t)k0 : (int64_t)k0 * ldl));
+    const char* br = reinterpret_cast<const char*>(R + k0);
+    if (k0 + KB <= K) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        v.l[q] = *reinterpret_cast<const T*>(bl + ol[q]);
+        v.r[q] = *reinterpret_cast<const T*>(br + orr[q]);
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        const int e = tid + 256 * q;
+        v.l[q] = k0 + (KL ? e % KB : e / BT) < K ? *reinterpret_cast<const T*>(bl + ol[q]) : s_zero(T());
+        v.r[q] = k0 + e % KB < K ? *reinterpret_cast<const T*>(br + orr[q]) : s_zero(T());
+      }
+    }
+  };
+  auto store = [&](const Regs& v, T* st) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int e = tid + 256 * q;
+      if constexpr (KL) st[(e / KB) * C::PK + e % KB] = v.l[q];
+      else st[(e / BT) * C::PR + e % BT] = v.l[q];
+      st[C::L + (e / KB) * C::PK + e % KB] = v.r[q];
+    }
+  };
+  auto compute = [&](const T* st) {
+#pragma unroll
+    for (int kk = 0; kk < KB; kk += 4) {
+      T a[2], b[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int row = wm * 32 + i * 16 + lr, col = wn * 32 + i * 16 + lr;
+        if constexpr (KL) a[i] = st[row * C::PK + kk + lq];
+        else a[i] = st[(kk + lq) * C::PR + row];
+        b[i] = st[C::L + col * C::PK + kk + lq];
+      }
+      acc.template step<KL>(a, b);
+    }
+  };
+  // stage t is in LDS buffer t % 2, t + 1 in registers, t + 2 being loaded
+  T* s0 = pool;
+  T* s1 = pool + C::STAGE;
+  load(v0, 0);
+  if (KB < K) load(v1, KB);
+  store(v0, s0);
+  for (int k0 = 0; k0 < K; k0 += 2 * KB) {
+    if (k0 + 2 * KB < K) load(v0, k0 + 2 * KB);
+    __syncthreads();
+    compute(s0);
+    if (k0 + KB >= K) break;
+    store(v1, s1);
+    if (k0 + 3 * KB < K) load(v1, k0 + 3 * KB);
+    __syncthreads();
+    compute(s1);
+    if (k0 + 2 * KB < K) store(v0, s0);
+  }
+  __syncthreads();
+}
+
+// One stage of KX inner indices held in the pool: left as [k][row], right as [col][k].
+template <typename T, bool CL>
+__device__ __forceinline__ void bcx_step(BcAcc<T>& acc, const T* left, const T* right) {
+  using X = BcX<T>;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lr = lane & 15, lq = lane >> 4, wm = w & 1, wn = w >> 1;
+#pragma unroll
+  for (int kk = 0; kk < KX; kk += 4) {
+    T a[2], b[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      a[i] = left[(kk + lq) * X::PR + wm * 32 + i * 16 + lr];
+      b[i] = right[(wn * 32 + i * 16 + lr) * X::PK + kk + lq];
+    }
+    acc.template step<CL>(a, b);
+  }
+}
+
+// acc = V X, V the workgroup's 64 x 64 tile in registers (accumulator layout),
+// X 64 x 64: quarters of 16 inner indices through the pool.
+template <typename T>
+__device__ __forceinline__ void bc_times_x(BcAcc<T>& acc, T* pool, const T (&v)[2][2][4], const T* X, int ldx) {
+  using C = BcX<T>;
+  T* left = pool;
+  T* right = pool + KX * C::PR;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int lr = lane & 15, lq = lane >> 4, wm = w & 1, wn = w >> 1;
+  acc.zero();
+#pragma unroll
+  for (int h = 0; h < BT / KX; ++h) {
+    T x[BT * KX / 256];
+#pragma unroll
+    for (int q = 0; q < BT * KX / 256; ++q) {
+      const int e = tid + 256 * q;
+      x[q] = X[h * KX + e % KX + (e / KX) * ldx];
+    }
+    if (h > 0) __syncthreads();
+    if (wn == h / 2) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) left[(4 * u + lq) * C::PR + wm * 32 + i * 16 + lr] = v[i][h % 2][u];
+    }
+#pragma unroll
+    for (int q = 0; q < BT * KX / 256; ++q) {
+      const int e = tid + 256 * q;
+      right[(e / KX) * C::PK + e % KX] = x[q];
+    }
+    __syncthreads();
+    bcx_step<T, false>(acc, left, right);
+  }
+  __syncthreads();
+}
+
+// acc = X^H V, as above
+template <typename T> __device__ __forceinline__ void bc_xh_times(BcAcc<T>& acc, T* pool, const T* X, const T (&v)[2][2][4]) {
+  using C = BcX<T>;
+  T* left = pool;
+  T* right = pool + KX * C::PR;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int lr = lane & 15, lq = lane >> 4, wm = w & 1, wn = w >> 1;
+  acc.zero();
+#pragma unroll
+  for (int h = 0; h < BT / KX; ++h) {
+    T x[BT * KX / 256];
+#pragma unroll
+    for (int q = 0; q < BT * KX / 256; ++q) {
+      const int e = tid + 256 * q;
+      x[q] = X[h * KX + e % KX + (e / KX) * BT];
+    }
+    if (h > 0) __syncthreads();
+#pragma unroll
+    for (int q = 0; q < BT * KX / 256; ++q) {
+      const int e = tid + 256 * q;
+      left[(e % KX) * C::PR + e / KX] = x[q];
+    }
+    if (wm == h / 2) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) right[(wn * 32 + j * 16 + 4 * u + lq) * C::PK + lr] = v[h % 2][j][u];
+    }
+    __syncthreads();
+    bcx_step<T, true>(acc, left, right);
+  }
+  __syncthreads();
+}
+
+// A leading dimension whose products with column indices are formed where they
+// are used, not kept in registers over the loop around.
+__device__ __forceinline__ int bc_local(int64_t ld) {
+  int v = (int)ld;
+  asm volatile("" : "+s"(v));
+  return v;
+}
+
+// Status words of a replay: nothing rejected, no panel rejected.
+__global__ void bchol_init_kernel(int* state, unsigned long long* dev, int n, int* any, int* status, int nst) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < n) {
+    state[e] = 0;
+    dev[e] = 0ull;
+  }
+  if (e < nst) status[e] = 0;
+  if (e == 0) *any = 0;
+}
+
+// States of a block: 0 factored in one pass, 2 in two, 1 rejected.
+__device__ __forceinline__ bool bc_skip(const BCholProb& p, int pass) { return *p.state != (pass == 2 ? 2 : 0); }
+
+// State after E of this pass; any |= rejected.
+__global__ void bchol_decide_kernel(const BCholProb* P, int n, int* any, int pass) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= n) return;
+  const BCholProb p = P[e];
+  const int nt = p.np / BT;
+  const double s = __longlong_as_double((long long)*p.dev) * nt * nt;  // bounds ||E||_F^2
+  int st = *p.state;
+  if (!bc_skip(p, pass)) {
+    if (pass == 1) st = s <= kBCholMaxE * kBCholMaxE ? 0 : s <= kBCholMaxE2 * kBCholMaxE2 ? 2 : 1;  // not a number: 1
+    else if (!(s <= kBCholMaxE * kBCholMaxE)) st = 1;
+    *p.state = st;
+    *p.dev = 0ull;
+  }
+  if (st == 1) *any = 1;  // every writer writes 1
+}
+
+// Tile (a, b), a <= b: of A^H A in W, in the second pass of Q1^H Q1 in U
+// (padding: the identity), or, HALF, of U from E = Q1^H Q1 - I (padding: 0)
+// with the tile's norm.
+template <typename T, bool HALF>
+__global__ void __launch_bounds__(256, BcCfg<T>::OCC_GRAM)
+    bchol_gram_kernel(const BCholProb* P, const BCholTask* tasks, int pass) {
+  using C = BcCfg<T>;
+  __shared__ T pool[C::POOL];
+  __shared__ double part[4];
+  const BCholTask t = tasks[blockIdx.x];
+  if (t.prob < 0) return;
+  const BCholProb p = P[t.prob];
+  if (bc_skip(p, pass)) return;
+  const int i0 = t.a * BT, j0 = t.b * BT;
+  const bool second = HALF || pass == 2;
+  const T* X = reinterpret_cast<const T*>(second ? p.Q : p.A);
+  const int64_t ldx = second ? p.ldq : p.lda;
+  BcAcc<T> acc;
+  acc.zero();
+  bc_product<T, true>(acc, pool, X + (int64_t)i0 * ldx, ldx, p.n - i0, X + (int64_t)j0 * ldx, ldx, p.n - j0, p.m);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lr = lane & 15, lq = lane >> 4, wm = w & 1, wn = w >> 1;
+  T* G = reinterpret_cast<T*>(second ? p.U : p.W);
+  double s2 = 0.0;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int gi = i0 + wm * 32 + i * 16 + lr, gj = j0 + wn * 32 + j * 16 + 4 * u + lq;
+        T v = acc.get(i, j, u);
+        if (gi == gj) v = s_from_real<T>(HALF ? s_re(v) - 1.0 : s_re(v));
+        if (gi >= p.n || gj >= p.n) v = (!HALF && gi == gj) ? s_one(T()) : s_zero(T());
+        if constexpr (HALF) {
+          s2 += s_abs2(v);
+          v = gi > gj ? s_zero(T()) : (gi == gj ? s_scale(v, 0.5) : v);
+        }
+        G[gi + (int64_t)gj * p.np] = v;
+      }
+  if constexpr (HALF) {
+    s2 = wave_sum(s2);
+    if (lane == 0) part[w] = s2;
+    __syncthreads();
+    // non-negative doubles order like their bits (and a NaN above them all)
+    if (threadIdx.x == 0)
+      atomicMax(p.dev, (unsigned long long)__double_as_longlong(fabs(part[0] + part[1] + part[2] + part[3])));
+  }
+}
+
+// Step k of the factorisation of G: tile R_kb and its term of diagonal tile b,
+// then for b = k + 1 the factor of that tile (k = -1: only that).  The diagonal tile of 64 is factored with its
+// inverse as 32 x 32 blocks by wave 0.
+template <typename T>
+__global__ void __launch_bounds__(256) bchol_factor_kernel(const BCholProb* P, const BCholTask* tasks, int pass) {
+  using C = BcCfg<T>;
+  __shared__ T pool[C::POOL > 5 * 32 * 33 ? C::POOL : 5 * 32 * 33];
+  __shared__ int bad_s;
+  const BCholTask t = tasks[blockIdx.x];
+  if (t.prob < 0) return;
+  const BCholProb p = P[t.prob];
+  if (bc_skip(p, pass)) return;
+  const int k = t.a, b = t.b;
+  const int64_t ld = p.np;
+  T* W = reinterpret_cast<T*>(pass == 2 ? p.U : p.W);
+  T* Xd = reinterpret_cast<T*>(p.X);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lr = lane & 15, lq = lane >> 4, wm = w & 1, wn = w >> 1;
+  const int ri = wm * 32 + lr, cj = wn * 32 + lq;  // + 16 i, + 16 j + 4 u
+  const T* Wb = W + (int64_t)b * BT * ld;
+  BcAcc<T> acc;
+  if (k >= 0) {
+    T* Wkb = W + (int64_t)k * BT + (int64_t)b * BT * ld;
+    acc.zero();
+    bc_product<T, true>(acc, pool, W + (int64_t)k * BT * ld, ld, BT, Wb, ld, BT, k * BT);
+    T v[2][2][4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          v[i][j][u] = s_sub(Wkb[ri + 16 * i + (int64_t)(cj + 16 * j + 4 * u) * ld], acc.get(i, j, u));
+    bc_xh_times<T>(acc, pool, Xd + (int64_t)k * BT * BT, v);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) Wkb[ri + 16 * i + (int64_t)(cj + 16 * j + 4 * u) * ld] = acc.get(i, j, u);
+    __syncthreads();  // R_kb is read by every wave below
+  }
+  // S = G_bb - sum_i<=k R_ib^H R_ib, one term per step: kept in G_bb, or for the
+  // next diagonal block in three 32 x 32 blocks of the pool
+  T (*S11)[33] = reinterpret_cast<T (*)[33]>(pool);
+  T (*Y11)[33] = S11 + 32;
+  T (*S12)[33] = S11 + 64;  // then Y22
+  T (*W12)[33] = S11 + 96;
+  T (*S22)[33] = S11 + 128;  // then W12 Y22
+  T* Wbb = W + (int64_t)b * BT * (ld + 1);
+  acc.zero();
+  if (k >= 0) bc_product<T, true>(acc, pool, Wb + k * BT, ld, BT, Wb + k * BT, ld, BT, BT);
+  if (b != k + 1) {
+    if (wm <= wn)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            T* g = Wbb + ri + 16 * i + (int64_t)(cj + 16 * j + 4 * u) * ld;
+            *g = s_sub(*g, acc.get(i, j, u));
+          }
+    return;
+  }
+  if (wm <= wn) {
+    T (*S)[33] = wn == 0 ? S11 : wm == 0 ? S12 : S22;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          S[16 * i + lr][16 * j + 4 * u + lq] =
+              s_sub(Wbb[ri + 16 * i + (int64_t)(cj + 16 * j + 4 * u) * ld], acc.get(i, j, u));
+  }
+  if (threadIdx.x == 0) bad_s = 0;
+  __syncthreads();
+  if (w == 0) {
+    const int bad = wave_chol_inv32<T>(S11, Y11);
+    if (bad && lane == 0) bad_s = 1;
+  }
+  __syncthreads();
+  mm32<T>(W12, Y11, true, S12, false, 1.0, false);
+  mm32<T>(S22, W12, true, W12, false, -1.0, true);
+  if (w == 0) {
+    const int bad = wave_chol_inv32<T>(S22, S12);
+    if (bad && lane == 0) bad_s = 1;
+  }
+  __syncthreads();
+  T* Xb = Xd + (int64_t)b * BT * BT;
+  for (int e = threadIdx.x; e < BT * BT; e += 256) {
+    const int i = e % BT, j = e / BT;
+    T wv = s_zero(T()), xv = s_zero(T());
+    if (j < 32) {
+      if (i < 32) {
+        wv = S11[i][j];
+        xv = Y11[i][j];
+      }
+    } else if (i < 32) {
+      wv = W12[i][j - 32];
+    } else {
+      wv = S22[i - 32][j - 32];
+      xv = S12[i - 32][j - 32];
+    }
+    Wbb[i + (int64_t)j * ld] = wv;
+    if (i >= 32 || j < 32) Xb[e] = xv;
+  }
+  __syncthreads();
+  mm32<T>(S22, W12, false, S12, false, 1.0, false);
+  mm32<T>(S22, Y11, false, S22, false, -1.0, false);
+  for (int e = threadIdx.x; e < 32 * 32; e += 256) Xb[e % 32 + (32 + e / 32) * BT] = S22[e % 32][e / 32];
+  if (threadIdx.x == 0 && bad_s) *p.state = 1;
+}
+
+// Strip a (64 rows) of Q1 = A R1^{-1}; second: of Q1 <- Q1 R2^{-1}, in place.
+// REFINE: with Q1_j += (B_j - Q1_j R_jj) R_jj^{-1} for each block column.
+template <typename T, bool REFINE>
+__global__ void __launch_bounds__(256, BcCfg<T>::OCC)
+    bchol_solve_kernel(const BCholProb* P, const BCholTask* tasks, int pass, int second) {
+  using C = BcCfg<T>;
+  __shared__ T pool[C::POOL];
+  const BCholTask t = tasks[blockIdx.x];
+  if (t.prob < 0) return;
+  const BCholProb p = P[t.prob];
+  if (bc_skip(p, pass)) return;
+  const int r0 = t.a * BT, rows = p.m - r0;
+  const T* A = reinterpret_cast<const T*>(second ? p.Q : p.A) + r0;
+  T* Q = reinterpret_cast<T*>(p.Q) + r0;
+  const T* W = reinterpret_cast<const T*>(second ? p.U : p.W);
+  const T* Xd = reinterpret_cast<const T*>(p.X);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lr = lane & 15, lq = lane >> 4, wm = w & 1, wn = w >> 1;
+  const int ri = wm * 32 + lr, cj = wn * 32 + lq;
+  BcAcc<T> acc;
+  for (int jb = 0; jb * BT < p.n; ++jb) {
+    const int j0 = jb * BT, lda = bc_local(second ? p.ldq : p.lda), ldq = bc_local(p.ldq);
+    acc.zero();
+    bc_product<T, false>(acc, pool, Q, ldq, rows, W + (int64_t)j0 * p.np, p.np, BT, j0);
+    T v[2][2][4];
+    const T* Aj = A + (int64_t)j0 * p.lda;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int r = ri + 16 * i, c = cj + 16 * j + 4 * u;
+          v[i][j][u] = (r < rows && j0 + c < p.n) ? s_sub(Aj[r + c * lda], acc.get(i, j, u)) : s_zero(T());
+        }
+    const T* X = Xd + (int64_t)jb * BT * BT;
+    bc_times_x<T>(acc, pool, v, X, BT);
+    if constexpr (REFINE) {
+      T q[2][2][4];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) q[i][j][u] = acc.get(i, j, u);
+      bc_times_x<T>(acc, pool, q, W + (int64_t)j0 * (p.np + 1), p.np);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[i][j][u] = s_sub(v[i][j][u], acc.get(i, j, u));
+      bc_times_x<T>(acc, pool, v, X, BT);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[i][j][u] = s_add(q[i][j][u], acc.get(i, j, u));
+    } else {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[i][j][u] = acc.get(i, j, u);
+    }
+    T* Qj = Q + (int64_t)j0 * p.ldq;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int r = ri + 16 * i, c = cj + 16 * j + 4 * u;
+          if (r < rows && j0 + c < p.n) Qj[r + c * ldq] = v[i][j][u];
+        }
+    __syncthreads();  // the next block column reads this one in every wave
+  }
+}
+
+// kind 0: strip a of Q = Q1 - Q1 U, in place from the last block column to the
+// first; kind 1: tile (a, b), a <= b, of R = R1 + U R1, and zeros in (b, a);
+// between the passes, kind 2: the tile of R = R2 R1, kind 3: of R1 = R.
+template <typename T>
+__global__ void __launch_bounds__(256, BcCfg<T>::OCC)
+    bchol_correct_kernel(const BCholProb* P, const BCholTask* tasks, int pass) {
+  using C = BcCfg<T>;
+  __shared__ T pool[C::POOL];
+  const BCholTask t = tasks[blockIdx.x];
+  if (t.prob < 0) return;
+  const BCholProb p = P[t.prob];
+  if (bc_skip(p, pass)) return;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lr = lane & 15, lq = lane >> 4, wm = w & 1, wn = w >> 1;
+  const int ri = wm * 32 + lr, cj = wn * 32 + lq;
+  const T* U = reinterpret_cast<const T*>(p.U);
+  BcAcc<T> acc;
+  if (t.kind == 0) {
+    const int r0 = t.a * BT, rows = p.m - r0;
+    T* Q = reinterpret_cast<T*>(p.Q) + r0;
+    for (int jb = p.np / BT - 1; jb >= 0; --jb) {
+      const int j0 = jb * BT, ldq = bc_local(p.ldq);
+      acc.zero();
+      bc_product<T, false>(acc, pool, Q, ldq, rows, U + (int64_t)j0 * p.np, p.np, BT, min(j0 + BT, p.n));
+      T* Qj = Q + (int64_t)j0 * p.ldq;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int r = ri + 16 * i, c = cj + 16 * j + 4 * u;
+            if (r < rows && j0 + c < p.n) {
+              T* q = Qj + r + c * ldq;
+              *q = s_sub(*q, acc.get(i, j, u));
+            }
+          }
+    }
+    return;
+  }
+  const T* W = reinterpret_cast<const T*>(p.W);
+  T* R = reinterpret_cast<T*>(p.R);
+  const int i0 = t.a * BT, j0 = t.b * BT;
+  acc.zero();
+  if (t.kind == 3) {
+    T* Wij = reinterpret_cast<T*>(p.W) + i0 + (int64_t)j0 * p.np;
+    for (int e = threadIdx.x; e < BT * BT; e += 256) {
+      const int r = e % BT, c = e / BT;
+      if (i0 + r < p.n && j0 + c < p.n) Wij[r + (int64_t)c * p.np] = R[i0 + r + (int64_t)(j0 + c) * p.ldr];
+    }
+    return;
+  }
+  bc_product<T, false>(acc, pool, U + i0 + (int64_t)i0 * p.np, p.np, BT, W + i0 + (int64_t)j0 * p.np, p.np, BT,
+                       j0 + BT - i0);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int r = ri + 16 * i, c = cj + 16 * j + 4 * u;
+        const T w1 = t.kind == 2 ? s_zero(T()) : W[i0 + r + (int64_t)(j0 + c) * p.np];
+        const T v = s_add(w1, acc.get(i, j, u));
+        if (i0 + r < p.n && j0 + c < p.n) R[i0 + r + (int64_t)(j0 + c) * p.ldr] = i0 + r > j0 + c ? s_zero(T()) : v;
+        if (i0 < j0 && j0 + r < p.n && i0 + c < p.n) R[j0 + r + (int64_t)(i0 + c) * p.ldr] = s_zero(T());
+      }
+}
+
+}  // namespace
+
+void launch_bchol_init(int* state, unsigned long long* dev, int n, int* any, int* status, int nst, hipStream_t s) {
+  const int tot = std::max(std::max(n, nst), 1);
+  hipLaunchKernelGGL(bchol_init_kernel, dim3(cdiv(tot, 256)), dim3(256), 0, s, state, dev, n, any, status, nst);
+}
+void launch_bchol_decide(const BCholProb* P, int n, int* any, int pass, hipStream_t s) {
+  hipLaunchKernelGGL(bchol_decide_kernel, dim3(cdiv(n, 256)), dim3(256), 0, s, P, n, any, pass);
+}
+template <typename T>
+void launch_bchol(BCholPhase phase, const BCholProb* P, const BCholTask* tasks, int n, int pass, hipStream_t s) {
+  if (n <= 0) return;
+  const dim3 g(n), b(256);
+  switch (phase) {
+    case BCHOL_GRAM1: hipLaunchKernelGGL((bchol_gram_kernel<T, false>), g, b, 0, s, P, tasks, pass); break;
+    case BCHOL_FACTOR: hipLaunchKernelGGL((bchol_factor_kernel<T>), g, b, 0, s, P, tasks, pass); break;
+    case BCHOL_SOLVE: hipLaunchKernelGGL((bchol_solve_kernel<T, false>), g, b, 0, s, P, tasks, pass, pass == 2); break;
+    case BCHOL_RESOLVE: hipLaunchKernelGGL((bchol_solve_kernel<T, true>), g, b, 0, s, P, tasks, pass, 0); break;
+    case BCHOL_GRAM2: hipLaunchKernelGGL((bchol_gram_kernel<T, true>), g, b, 0, s, P, tasks, pass); break;
+    case BCHOL_CORRECT:
+    case BCHOL_COMPOSE: hipLaunchKernelGGL((bchol_correct_kernel<T>), g, b, 0, s, P, tasks, pass); break;
+  }
+}
+template void launch_bchol<double>(BCholPhase, const BCholProb*, const BCholTask*, int, int, hipStream_t);
+template void launch_bchol<zd>(BCholPhase, const BCholProb*, const BCholTask*, int, int, hipStream_t);
+
+}  // namespace mak

@@ -663,6 +663,7 @@ __global__ void __launch_bounds__(256) cholqr2_panel_tasks_kernel(const CholQrTa
   __shared__ int bad_s;
   __shared__ double dev_s[4];
   const CholQrTask tk = tasks[blockIdx.x];
+  if (tk.gate != nullptr && *tk.gate != 1) return;
   T* X = reinterpret_cast<T*>(tk.X);
   T* Q1 = reinterpret_cast<T*>(tk.Q1);
   const int64_t ldx = tk.ldx, ldq = tk.ldq;

@@ -52,10 +52,37 @@ struct CholQrTask {
   int64_t ldq;
   void* Tout;       // 32 x 32 T factor (ld 32)
   int* status;      // out: 0 accepted, 1 rejected (the Householder launches gated on it run)
+  const int* gate;  // optional: the task runs only if *gate == 1 (its block's CholeskyQR2 was rejected)
   int H;
   int nbc;
 };
 template <typename T> void launch_cholqr2_panel_tasks(const CholQrTask* tasks, int ntasks, hipStream_t s);
+
+// Whole blocks of a batch by CholeskyQR2 (mak_bchol.hip).
+constexpr int kBCholTile = 64;
+struct BCholProb {
+  const void* A;  // m x n, only read
+  int64_t lda;
+  void* Q;        // m x n
+  int64_t ldq;
+  void* R;        // n x n (written by the kind 1 tasks of BCHOL_CORRECT)
+  int64_t ldr;
+  void* W;        // np x np scratch: Gram matrix, then R1 (upper tiles)
+  void* U;        // np x np scratch: U (upper tiles)
+  void* X;        // np / 64 scratch blocks of 64 x 64: inverses of R1's diagonal tiles
+  int* state;     // out: 1 if the block is left to the gated Householder launches
+  unsigned long long* dev;  // bits of the largest squared tile norm of E
+  int m, n, np;   // np: n rounded up to a multiple of 64; m >= n >= 1
+};
+struct BCholTask {
+  int prob;  // < 0: nothing to do
+  int a, b, kind;
+};
+enum BCholPhase { BCHOL_GRAM1, BCHOL_FACTOR, BCHOL_SOLVE, BCHOL_RESOLVE, BCHOL_GRAM2, BCHOL_CORRECT, BCHOL_COMPOSE };
+void launch_bchol_init(int* state, unsigned long long* dev, int n, int* any, int* status, int nst, hipStream_t s);
+void launch_bchol_decide(const BCholProb* P, int n, int* any, int pass, hipStream_t s);
+template <typename T>
+void launch_bchol(BCholPhase phase, const BCholProb* P, const BCholTask* tasks, int n, int pass, hipStream_t s);
 
 constexpr int kMaxTreeLevels = 8;
 
