@@ -677,7 +677,8 @@ bool whole_block(const BProb& p) {
 int whole_np(const BProb& p) { return cdiv(p.n, kBCholTile) * kBCholTile; }
 template <typename T> size_t whole_elems(const BProb& p) {
   const size_t np = whole_np(p);
-  return 2 * np * np + np * kBCholTile;
+  const size_t nt = np / kBCholTile;
+  return 2 * np * np + np * kBCholTile + nt * nt;  // W, U, X, dev
 }
 
 // Task lists of the whole blocks (problem q of the list is P[idx[q]]).  Each
@@ -779,8 +780,8 @@ WholeLists whole_lists(const std::vector<BProb>& P, const std::vector<int>& idx,
 // CholeskyQR2 of the whole blocks; returns the number of launches.
 template <typename T>
 int enqueue_whole(const WholeLists& wl, const BCholProb* dprobs, const BCholTask* dtasks, int n, int* state,
-                  unsigned long long* dev, int* any, int* status, int nst, hipStream_t s) {
-  launch_bchol_init(state, dev, n, any, status, nst, s);
+                  int* any, int* status, int nst, hipStream_t s) {
+  launch_bchol_init(state, n, any, status, nst, s);
   for (const WholeLists::Launch& l : wl.launches) {
     if (l.phase == BCHOL_CORRECT) launch_bchol_decide(dprobs, n, any, l.pass, s);
     launch_bchol<T>(l.phase, dprobs, dtasks + l.off, l.cnt, l.pass, s);
@@ -863,9 +864,7 @@ struct Sizes {
            whole + wholeProbs + wholeTasks;
   }
 };
-// status area: one word per panel, then `any`; whole-block status area: the
-// largest tile norms, then the states
-inline size_t whole_status_bytes(size_t n) { return al256(n * (sizeof(unsigned long long) + sizeof(int))); }
+// status area: one word per panel, then `any`
 
 template <typename T>
 Sizes plan_sizes(const std::vector<BProb>& P, const std::vector<int>& batched, const std::vector<int>& fallback,
@@ -897,7 +896,7 @@ Sizes plan_sizes(const std::vector<BProb>& P, const std::vector<int>& batched, c
       we += whole_elems<T>(P[i]);
     }
   z.whole = al256(we * sizeof(T));
-  z.wholeProbs = al256(sizeof(BCholProb) * wi.size()) + whole_status_bytes(wi.size());
+  z.wholeProbs = al256(sizeof(BCholProb) * wi.size()) + al256(sizeof(int) * wi.size());  // and the states
   z.wholeTasks = wi.empty() ? 0 : al256(sizeof(BCholTask) * whole_lists(P, wi, true).tasks.size());
   z.tree = al256(sizeof(T) * kTreeElems * std::max<size_t>(ntall, 1));
   z.rfTasks = al256(sizeof(TsqrRootArgs) * std::max<size_t>(tall, 1));
@@ -1026,9 +1025,7 @@ int plan_create(BatchedQrPlan* pl, int count, const int* m, const int* n, void* 
   // whole blocks: scratch, status words and task lists
   BCholProb* dwp = reinterpret_cast<BCholProb*>(pl->ws + pl->offWholeProbs);
   BCholTask* dwt = reinterpret_cast<BCholTask*>(pl->ws + pl->offWholeTasks);
-  unsigned long long* wdev =
-      reinterpret_cast<unsigned long long*>(pl->ws + pl->offWholeProbs + al256(sizeof(BCholProb) * whole.size()));
-  int* wstate = reinterpret_cast<int*>(wdev + whole.size());
+  int* wstate = reinterpret_cast<int*>(pl->ws + pl->offWholeProbs + al256(sizeof(BCholProb) * whole.size()));
   const WholeLists wl = whole_lists(pl->probs, whole, false);
   if (!whole.empty()) {
     std::vector<BCholProb> wp;
@@ -1038,7 +1035,8 @@ int plan_create(BatchedQrPlan* pl, int count, const int* m, const int* n, void* 
       p.gate = wstate + q;
       const size_t np = whole_np(p);
       wp.push_back(BCholProb{p.A, p.lda, p.Q, p.ldq, p.R, p.ldr, wbase, wbase + np * np, wbase + 2 * np * np,
-                             wstate + q, wdev + q, p.m, p.n, (int)np});
+                             wstate + q,
+                             reinterpret_cast<double*>(wbase + 2 * np * np + np * kBCholTile), p.m, p.n, (int)np});
       wbase += whole_elems<T>(p);
     }
     if (hipMemcpy(dwp, wp.data(), sizeof(BCholProb) * wp.size(), hipMemcpyHostToDevice) != hipSuccess ||
@@ -1141,7 +1139,7 @@ int plan_create(BatchedQrPlan* pl, int count, const int* m, const int* n, void* 
   if (hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal) != hipSuccess) st = 1;
   if (!st) {
     if (!whole.empty())
-      pl->launches = enqueue_whole<T>(wl, dwp, dwt, (int)whole.size(), wstate, wdev, any, stBase, (int)npanels, cs);
+      pl->launches = enqueue_whole<T>(wl, dwp, dwt, (int)whole.size(), wstate, any, stBase, (int)npanels, cs);
     pl->launches += enqueue<T>(*pl, steps, qOff, qCnt, qFree, any, dprobs, pl->probs, (int)pl->batched.size(), dcq,
                                dnode, drf, dex, dapply, pl->nc, pl->gridMult * pl->cus, pl->positive, true, cs);
     if (hipStreamEndCapture(cs, &pl->graph) != hipSuccess) st = 1;

@@ -306,12 +306,9 @@ __device__ __forceinline__ int bc_local(int64_t ld) {
 }
 
 // Status words of a replay: nothing rejected, no panel rejected.
-__global__ void bchol_init_kernel(int* state, unsigned long long* dev, int n, int* any, int* status, int nst) {
+__global__ void bchol_init_kernel(int* state, int n, int* any, int* status, int nst) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < n) {
-    state[e] = 0;
-    dev[e] = 0ull;
-  }
+  if (e < n) state[e] = 0;
   if (e < nst) status[e] = 0;
   if (e == 0) *any = 0;
 }
@@ -319,21 +316,30 @@ __global__ void bchol_init_kernel(int* state, unsigned long long* dev, int n, in
 // States of a block: 0 factored in one pass, 2 in two, 1 rejected.
 __device__ __forceinline__ bool bc_skip(const BCholProb& p, int pass) { return *p.state != (pass == 2 ? 2 : 0); }
 
-// State after E of this pass; any |= rejected.
+// State after E of this pass; any |= rejected.  One wave per block sums the
+// squared norms of E's upper tiles, in a fixed order.  (nt^2 times their
+// maximum instead overestimates ||E||_F up to nt times: E sits in its last rows
+// and columns, and a set of 4096 Gaussian blocks then nearly always had one in
+// the second pass, 2.5 ms of 21.)
 __global__ void bchol_decide_kernel(const BCholProb* P, int n, int* any, int pass) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  const int e = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64, lane = threadIdx.x & 63;
   if (e >= n) return;
   const BCholProb p = P[e];
-  const int nt = p.np / BT;
-  const double s = __longlong_as_double((long long)*p.dev) * nt * nt;  // bounds ||E||_F^2
-  int st = *p.state;
+  const int nt = p.np / BT, st = *p.state;
   if (!bc_skip(p, pass)) {
-    if (pass == 1) st = s <= kBCholMaxE * kBCholMaxE ? 0 : s <= kBCholMaxE2 * kBCholMaxE2 ? 2 : 1;  // not a number: 1
-    else if (!(s <= kBCholMaxE * kBCholMaxE)) st = 1;
-    *p.state = st;
-    *p.dev = 0ull;
+    double s = 0.0;
+    for (int t = lane; t < nt * nt; t += 64)
+      if (t % nt <= t / nt) s += (t % nt < t / nt ? 2.0 : 1.0) * p.dev[t];
+    s = wave_sum(s);
+    const bool ok = s <= kBCholMaxE * kBCholMaxE;  // false for a NaN
+    const int to = ok ? st : pass == 1 && s <= kBCholMaxE2 * kBCholMaxE2 ? 2 : 1;
+    if (lane == 0) {
+      *p.state = to;
+      if (to == 1) *any = 1;  // every writer writes 1
+    }
+  } else if (st == 1 && lane == 0) {
+    *any = 1;
   }
-  if (st == 1) *any = 1;  // every writer writes 1
 }
 
 // Tile (a, b), a <= b: of A^H A in W, in the second pass of Q1^H Q1 in U
@@ -380,9 +386,7 @@ __global__ void __launch_bounds__(256, BcCfg<T>::OCC_GRAM)
     s2 = wave_sum(s2);
     if (lane == 0) part[w] = s2;
     __syncthreads();
-    // non-negative doubles order like their bits (and a NaN above them all)
-    if (threadIdx.x == 0)
-      atomicMax(p.dev, (unsigned long long)__double_as_longlong(fabs(part[0] + part[1] + part[2] + part[3])));
+    if (threadIdx.x == 0) p.dev[t.a + t.b * (p.np / BT)] = part[0] + part[1] + part[2] + part[3];
   }
 }
 
@@ -652,12 +656,12 @@ __global__ void __launch_bounds__(256, BcCfg<T>::OCC)
 
 }  // namespace
 
-void launch_bchol_init(int* state, unsigned long long* dev, int n, int* any, int* status, int nst, hipStream_t s) {
+void launch_bchol_init(int* state, int n, int* any, int* status, int nst, hipStream_t s) {
   const int tot = std::max(std::max(n, nst), 1);
-  hipLaunchKernelGGL(bchol_init_kernel, dim3(cdiv(tot, 256)), dim3(256), 0, s, state, dev, n, any, status, nst);
+  hipLaunchKernelGGL(bchol_init_kernel, dim3(cdiv(tot, 256)), dim3(256), 0, s, state, n, any, status, nst);
 }
 void launch_bchol_decide(const BCholProb* P, int n, int* any, int pass, hipStream_t s) {
-  hipLaunchKernelGGL(bchol_decide_kernel, dim3(cdiv(n, 256)), dim3(256), 0, s, P, n, any, pass);
+  hipLaunchKernelGGL(bchol_decide_kernel, dim3(cdiv(n, 4)), dim3(256), 0, s, P, n, any, pass);
 }
 template <typename T>
 void launch_bchol(BCholPhase phase, const BCholProb* P, const BCholTask* tasks, int n, int pass, hipStream_t s) {
