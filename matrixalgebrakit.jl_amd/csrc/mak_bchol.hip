@@ -119,6 +119,25 @@ template <> struct BcAcc<zd> {
   }
 };
 
+// One 16 x 16 block of a wave: row lane % 16, column 4 u + lane / 16.
+template <typename T> struct BcRow;
+template <> struct BcRow<double> {
+  v4d r;
+  __device__ __forceinline__ void zero() { r = v4d{0.0, 0.0, 0.0, 0.0}; }
+  __device__ __forceinline__ void step(double a, double b) { r = mfma_f64(b, a, r); }
+  __device__ __forceinline__ double get(int u) const { return r[u]; }
+};
+template <> struct BcRow<zd> {
+  v4d p, q, s;
+  __device__ __forceinline__ void zero() { p = q = s = v4d{0.0, 0.0, 0.0, 0.0}; }
+  __device__ __forceinline__ void step(const zd& a, const zd& b) {
+    p = mfma_f64(b.x, a.x, p);
+    q = mfma_f64(b.y, a.y, q);
+    s = mfma_f64(b.x + b.y, a.x + a.y, s);
+  }
+  __device__ __forceinline__ zd get(int u) const { return mkz(p[u] - q[u], s[u] - p[u] - q[u]); }
+};
+
 // acc += op(L) R over K inner indices, for a 64 x 64 tile:
 //   KL:  op(L)(i, k) = conj(L[k + i ldl]);  otherwise L[i + k ldl];
 //   R(k, j) = R[k + j ldr].
@@ -654,6 +673,250 @@ __global__ void __launch_bounds__(256, BcCfg<T>::OCC)
       }
 }
 
+// ---------------------------------------------------------------------------
+// One matrix with n <= m < 64 by one workgroup in LDS: the same CholeskyQR2,
+// and Householder QR (xGEQR2, xORG2R, gauge) in the same kernel when it is
+// rejected, so that the call stays a single launch without a host check.
+//   As  the matrix, then Q1, as [row][column] (rows >= m and columns >= n: 0)
+//   Wg  64 x 64 global scratch (R1)
+// Products with a factor on the right belong to one wave per 16 rows and need
+// no workgroup barrier.  What bounds it: latency of the two 32 x 32 in-wave
+// Choleskys (3 us each Float64) and of the ~10 steps between barriers.
+// ---------------------------------------------------------------------------
+constexpr int SP = 65;  // pitch of As
+
+// acc[j] (16 rows of the wave x 16 columns each) += As(rows, a0 + k) B(k, 16 j ..), k < 32
+template <typename T>
+__device__ __forceinline__ void small_rows_mm(BcRow<T> (&acc)[2], const T (*As)[SP], int a0, const T (*B)[33]) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lr = lane & 15, lq = lane >> 4;
+#pragma unroll
+  for (int kk = 0; kk < 32; kk += 4) {
+    const T a = As[16 * w + lr][a0 + kk + lq];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[j].step(a, B[kk + lq][16 * j + lr]);
+  }
+}
+
+template <typename T>
+__device__ __forceinline__ void small_householder(T (*As)[SP], T (*Qs)[SP], T* tau_s, const T* A, int64_t lda, T* Q,
+                                                  int64_t ldq, T* R, int64_t ldr, int m, int n) {
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  for (int e = tid; e < 64 * 64; e += 256) {
+    const int r = e % 64, c = e / 64;
+    As[r][c] = r < m && c < n ? A[r + (int64_t)c * lda] : s_zero(T());
+    Qs[r][c] = r == c ? s_one(T()) : s_zero(T());
+  }
+  __syncthreads();
+  for (int j = 0; j < n; ++j) {
+    // every wave forms the reflector; wave 0 stores it after the barrier
+    const T alpha = As[j][j];
+    const T x = lane > j ? As[lane][j] : s_zero(T());
+    const double nu2 = wave_sum(s_abs2(x));
+    const double bn = sqrt(s_abs2(alpha) + nu2);
+    T tau = s_zero(T()), beta = alpha, scale = s_zero(T());
+    if (!((nu2 == 0.0 && s_im(alpha) == 0.0) || !(bn > 0.0))) {
+      const double br = s_re(alpha) >= 0.0 ? -bn : bn;
+      beta = s_from_real<T>(br);
+      tau = s_scale(s_sub(beta, alpha), 1.0 / br);
+      scale = s_div(s_one(T()), s_sub(alpha, beta));
+    }
+    const T v = lane == j ? s_one(T()) : s_mul(x, scale);  // 0 above the diagonal
+    for (int c = j + 1 + w; c < n; c += 4) {
+      const T a = lane >= j ? As[lane][c] : s_zero(T());
+      const T d = s_mul(s_conj(tau), wave_sum(s_mul(s_conj(v), a)));
+      if (lane >= j) As[lane][c] = s_sub(a, s_mul(v, d));
+    }
+    __syncthreads();
+    if (w == 0 && lane >= j) As[lane][j] = lane == j ? beta : v;
+    if (tid == 0) tau_s[j] = tau;
+    __syncthreads();
+  }
+  for (int j = n - 1; j >= 0; --j) {
+    const T v = lane < j ? s_zero(T()) : lane == j ? s_one(T()) : As[lane][j];
+    const T tau = tau_s[j];
+    for (int c = j + w; c < n; c += 4) {
+      const T a = Qs[lane][c];
+      const T d = s_mul(tau, wave_sum(s_mul(s_conj(v), a)));
+      Qs[lane][c] = s_sub(a, s_mul(v, d));
+    }
+    __syncthreads();
+  }
+  for (int e = tid; e < 64 * n; e += 256) {
+    const int r = e % 64, c = e / 64;
+    if (r < m) Q[r + (int64_t)c * ldq] = s_mul(Qs[r][c], sign_safe(As[c][c]));
+    if (R != nullptr && r < n) {
+      T v = s_zero(T());
+      if (r == c) v = s_from_real<T>(s_absv(As[r][r]));
+      else if (r < c) v = s_mul(s_conj(sign_safe(As[r][r])), As[r][c]);
+      R[r + (int64_t)c * ldr] = v;
+    }
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) qr_small_kernel(const T* A, int64_t lda, T* Q, int64_t ldq, T* R, int64_t ldr,
+                                                       T* Wg, int* status, int m, int n) {
+  __shared__ T As[64][SP];
+  __shared__ T tiles[5][32][33];
+  __shared__ T tau_s[64];
+  __shared__ double part[4];
+  __shared__ int bad_s;
+  T (*S11)[33] = tiles[0];
+  T (*Y11)[33] = tiles[1];  // then U11
+  T (*S12)[33] = tiles[2];  // then Y22, U22
+  T (*W12)[33] = tiles[3];  // then U12
+  T (*S22)[33] = tiles[4];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int lr = lane & 15, lq = lane >> 4, wm = w & 1, wn = w >> 1;
+  const bool two = n > 32;  // a second block column
+  for (int e = tid; e < 64 * 64; e += 256) {
+    const int r = e % 64, c = e / 64;
+    As[r][c] = r < m && c < n ? A[r + (int64_t)c * lda] : s_zero(T());
+  }
+  if (tid == 0) bad_s = 0;
+  if (status != nullptr && tid < 8) status[tid] = 0;
+  __syncthreads();
+  // pass 0: G = A^H A to S11, S12, S22; pass 1: U from E = Q1^H Q1 - I to Y11, W12, S12
+  const bool quad = wm <= wn && (two || wn == 0);
+  for (int pass = 0; pass < 2; ++pass) {
+    double s2 = 0.0;
+    if (quad) {
+      BcAcc<T> acc;
+      acc.zero();
+      for (int kk = 0; kk < m; kk += 4) {
+        T a[2], b[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          a[i] = As[kk + lq][wm * 32 + 16 * i + lr];
+          b[i] = As[kk + lq][wn * 32 + 16 * i + lr];
+        }
+        acc.template step<true>(a, b);
+      }
+      T (*D)[33] = wn == 0 ? (pass ? Y11 : S11) : wm == 0 ? (pass ? W12 : S12) : (pass ? S12 : S22);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int r = 16 * i + lr, c = 16 * j + 4 * u + lq;
+            const int gr = wm * 32 + r, gc = wn * 32 + c;
+            T v = acc.get(i, j, u);
+            if (gr == gc) v = s_from_real<T>(gr >= n ? (pass ? 0.0 : 1.0) : s_re(v) - (pass ? 1.0 : 0.0));
+            if (pass) {
+              s2 += (wm < wn ? 2.0 : 1.0) * s_abs2(v);
+              v = gr > gc ? s_zero(T()) : gr == gc ? s_scale(v, 0.5) : v;
+            }
+            D[r][c] = v;
+          }
+    }
+    if (pass) {
+      s2 = wave_sum(s2);
+      if (lane == 0) part[w] = s2;
+    }
+    __syncthreads();
+    if (pass) break;
+    for (int h = 0; h < (two ? 2 : 1); ++h) {
+      if (w == 0) {
+        const int bad = wave_chol_inv32<T>(h ? S22 : S11, h ? S12 : Y11);
+        if (bad && lane == 0) bad_s = 1;
+      }
+      __syncthreads();
+      if (h == 0 && two) {
+        mm32<T>(W12, Y11, true, S12, false, 1.0, false);
+        mm32<T>(S22, W12, true, W12, false, -1.0, true);
+      }
+    }
+    // R1 to the scratch; Q1 = A R1^{-1} by rows
+    if (R != nullptr)
+      for (int e = tid; e < 64 * 64; e += 256) {
+        const int r = e % 64, c = e / 64;
+        T v = s_zero(T());
+        if (r <= c && c < (two ? 64 : 32)) v = c < 32 ? S11[r][c] : r < 32 ? W12[r][c - 32] : S22[r - 32][c - 32];
+        Wg[e] = v;
+      }
+    BcRow<T> q[2];
+    q[0].zero();
+    q[1].zero();
+    small_rows_mm<T>(q, As, 0, Y11);
+    wave_lds_sync();
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) As[16 * w + lr][16 * j + 4 * u + lq] = q[j].get(u);
+    wave_lds_sync();
+    if (two) {
+      q[0].zero();
+      q[1].zero();
+      small_rows_mm<T>(q, As, 0, W12);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          T* p = &As[16 * w + lr][32 + 16 * j + 4 * u + lq];
+          *p = s_sub(*p, q[j].get(u));
+        }
+      wave_lds_sync();
+      q[0].zero();
+      q[1].zero();
+      small_rows_mm<T>(q, As, 32, S12);
+      wave_lds_sync();
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) As[16 * w + lr][32 + 16 * j + 4 * u + lq] = q[j].get(u);
+    }
+    __syncthreads();
+  }
+  const double dev = part[0] + part[1] + part[2] + part[3];
+  if (bad_s || !(dev <= kBCholMaxE * kBCholMaxE)) {  // uniform
+    __syncthreads();
+    small_householder<T>(As, reinterpret_cast<T (*)[SP]>(&tiles[0][0][0]), tau_s, A, lda, Q, ldq, R, ldr, m, n);
+    return;
+  }
+  // Q = Q1 - Q1 U
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if (h == 1 && !two) break;
+    BcRow<T> q[2];
+    q[0].zero();
+    q[1].zero();
+    small_rows_mm<T>(q, As, 0, h ? W12 : Y11);
+    if (h) small_rows_mm<T>(q, As, 32, S12);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int r = 16 * w + lr, c = 32 * h + 16 * j + 4 * u + lq;
+        if (r < m && c < n) Q[r + (int64_t)c * ldq] = s_sub(As[r][c], q[j].get(u));
+      }
+  }
+  if (R == nullptr) return;
+  // R = R1 + U R1, wave w its rows 16 w ..
+  __syncthreads();
+  for (int e = tid; e < 64 * 64; e += 256) As[e % 64][e / 64] = Wg[e];
+  __syncthreads();
+  for (int jp = 0; jp < (two ? 2 : 1); ++jp) {
+    BcRow<T> q[2];
+    q[0].zero();
+    q[1].zero();
+    for (int kk = 16 * w / 32 * 32; kk < 32 * (jp + 1); kk += 4) {
+      const int i = 16 * w + lr, k = kk + lq;
+      const T a = i >= 32 ? S12[i - 32][k - 32] : k < 32 ? Y11[i][k] : W12[i][k - 32];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) q[j].step(a, As[k][32 * jp + 16 * j + lr]);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int r = 16 * w + lr, c = 32 * jp + 16 * j + 4 * u + lq;
+        if (r < n && c < n) R[r + (int64_t)c * ldr] = r <= c ? s_add(As[r][c], q[j].get(u)) : s_zero(T());
+      }
+  }
+}
+
 }  // namespace
 
 void launch_bchol_init(int* state, int n, int* any, int* status, int nst, hipStream_t s) {
@@ -679,5 +942,17 @@ void launch_bchol(BCholPhase phase, const BCholProb* P, const BCholTask* tasks, 
 }
 template void launch_bchol<double>(BCholPhase, const BCholProb*, const BCholTask*, int, int, hipStream_t);
 template void launch_bchol<zd>(BCholPhase, const BCholProb*, const BCholTask*, int, int, hipStream_t);
+
+
+template <typename T>
+void launch_qr_small(const T* A, int64_t lda, T* Q, int64_t ldq, T* R, int64_t ldr, T* scratch, int* status, int m,
+                     int n, hipStream_t s) {
+  hipLaunchKernelGGL((qr_small_kernel<T>), dim3(1), dim3(256), 0, s, A, lda, Q, ldq, R, ldr, scratch, status,
+                     m, n);
+}
+template void launch_qr_small<double>(const double*, int64_t, double*, int64_t, double*, int64_t, double*, int*, int,
+                                      int, hipStream_t);
+template void launch_qr_small<zd>(const zd*, int64_t, zd*, int64_t, zd*, int64_t, zd*, int*, int, int,
+                                  hipStream_t);
 
 }  // namespace mak

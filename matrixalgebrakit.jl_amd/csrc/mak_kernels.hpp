@@ -83,6 +83,11 @@ void launch_bchol_init(int* state, int n, int* any, int* status, int nst, hipStr
 void launch_bchol_decide(const BCholProb* P, int n, int* any, int pass, hipStream_t s);
 template <typename T>
 void launch_bchol(BCholPhase phase, const BCholProb* P, const BCholTask* tasks, int n, int pass, hipStream_t s);
+// qr_compact! with positive = true of one matrix, n <= m < 64; scratch: 64 x 64;
+// status: eight words cleared, or null
+template <typename T>
+void launch_qr_small(const T* A, int64_t lda, T* Q, int64_t ldq, T* R, int64_t ldr, T* scratch, int* status, int m,
+                     int n, hipStream_t s);
 
 constexpr int kMaxTreeLevels = 8;
 

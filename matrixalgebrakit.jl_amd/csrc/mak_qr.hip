@@ -597,6 +597,14 @@ int qr_driver(hipStream_t s, int full, int m, int n, T* A, int64_t lda, T* Q, in
   if (work == nullptr || work_bytes < need) return -11;
   char* ws = reinterpret_cast<char*>(work);
   QrLayout<T> L = qr_layout<T>(m, n, qcols);
+  // Below the rows of a CholeskyQR2 panel one workgroup does everything in LDS
+  // (one launch instead of 22 and no Householder panel of 33 dependent
+  // columns).
+  if (!full && positive && Tout == nullptr && m >= n && n > 0 && m < kCholQrMinRows) {
+    launch_qr_small<T>(A, lda, Q, ldq, R, ldr, reinterpret_cast<T*>(ws + L.offWp),
+                       L.offCq2 ? cholqr2_status<T>(ws + L.offCq2, m, n) : nullptr, m, n, s);
+    return hipGetLastError() == hipSuccess ? 0 : 1;
+  }
   if (L.offCq2) zero_ints(cholqr2_status<T>(ws + L.offCq2, m, n), 8, s);
   if (L.offFlags) zero_ints(reinterpret_cast<int*>(ws + L.offFlags), 3, s);
   if (minmn == 0) {
