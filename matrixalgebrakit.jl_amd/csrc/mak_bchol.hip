@@ -43,6 +43,7 @@ namespace {
 
 constexpr int BT = kBCholTile;  // 64
 constexpr double kBCholMaxE = 1e-8, kBCholMaxE2 = 0.1;
+constexpr double kTallMaxE = 1e-6;
 
 // LDS of one stage of a tile product: KB inner indices of the two operands.
 // The pitches keep the fragment reads (16 rows x 4 k of a wave) off each
@@ -409,6 +410,56 @@ __global__ void __launch_bounds__(256, BcCfg<T>::OCC_GRAM)
   }
 }
 
+// Cholesky with inverse of a 64 x 64 Hermitian matrix by 256 threads: its upper
+// 32 x 32 blocks in S[0], S[64], S[128] (rows of 33; S[32], S[96] scratch) become
+// R (W, ld) and R^{-1} (X, ld 64) with zeros below the diagonal.  True if a
+// pivot was not positive.  The blocks were written before a barrier here.
+template <typename T>
+__device__ __forceinline__ bool bc_chol64(T (*S)[33], int* bad_s, T* W, int64_t ld, T* X) {
+  T (*S11)[33] = S;
+  T (*Y11)[33] = S + 32;
+  T (*S12)[33] = S + 64;  // then Y22
+  T (*W12)[33] = S + 96;
+  T (*S22)[33] = S + 128;  // then W12 Y22
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (threadIdx.x == 0) *bad_s = 0;
+  __syncthreads();
+  if (w == 0) {
+    const int bad = wave_chol_inv32<T>(S11, Y11);
+    if (bad && lane == 0) *bad_s = 1;
+  }
+  __syncthreads();
+  mm32<T>(W12, Y11, true, S12, false, 1.0, false);
+  mm32<T>(S22, W12, true, W12, false, -1.0, true);
+  if (w == 0) {
+    const int bad = wave_chol_inv32<T>(S22, S12);
+    if (bad && lane == 0) *bad_s = 1;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < BT * BT; e += 256) {
+    const int i = e % BT, j = e / BT;
+    T wv = s_zero(T()), xv = s_zero(T());
+    if (j < 32) {
+      if (i < 32) {
+        wv = S11[i][j];
+        xv = Y11[i][j];
+      }
+    } else if (i < 32) {
+      wv = W12[i][j - 32];
+    } else {
+      wv = S22[i - 32][j - 32];
+      xv = S12[i - 32][j - 32];
+    }
+    W[i + (int64_t)j * ld] = wv;
+    if (i >= 32 || j < 32) X[e] = xv;
+  }
+  __syncthreads();
+  mm32<T>(S22, W12, false, S12, false, 1.0, false);
+  mm32<T>(S22, Y11, false, S22, false, -1.0, false);
+  for (int e = threadIdx.x; e < 32 * 32; e += 256) X[e % 32 + (32 + e / 32) * BT] = S22[e % 32][e / 32];
+  return *bad_s != 0;
+}
+
 // Step k of the factorisation of G: tile R_kb and its term of diagonal tile b,
 // then for b = k + 1 the factor of that tile (k = -1: only that).  The diagonal tile of 64 is factored with its
 // inverse as 32 x 32 blocks by wave 0.
@@ -454,10 +505,6 @@ __global__ void __launch_bounds__(256) bchol_factor_kernel(const BCholProb* P, c
   // S = G_bb - sum_i<=k R_ib^H R_ib, one term per step: kept in G_bb, or for the
   // next diagonal block in three 32 x 32 blocks of the pool
   T (*S11)[33] = reinterpret_cast<T (*)[33]>(pool);
-  T (*Y11)[33] = S11 + 32;
-  T (*S12)[33] = S11 + 64;  // then Y22
-  T (*W12)[33] = S11 + 96;
-  T (*S22)[33] = S11 + 128;  // then W12 Y22
   T* Wbb = W + (int64_t)b * BT * (ld + 1);
   acc.zero();
   if (k >= 0) bc_product<T, true>(acc, pool, Wb + k * BT, ld, BT, Wb + k * BT, ld, BT, BT);
@@ -475,7 +522,7 @@ __global__ void __launch_bounds__(256) bchol_factor_kernel(const BCholProb* P, c
     return;
   }
   if (wm <= wn) {
-    T (*S)[33] = wn == 0 ? S11 : wm == 0 ? S12 : S22;
+    T (*S)[33] = S11 + 64 * (wm + wn);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -485,43 +532,8 @@ __global__ void __launch_bounds__(256) bchol_factor_kernel(const BCholProb* P, c
           S[16 * i + lr][16 * j + 4 * u + lq] =
               s_sub(Wbb[ri + 16 * i + (int64_t)(cj + 16 * j + 4 * u) * ld], acc.get(i, j, u));
   }
-  if (threadIdx.x == 0) bad_s = 0;
-  __syncthreads();
-  if (w == 0) {
-    const int bad = wave_chol_inv32<T>(S11, Y11);
-    if (bad && lane == 0) bad_s = 1;
-  }
-  __syncthreads();
-  mm32<T>(W12, Y11, true, S12, false, 1.0, false);
-  mm32<T>(S22, W12, true, W12, false, -1.0, true);
-  if (w == 0) {
-    const int bad = wave_chol_inv32<T>(S22, S12);
-    if (bad && lane == 0) bad_s = 1;
-  }
-  __syncthreads();
-  T* Xb = Xd + (int64_t)b * BT * BT;
-  for (int e = threadIdx.x; e < BT * BT; e += 256) {
-    const int i = e % BT, j = e / BT;
-    T wv = s_zero(T()), xv = s_zero(T());
-    if (j < 32) {
-      if (i < 32) {
-        wv = S11[i][j];
-        xv = Y11[i][j];
-      }
-    } else if (i < 32) {
-      wv = W12[i][j - 32];
-    } else {
-      wv = S22[i - 32][j - 32];
-      xv = S12[i - 32][j - 32];
-    }
-    Wbb[i + (int64_t)j * ld] = wv;
-    if (i >= 32 || j < 32) Xb[e] = xv;
-  }
-  __syncthreads();
-  mm32<T>(S22, W12, false, S12, false, 1.0, false);
-  mm32<T>(S22, Y11, false, S22, false, -1.0, false);
-  for (int e = threadIdx.x; e < 32 * 32; e += 256) Xb[e % 32 + (32 + e / 32) * BT] = S22[e % 32][e / 32];
-  if (threadIdx.x == 0 && bad_s) *p.state = 1;
+  const bool bad = bc_chol64<T>(S11, &bad_s, Wbb, ld, Xd + (int64_t)b * BT * BT);
+  if (threadIdx.x == 0 && bad) *p.state = 1;
 }
 
 // Strip a (64 rows) of Q1 = A R1^{-1}; second: of Q1 <- Q1 R2^{-1}, in place.
@@ -917,6 +929,247 @@ __global__ void __launch_bounds__(256) qr_small_kernel(const T* A, int64_t lda, 
   }
 }
 
+// ---------------------------------------------------------------------------
+// One matrix with m >= 64 rows and n < 64 columns: CholeskyQR2 in three
+// launches.  Workgroup s has rows s rps ..; the last one of a launch to finish
+// sums the partial Gram matrices in order and does the 64 x 64 work:
+//   0  partial A^H A;            R1 (W), R1^{-1} (X)
+//   1  Q1 = A R1^{-1}, partial Q1^H Q1;   U, D = (I + U)^{-1} - I, R = (I + U) R1
+//   2  Q = Q1 + Q1 D
+// What bounds it: latency (1024 x 32 Float64: 23, 20 and 7 us, most of it the
+// 64 x 64 work of one workgroup).  U to second order in E (as in mak_cholqr2.hip) where ||E||_F > 1e-9; accepted
+// (*state = 0) up to 1e-6.
+// ---------------------------------------------------------------------------
+struct TallArgs {
+  const void* A;
+  int64_t lda;
+  void* Q;
+  int64_t ldq;
+  void* R;
+  int64_t ldr;
+  void *part, *W, *X, *D;  // gridDim.x blocks of 64 x 64; 64 x 64 each
+  int* ctl;                // state (1 until accepted), a ticket per launch; set by the caller to 1, 0, 0
+  int m, n, rps;
+};
+
+template <typename T, int PASS>
+__global__ void __launch_bounds__(256) qr_tall_kernel(const TallArgs p) {
+  using C = BcCfg<T>;
+  __shared__ T pool[C::POOL > 5 * 32 * 33 ? C::POOL : 5 * 32 * 33];
+  __shared__ double red[4];
+  __shared__ int flag_s, bad_s;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int lr = lane & 15, lq = lane >> 4, wm = w & 1, wn = w >> 1;
+  const int ri = wm * 32 + lr, cj = wn * 32 + lq;
+  const int r0 = blockIdx.x * p.rps, rows = min(p.rps, p.m - r0), n = p.n;
+  const T* A = reinterpret_cast<const T*>(p.A) + r0;
+  T* Q = reinterpret_cast<T*>(p.Q) + r0;
+  T* X = reinterpret_cast<T*>(p.X);
+  T* W = reinterpret_cast<T*>(p.W);
+  BcAcc<T> acc;
+  if constexpr (PASS == 1) {
+    if (p.ctl[3]) return;  // G was not positive definite
+    for (int b0 = 0; b0 < rows; b0 += BT) {
+      T v[2][2][4];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int r = b0 + ri + 16 * i, c = cj + 16 * j + 4 * u;
+            v[i][j][u] = r < rows && c < n ? A[r + (int64_t)c * p.lda] : s_zero(T());
+          }
+      bc_times_x<T>(acc, pool, v, X, BT);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int r = b0 + ri + 16 * i, c = cj + 16 * j + 4 * u;
+            if (r < rows && c < n) Q[r + (int64_t)c * p.ldq] = acc.get(i, j, u);
+          }
+    }
+    __syncthreads();
+  }
+  {
+    const T* G = PASS == 0 ? A : Q;
+    const int64_t ld = PASS == 0 ? p.lda : p.ldq;
+    acc.zero();
+    bc_product<T, true>(acc, pool, G, ld, n, G, ld, n, rows);
+  }
+  // upper 32 x 32 blocks of the partial
+  const bool quad = wm <= wn && 32 * wn < n;
+  T* part = reinterpret_cast<T*>(p.part) + (int64_t)blockIdx.x * BT * BT;
+  if (quad)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) part[ri + 16 * i + (cj + 16 * j + 4 * u) * BT] = acc.get(i, j, u);
+  __threadfence();
+  __syncthreads();
+  if (tid == 0) flag_s = atomicAdd(p.ctl + 1 + PASS, 1) == (int)gridDim.x - 1;
+  __syncthreads();
+  if (!flag_s) return;
+  __threadfence();
+  // blocks 11, 12, 22 of the sum to S[0], S[64], S[128]; PASS 1: of U1 = up(E)
+  T (*S)[33] = reinterpret_cast<T (*)[33]>(pool);
+  const T* P0 = reinterpret_cast<const T*>(p.part);
+  double s2 = 0.0;
+  for (int e = tid; e < 3 * 32 * 32; e += 256) {
+    const int q = e >> 10, r = e & 31, c = (e >> 5) & 31;
+    const int gr = (q == 2 ? 32 : 0) + r, gc = (q ? 32 : 0) + c;
+    T v = s_zero(T());
+    if (gc < n && gr < n)
+      for (int k = 0; k < (int)gridDim.x; k += 16) {
+        T x[16];  // 16 loads in flight
+#pragma unroll
+        for (int h = 0; h < 16; ++h)
+          x[h] = P0[(int64_t)min(k + h, (int)gridDim.x - 1) * BT * BT + gr + gc * BT];
+#pragma unroll
+        for (int h = 0; h < 16; ++h) v = k + h < (int)gridDim.x ? s_add(v, x[h]) : v;
+      }
+    if (gr == gc) v = s_from_real<T>(gr >= n ? (PASS ? 0.0 : 1.0) : s_re(v) - (PASS ? 1.0 : 0.0));
+    if (PASS) {
+      s2 += (q == 1 ? 2.0 : 1.0) * s_abs2(v);
+      v = gr > gc ? s_zero(T()) : gr == gc ? s_scale(v, 0.5) : v;
+    }
+    S[64 * q + r][c] = v;
+  }
+  if constexpr (PASS == 0) {
+    const bool bad = bc_chol64<T>(S, &bad_s, W, BT, X);
+    if (tid == 0) p.ctl[3] = bad;
+  } else {
+    s2 = wave_sum(s2);
+    if (lane == 0) red[w] = s2;
+    __syncthreads();
+    const double dev = red[0] + red[1] + red[2] + red[3];
+    if (!(dev <= kTallMaxE * kTallMaxE)) return;  // rejected
+    T (*U11)[33] = S;
+    T (*T1)[33] = S + 32;
+    T (*U12)[33] = S + 64;
+    T (*T2)[33] = S + 96;
+    T (*U22)[33] = S + 128;
+    T* D = reinterpret_cast<T*>(p.D);
+    const bool two = n > 32, second = dev > 1e-18;
+    if (second) {  // U = up(E - U1^H U1): E's halves are U1
+      auto up_sub = [&](T (*U)[33], T (*N)[33], bool diag) {
+        for (int e = tid; e < 32 * 32; e += 256) {
+          const int r = e & 31, c = e >> 5;
+          if (!diag || r < c) U[r][c] = s_sub(U[r][c], N[r][c]);
+          else if (r == c) U[r][c] = s_from_real<T>(s_re(U[r][c]) - 0.5 * s_re(N[r][c]));
+        }
+        __syncthreads();
+      };
+      if (two) {
+        mm32<T>(T2, U12, true, U12, false, 1.0, false);
+        mm32<T>(T2, U22, true, U22, false, 1.0, true);
+        mm32<T>(T1, U11, true, U12, false, 1.0, false);
+        up_sub(U22, T2, true);
+        up_sub(U12, T1, false);
+      }
+      mm32<T>(T1, U11, true, U11, false, 1.0, false);
+      up_sub(U11, T1, true);
+    }
+    // D = -U + U^2, block by block; R = R1 + U R1
+    auto put_d = [&](T (*U)[33], T (*N)[33], int i0, int j0) {
+      for (int e = tid; e < 32 * 32; e += 256) {
+        const int r = e & 31, c = e >> 5;
+        const T v = second ? s_sub(N[r][c], U[r][c]) : s_neg(U[r][c]);
+        D[i0 + r + (j0 + c) * BT] = v;
+      }
+      __syncthreads();
+    };
+    if (second) mm32<T>(T1, U11, false, U11, false, 1.0, false);
+    put_d(U11, T1, 0, 0);
+    for (int e = tid; e < 32 * 32; e += 256) {  // below the diagonal blocks
+      D[32 + (e & 31) + (e >> 5) * BT] = s_zero(T());
+      if (!two) {
+        D[(e & 31) + (32 + (e >> 5)) * BT] = s_zero(T());
+        D[32 + (e & 31) + (32 + (e >> 5)) * BT] = s_zero(T());
+      }
+    }
+    if (two) {
+      if (second) {
+        mm32<T>(T1, U11, false, U12, false, 1.0, false);
+        mm32<T>(T1, U12, false, U22, false, 1.0, true);
+        mm32<T>(T2, U22, false, U22, false, 1.0, false);
+      }
+      put_d(U12, T1, 0, 32);
+      put_d(U22, T2, 32, 32);
+    }
+    if (p.R != nullptr) {
+      T* R = reinterpret_cast<T*>(p.R);
+      auto get_w = [&](T (*N)[33], int i0, int j0) {
+        __syncthreads();
+        for (int e = tid; e < 32 * 32; e += 256) N[e & 31][e >> 5] = W[i0 + (e & 31) + (j0 + (e >> 5)) * BT];
+        __syncthreads();
+      };
+      // R block = N (+ N0), zeros below the diagonal
+      auto put_r = [&](T (*N)[33], T (*N0)[33], int i0, int j0) {
+        for (int e = tid; e < 32 * 32; e += 256) {
+          const int r = e & 31, c = e >> 5;
+          const T v = i0 + r <= j0 + c ? s_add(N[r][c], N0[r][c]) : s_zero(T());
+          if (i0 + r < n && j0 + c < n) R[i0 + r + (int64_t)(j0 + c) * p.ldr] = v;
+        }
+      };
+      get_w(T2, 0, 0);
+      mm32<T>(T1, U11, false, T2, false, 1.0, false);
+      put_r(T1, T2, 0, 0);
+      if (two) {
+        for (int e = tid; e < 32 * 32; e += 256)
+          if (32 + (e & 31) < n) R[32 + (e & 31) + (int64_t)(e >> 5) * p.ldr] = s_zero(T());
+        get_w(T2, 0, 32);
+        mm32<T>(T1, U11, false, T2, false, 1.0, false);
+        for (int e = tid; e < 32 * 32; e += 256) T1[e & 31][e >> 5] = s_add(T1[e & 31][e >> 5], T2[e & 31][e >> 5]);
+        get_w(T2, 32, 32);
+        mm32<T>(U11, U12, false, T2, false, 1.0, false);
+        put_r(T1, U11, 0, 32);
+        __syncthreads();
+        mm32<T>(T1, U22, false, T2, false, 1.0, false);
+        put_r(T1, T2, 32, 32);
+      }
+    }
+    if (tid == 0) p.ctl[0] = 0;
+  }
+}
+
+// Q = Q1 + Q1 D, 64 rows a workgroup
+template <typename T> __global__ void __launch_bounds__(256) qr_tall_correct_kernel(const TallArgs p) {
+  using C = BcCfg<T>;
+  __shared__ T pool[C::POOL];
+  if (p.ctl[0]) return;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lr = lane & 15, lq = lane >> 4, wm = w & 1, wn = w >> 1;
+  const int r0 = blockIdx.x * BT, rows = p.m - r0;
+  T* Q = reinterpret_cast<T*>(p.Q) + r0;
+  BcAcc<T> acc;
+  acc.zero();
+  bc_product<T, false>(acc, pool, Q, p.ldq, rows, reinterpret_cast<const T*>(p.D), BT, BT, p.n);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int r = wm * 32 + lr + 16 * i, c = wn * 32 + lq + 16 * j + 4 * u;
+        if (r < rows && c < p.n) {
+          T* q = Q + r + (int64_t)c * p.ldq;
+          *q = s_add(*q, acc.get(i, j, u));
+        }
+      }
+}
+
+__global__ void qr_tall_init_kernel(int* ctl, int* status, int* flags) {
+  const int t = threadIdx.x;
+  if (t < 4) ctl[t] = t == 0;
+  if (t < 8 && status != nullptr) status[t] = 0;
+  if (t < 3 && flags != nullptr) flags[t] = 0;
+}
+
 }  // namespace
 
 void launch_bchol_init(int* state, int n, int* any, int* status, int nst, hipStream_t s) {
@@ -953,6 +1206,23 @@ void launch_qr_small(const T* A, int64_t lda, T* Q, int64_t ldq, T* R, int64_t l
 template void launch_qr_small<double>(const double*, int64_t, double*, int64_t, double*, int64_t, double*, int*, int,
                                       int, hipStream_t);
 template void launch_qr_small<zd>(const zd*, int64_t, zd*, int64_t, zd*, int64_t, zd*, int*, int, int,
+                                  hipStream_t);
+
+template <typename T>
+void qr_tall_enqueue(const T* A, int64_t lda, T* Q, int64_t ldq, T* R, int64_t ldr, T* scratch, int* status,
+                     int* flags, int m, int n, hipStream_t s) {
+  const int rps = cdiv(cdiv(m, kTallMaxWgs), BT) * BT, wgs = cdiv(m, rps);
+  T* W = scratch + kTallCtlElems;
+  const TallArgs a{A, lda, Q, ldq, R, ldr, W + 3 * BT * BT, W, W + BT * BT, W + 2 * BT * BT,
+                   reinterpret_cast<int*>(scratch), m, n, rps};
+  hipLaunchKernelGGL(qr_tall_init_kernel, dim3(1), dim3(64), 0, s, a.ctl, status, flags);
+  hipLaunchKernelGGL((qr_tall_kernel<T, 0>), dim3(wgs), dim3(256), 0, s, a);
+  hipLaunchKernelGGL((qr_tall_kernel<T, 1>), dim3(wgs), dim3(256), 0, s, a);
+  hipLaunchKernelGGL((qr_tall_correct_kernel<T>), dim3(cdiv(m, BT)), dim3(256), 0, s, a);
+}
+template void qr_tall_enqueue<double>(const double*, int64_t, double*, int64_t, double*, int64_t, double*, int*, int*,
+                                      int, int, hipStream_t);
+template void qr_tall_enqueue<zd>(const zd*, int64_t, zd*, int64_t, zd*, int64_t, zd*, int*, int*, int, int,
                                   hipStream_t);
 
 }  // namespace mak

@@ -72,6 +72,13 @@ template <typename T> TreePlan plan_tree(int H, int nbc, size_t base) {
 constexpr int kCholQrMinRows = 64;
 // Columns from which the whole-matrix CholeskyQR2 path is tried first.
 constexpr int kCholQr2MinN = 64;
+// Rows up to which narrower matrices take the three-launch CholeskyQR2: one
+// workgroup sums its partial Gram matrices, and 64 workgroups do not fill the
+// chip.  Against the panels (us a call): 1024 x 32 Float64 164 -> 93,
+// 8192 x 63 310 -> 179, 8192 x 32 177 -> 127; 32768 x 32 230 -> 216 and ComplexF64
+// 385 -> 398, 131072 x 16 383 -> 439.  An input that it rejects (||E||_F > 1e-6,
+// condition numbers from about 1e5) pays the attempt: 512 x 32 201 -> 266.
+constexpr int kTallMaxM = 1 << 14;
 
 template <typename T> struct QrLayout {
   size_t offTpanels = 0;  // NB*NB per panel
@@ -605,6 +612,23 @@ int qr_driver(hipStream_t s, int full, int m, int n, T* A, int64_t lda, T* Q, in
                        L.offCq2 ? cholqr2_status<T>(ws + L.offCq2, m, n) : nullptr, m, n, s);
     return hipGetLastError() == hipSuccess ? 0 : 1;
   }
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cs) != hipSuccess) cs = hipStreamCaptureStatusActive;
+  // m >= 64 > n: CholeskyQR2 in three launches, each summing its partial Gram
+  // matrices in its last workgroup (8 to 10 launches on panels)
+  if (!full && positive && Tout == nullptr && n > 0 && n < kCholQr2MinN && m >= kCholQrMinRows && m <= kTallMaxM &&
+      std::max(lda, ldq) <= (1 << 20) && (int64_t)L.wpElems >= kTallScratchElems &&
+      cs == hipStreamCaptureStatusNone) {
+    T* scratch = reinterpret_cast<T*>(ws + L.offWp);
+    qr_tall_enqueue<T>(A, lda, Q, ldq, R, ldr, scratch,
+                       L.offCq2 ? cholqr2_status<T>(ws + L.offCq2, m, n) : nullptr,
+                       L.offFlags ? reinterpret_cast<int*>(ws + L.offFlags) : nullptr, m, n, s);
+    int st = 1;
+    if (hipMemcpyAsync(&st, scratch, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess)
+      return 1;
+    if (st == 0) return hipGetLastError() == hipSuccess ? 0 : 1;
+  }
   if (L.offCq2) zero_ints(cholqr2_status<T>(ws + L.offCq2, m, n), 8, s);
   if (L.offFlags) zero_ints(reinterpret_cast<int*>(ws + L.offFlags), 3, s);
   if (minmn == 0) {
@@ -612,8 +636,6 @@ int qr_driver(hipStream_t s, int full, int m, int n, T* A, int64_t lda, T* Q, in
     if (R) qr_extract_r<T>(A, lda, R, ldr, rrows, n, 0, 0, s);
     return hipGetLastError() == hipSuccess ? 0 : 1;
   }
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &cs) != hipSuccess) cs = hipStreamCaptureStatusActive;
   // Whole-matrix CholeskyQR2 first (A is only read; a rejected input goes on
   // to the Householder path below); the trailing columns of qr_full! and the
   // Householder signs of positive = false follow from its Q.  The signs are
