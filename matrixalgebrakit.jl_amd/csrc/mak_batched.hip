@@ -311,9 +311,9 @@ __global__ void __launch_bounds__(256) apply_wy_tasks_kernel(const ApplyTask* ta
 }
 
 // Per-problem elementwise passes (grid.y = problem, grid.x strides elements).
-template <typename T> __global__ void batched_identity_kernel(const BProb* P) {
-  const BProb p = P[blockIdx.y];
-  if (p.gate != nullptr && *p.gate != 1) return;
+// Ungated problems one per blockIdx.y; gated ones (any != nullptr) by a small
+// grid that returns at once if none was rejected.
+template <typename T> __device__ void identity_of(const BProb& p) {
   const int k = min(p.m, p.n);
   T* Q = reinterpret_cast<T*>(p.Q);
   const int64_t tot = (int64_t)p.m * k;
@@ -323,9 +323,7 @@ template <typename T> __global__ void batched_identity_kernel(const BProb* P) {
   }
 }
 
-template <typename T> __global__ void batched_finalize_kernel(const BProb* P, int positive) {
-  const BProb p = P[blockIdx.y];
-  if (p.gate != nullptr && *p.gate != 1) return;
+template <typename T> __device__ void finalize_of(const BProb& p, int positive) {
   const int k = min(p.m, p.n);
   const T* A = reinterpret_cast<const T*>(p.A);
   T* Q = reinterpret_cast<T*>(p.Q);
@@ -348,6 +346,19 @@ template <typename T> __global__ void batched_finalize_kernel(const BProb* P, in
       Q[r + c * p.ldq] = s_mul(Q[r + c * p.ldq], sign_safe(A[c + c * p.lda]));
     }
   }
+}
+
+template <typename T>
+__global__ void batched_identity_kernel(const BProb* P, int n, const int* any) {
+  if (any != nullptr && *any == 0) return;
+  for (int i = blockIdx.y; i < n; i += gridDim.y)
+    if (P[i].gate == nullptr || *P[i].gate == 1) identity_of<T>(P[i]);
+}
+template <typename T>
+__global__ void batched_finalize_kernel(const BProb* P, int n, const int* any, int positive) {
+  if (any != nullptr && *any == 0) return;
+  for (int i = blockIdx.y; i < n; i += gridDim.y)
+    if (P[i].gate == nullptr || *P[i].gate == 1) finalize_of<T>(P[i], positive);
 }
 
 // deterministic pseudo-random fill of a tuning arena (values only steer no branch)
@@ -477,6 +488,11 @@ void build_tasks(const std::vector<BProb>& P, const std::vector<int>& idx, const
     while (off + c < (int)apply.size() && apply[off + c].gate == nullptr) ++c;
     return c;
   };
+  // Gated tasks rarely run: all in the class of the tallest nodes, one launch a
+  // step instead of three (5 us each).
+  auto node_cls = [&](const BProb& p, int H) {
+    return p.gate == nullptr ? cls_of(H) : cls_of(node_cap<T>());
+  };
   for (int s = 0; s < S; ++s) {
     const int j0 = s * NB;
     // CholeskyQR2 tasks of the step's panels of at least kCqMinRows rows
@@ -512,7 +528,7 @@ void build_tasks(const std::vector<BProb>& P, const std::vector<int>& idx, const
         T* A = reinterpret_cast<T*>(p.A);
         T* Ap = A + j0 + (int64_t)j0 * p.lda;
         if (H <= cap) {
-          if (cls_of(H) != cls) continue;
+          if (node_cls(p, H) != cls) continue;
           NodeTask t{};
           t.X = Ap;
           t.ldx = p.lda;
@@ -527,7 +543,7 @@ void build_tasks(const std::vector<BProb>& P, const std::vector<int>& idx, const
           const int H1 = L * nbc;
           for (int leaf = 0; leaf < L; ++leaf) {
             const int r0 = (int)(((int64_t)leaf * H) / L), r1 = (int)(((int64_t)(leaf + 1) * H) / L);
-            if (cls_of(r1 - r0) != cls) continue;
+            if (node_cls(p, r1 - r0) != cls) continue;
             NodeTask t{};
             t.X = Ap + r0;
             t.ldx = p.lda;
@@ -793,7 +809,7 @@ int enqueue_whole(const WholeLists& wl, const BCholProb* dprobs, const BCholTask
 template <typename T>
 int enqueue(const BatchedQrPlan& pl, const std::vector<BatchedQrPlan::Step>& steps, const std::vector<int>& qOff,
             const std::vector<int>& qCnt, const std::vector<int>& qFree, const int* any, const BProb* dprobs,
-            const std::vector<BProb>& P, int nprob_batched,
+            const std::vector<BProb>& P, int nprob_batched, int ngated,
             const CholQrTask* dcq, const NodeTask* dnode, const TsqrRootArgs* drf, const TsqrExpandArgs* dex,
             const ApplyTask* dapply, int nc, int grid, int positive, bool with_fallback, hipStream_t s) {
   int launches = 0;
@@ -818,20 +834,25 @@ int enqueue(const BatchedQrPlan& pl, const std::vector<BatchedQrPlan::Step>& ste
       ++launches;
     }
   }
-  if (nprob_batched > 0) {
-    hipLaunchKernelGGL((batched_identity_kernel<T>), dim3(64, nprob_batched), dim3(256), 0, s, dprobs);
-    ++launches;
-  }
+  // the ungated problems, then the gated ones
+  const int nfree = nprob_batched - ngated;
+  auto each_part = [&](auto&& launch) {
+    if (nfree > 0) launch(dim3(64, nfree), dprobs, nfree, (const int*)nullptr);
+    if (ngated > 0) launch(dim3(64, std::min(ngated, 64)), dprobs + nfree, ngated, any);
+    launches += (nfree > 0) + (ngated > 0);
+  };
+  each_part([&](dim3 g, const BProb* P0, int n, const int* a) {
+    hipLaunchKernelGGL((batched_identity_kernel<T>), g, dim3(256), 0, s, P0, n, a);
+  });
   for (int st = (int)steps.size() - 1; st >= 0; --st) {
     if (qCnt[st]) {
       launch_apply<T>(dapply + qOff[st], qCnt[st], qFree[st], any, nc, 0, grid, s);
       ++launches;
     }
   }
-  if (nprob_batched > 0) {
-    hipLaunchKernelGGL((batched_finalize_kernel<T>), dim3(64, nprob_batched), dim3(256), 0, s, dprobs, positive);
-    ++launches;
-  }
+  each_part([&](dim3 g, const BProb* P0, int n, const int* a) {
+    hipLaunchKernelGGL((batched_finalize_kernel<T>), g, dim3(256), 0, s, P0, n, a, positive);
+  });
   if (with_fallback) {
     for (int i : pl.fallback) {
       const BProb& p = P[i];
@@ -1103,7 +1124,7 @@ int plan_create(BatchedQrPlan* pl, int count, const int* m, const int* n, void* 
       for (int rep = 0; rep < 2; ++rep) {
         hipLaunchKernelGGL((arena_fill_kernel<T>), dim3(1024), dim3(256), 0, ts, ar, (int64_t)ao);
         hipEventRecord(e0, ts);
-        enqueue<T>(*pl, steps, qOff, qCnt, qFree, any, dprobs_arena, AP, (int)panels.size(), dcq, dnode, drf, dex,
+        enqueue<T>(*pl, steps, qOff, qCnt, qFree, any, dprobs_arena, AP, (int)panels.size(), 0, dcq, dnode, drf, dex,
                    dapply, c.first, c.second * pl->cus, pl->positive, false, ts);
         hipEventRecord(e1, ts);
         hipEventSynchronize(e1);
@@ -1140,7 +1161,8 @@ int plan_create(BatchedQrPlan* pl, int count, const int* m, const int* n, void* 
   if (!st) {
     if (!whole.empty())
       pl->launches = enqueue_whole<T>(wl, dwp, dwt, (int)whole.size(), wstate, any, stBase, (int)npanels, cs);
-    pl->launches += enqueue<T>(*pl, steps, qOff, qCnt, qFree, any, dprobs, pl->probs, (int)pl->batched.size(), dcq,
+    pl->launches += enqueue<T>(*pl, steps, qOff, qCnt, qFree, any, dprobs, pl->probs, (int)pl->batched.size(),
+                               (int)whole.size(), dcq,
                                dnode, drf, dex, dapply, pl->nc, pl->gridMult * pl->cus, pl->positive, true, cs);
     if (hipStreamEndCapture(cs, &pl->graph) != hipSuccess) st = 1;
   }
