@@ -14,7 +14,8 @@
  *     caller's stream wait for it with an event before it returns); no call
  *     synchronises the device or other streams.  Some calls wait for their
  *     own stream to read a small status word back to the host:
- *       mak_qr_*           once per call (the CholeskyQR2 acceptance check),
+ *       mak_qr_*           once per call (the CholeskyQR2 acceptance check;
+ *                          not for m < 64, which is one launch),
  *                          twice when the whole-matrix CholeskyQR2 result is
  *                          rejected; under stream capture never (the gated
  *                          form is enqueued instead);
@@ -62,7 +63,7 @@ extern "C" {
 int mak_qr_workspace_size(int dtype, int full, int m, int n, size_t* bytes);
 
 /* qr_compact!(A, (Q, R), Householder(; positive)) for Float64 / ComplexF64.
- * A (m x n) is destroyed (it holds the compact WY factors afterwards),
+ * A (m x n) is destroyed (its contents are undefined afterwards),
  * Q is m x min(m,n), R is min(m,n) x n or NULL (R not computed).
  * positive != 0 gives R a real non-negative diagonal (gauge fix).
  * The factors are FP64-accurate; on the whole-matrix CholeskyQR2 path the
@@ -84,7 +85,7 @@ int mak_qr_full_z(void* stream, int m, int n, void* A, int lda, void* Q, int ldq
                   int positive, void* work, size_t work_bytes);
 
 /* qr_compact! as the primal of the reverse rule: like mak_qr_compact_{d,z}, and
- * additionally keeps the compact WY factors the adjoint re-forms Q from: on
+ * additionally keeps the compact WY factors through which Q enters the adjoint: on
  * return A holds V (strictly below the diagonal) and R' (Householder signs),
  * Tout (32 x 32 x ceil(min(m,n)/32), column-major per panel) the T blocks.
  * Replaces the primal call inside rrule(::typeof(qr_compact!), A, QR, alg)
@@ -325,8 +326,12 @@ int mak_left_polar_pullback_z(void* stream, int batch, int m, int n, const void*
  * builds the task lists in the caller's workspace, optionally autotunes the
  * apply kernel (tune != 0: the workspace then also holds a scratch copy of the
  * shapes; results are cached per shape set for the process), and captures the
- * whole launch sequence in a hipGraph.  A_i is overwritten (compact WY form),
- * R may be NULL (no R) or hold NULL entries.
+ * whole launch sequence in a hipGraph.  A_i is destroyed (its contents are
+ * undefined afterwards), R may be NULL (no R) or hold NULL entries.
+ * With positive != 0, blocks with m_i >= n_i and m_i >= 64 are factored whole
+ * by CholeskyQR2 (condition numbers to about 1e7); the others, and blocks that
+ * it rejects on the device, by 32-column panels.  The workspace holds about
+ * 2 n_i^2 elements for each such block.
  * No counterpart in the reference, which has no batched API: it replaces a
  * caller's loop of qr_compact! over blocks (src/implementations/qr.jl:110-113). */
 typedef struct mak_qr_batched_plan mak_qr_batched_plan;

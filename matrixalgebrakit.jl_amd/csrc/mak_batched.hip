@@ -707,9 +707,20 @@ struct WholeLists {
     int off, cnt, pass;
   };
   std::vector<BCholTask> tasks;
+  size_t count = 0;
   std::vector<Launch> launches;
 };
-WholeLists whole_lists(const std::vector<BProb>& P, const std::vector<int>& idx, bool all_r) {
+// One queue of a launch's tasks; counted only, for the size query.
+struct WholeQueue {
+  std::vector<BCholTask> tasks;
+  size_t n = 0;
+  bool count_only = false;
+  void push_back(const BCholTask& t) {
+    if (!count_only) tasks.push_back(t);
+    ++n;
+  }
+};
+WholeLists whole_lists(const std::vector<BProb>& P, const std::vector<int>& idx, bool all_r, bool count_only) {
   constexpr int NQ = 8;
   WholeLists out;
   std::vector<int> queue(idx.size());
@@ -723,36 +734,44 @@ WholeLists whole_lists(const std::vector<BProb>& P, const std::vector<int>& idx,
     load[best] += cdiv(p.m, kBCholTile) * (double)kBCholTile * np * np;
     ntmax = std::max(ntmax, (int)np / kBCholTile);
   }
-  std::vector<BCholTask> lists[NQ];
+  WholeQueue lists[NQ];
+  for (auto& l : lists) l.count_only = count_only;
   auto flush = [&](BCholPhase phase) {
     size_t longest = 0;
-    for (auto& l : lists) longest = std::max(longest, l.size());
-    const int off = (int)out.tasks.size();
-    for (size_t t = 0; t < longest; ++t)
-      for (auto& l : lists) out.tasks.push_back(t < l.size() ? l[t] : BCholTask{-1, 0, 0, 0});
-    for (auto& l : lists) l.clear();
-    if (longest) out.launches.push_back({phase, off, (int)out.tasks.size() - off, 1});
+    for (auto& l : lists) longest = std::max(longest, l.n);
+    const int off = (int)out.count;
+    if (!count_only) {
+      out.tasks.resize(out.count + longest * NQ, BCholTask{-1, 0, 0, 0});
+      for (int q = 0; q < NQ; ++q)
+        for (size_t t = 0; t < lists[q].n; ++t) out.tasks[off + t * NQ + q] = lists[q].tasks[t];
+    }
+    out.count += longest * NQ;
+    for (auto& l : lists) {
+      l.tasks.clear();
+      l.n = 0;
+    }
+    if (longest) out.launches.push_back({phase, off, (int)(longest * NQ), 1});
   };
   auto each = [&](auto&& f) {
     for (size_t q = 0; q < idx.size(); ++q)
       f((int)q, P[idx[q]], whole_np(P[idx[q]]) / kBCholTile, lists[queue[q]]);
   };
-  auto gram = [&](int q, const BProb&, int nt, std::vector<BCholTask>& l) {
+  auto gram = [&](int q, const BProb&, int nt, WholeQueue& l) {
     for (int b = 0; b < nt; ++b)
       for (int a = 0; a <= b; ++a) l.push_back({q, a, b, 0});
   };
-  auto strips = [&](int q, const BProb& p, int, std::vector<BCholTask>& l) {
+  auto strips = [&](int q, const BProb& p, int, WholeQueue& l) {
     for (int a = 0; a * kBCholTile < p.m; ++a) l.push_back({q, a, 0, 0});
   };
   each(gram);
   flush(BCHOL_GRAM1);
   for (int k = -1; k < ntmax - 1; ++k) {
     // the task that goes on to factor the next diagonal tile first
-    each([&](int q, const BProb&, int nt, std::vector<BCholTask>& l) {
+    each([&](int q, const BProb&, int nt, WholeQueue& l) {
       if (k + 1 < nt) l.push_back({q, k, k + 1, 0});
     });
     if (k >= 0)
-      each([&](int q, const BProb&, int nt, std::vector<BCholTask>& l) {
+      each([&](int q, const BProb&, int nt, WholeQueue& l) {
         for (int b = k + 2; b < nt; ++b) l.push_back({q, k, b, 0});
       });
     flush(BCHOL_FACTOR);
@@ -763,7 +782,7 @@ WholeLists whole_lists(const std::vector<BProb>& P, const std::vector<int>& idx,
   flush(BCHOL_GRAM2);
   each(strips);
   auto r_tiles = [&](int kind) {
-    each([&](int q, const BProb& p, int nt, std::vector<BCholTask>& l) {
+    each([&](int q, const BProb& p, int nt, WholeQueue& l) {
       if (!all_r && p.R == nullptr) return;
       for (int b = 0; b < nt; ++b)
         for (int a = 0; a <= b; ++a) l.push_back({q, a, b, kind});
@@ -918,7 +937,7 @@ Sizes plan_sizes(const std::vector<BProb>& P, const std::vector<int>& batched, c
     }
   z.whole = al256(we * sizeof(T));
   z.wholeProbs = al256(sizeof(BCholProb) * wi.size()) + al256(sizeof(int) * wi.size());  // and the states
-  z.wholeTasks = wi.empty() ? 0 : al256(sizeof(BCholTask) * whole_lists(P, wi, true).tasks.size());
+  z.wholeTasks = wi.empty() ? 0 : al256(sizeof(BCholTask) * whole_lists(P, wi, true, true).count);
   z.tree = al256(sizeof(T) * kTreeElems * std::max<size_t>(ntall, 1));
   z.rfTasks = al256(sizeof(TsqrRootArgs) * std::max<size_t>(tall, 1));
   z.exTasks = al256(sizeof(TsqrExpandArgs) * std::max<size_t>(tall, 1));
@@ -1047,7 +1066,7 @@ int plan_create(BatchedQrPlan* pl, int count, const int* m, const int* n, void* 
   BCholProb* dwp = reinterpret_cast<BCholProb*>(pl->ws + pl->offWholeProbs);
   BCholTask* dwt = reinterpret_cast<BCholTask*>(pl->ws + pl->offWholeTasks);
   int* wstate = reinterpret_cast<int*>(pl->ws + pl->offWholeProbs + al256(sizeof(BCholProb) * whole.size()));
-  const WholeLists wl = whole_lists(pl->probs, whole, false);
+  const WholeLists wl = whole_lists(pl->probs, whole, false, false);
   if (!whole.empty()) {
     std::vector<BCholProb> wp;
     T* wbase = reinterpret_cast<T*>(pl->ws + pl->offWhole);

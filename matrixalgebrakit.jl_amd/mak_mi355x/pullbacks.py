@@ -4,10 +4,10 @@ Mirrors MatrixAlgebraKit's pullback API (declared public in
 src/MatrixAlgebraKit.jl:69-75):
 
 * ``qr_pullback_(dA, A, (Q, R), (dQ, dR), tape=...)`` adds the pullback of
-  ``qr_compact(A; positive=true)`` to dA (src/pullbacks/qr.jl:73-120).  Q is
-  re-formed on the device from the compact WY factors kept by
-  :func:`qr_compact_rrule` (the primal of the rule, cf.
-  ext/MatrixAlgebraKitChainRulesCoreExt.jl:26-43) instead of being read back.
+  ``qr_compact(A; positive=true)`` to dA (src/pullbacks/qr.jl:73-120).  Q
+  enters through the compact WY factors kept by :func:`qr_compact_rrule` (the
+  primal of the rule, cf. ext/MatrixAlgebraKitChainRulesCoreExt.jl:26-43); it is
+  neither read nor formed.
 * ``left_polar_pullback_(dA, A, (W, P), (dW, dP))`` and
   ``right_polar_pullback_(dA, A, (P, Wh), (dP, dWh))``
   (src/pullbacks/polar.jl:7-59).
