@@ -233,8 +233,8 @@ __device__ inline void st_coh(zd* p, zd v) {
 }
 
 // ---------------------------------------------------------------- tile I/O
-// Fast path (real data, a tile entirely inside the matrix, even leading
-// dimension, 16-byte aligned base): thread t moves rows 4 (t % 8) .. +3 of
+// Fast path (a tile entirely inside the matrix, 16-byte aligned base, real
+// data: even leading dimension): thread t moves rows 4 (t % 8) .. +3 of
 // column t / 8 with two 16-byte coherent (sc1) accesses, so a wave touches
 // four 256-byte column segments instead of 256 separate 8-byte locations.
 // Loads of up to three tiles are issued in one asm block and waited for
@@ -242,12 +242,16 @@ __device__ inline void st_coh(zd* p, zd v) {
 typedef double v2d __attribute__((ext_vector_type(2)));
 
 template <typename T> __device__ inline bool tile_fast(const T* M, int64_t ld, int n, int ti, int tj) {
-  if constexpr (ScalarTraits<T>::is_complex) {
-    return false;
-  } else {
-    return (ti + 1) * TB <= n && (tj + 1) * TB <= n && (ld & 1) == 0 &&
-           (reinterpret_cast<uintptr_t>(M) & 15) == 0;
-  }
+  return (ti + 1) * TB <= n && (tj + 1) * TB <= n && (ScalarTraits<T>::is_complex || (ld & 1) == 0) &&
+         (reinterpret_cast<uintptr_t>(M) & 15) == 0;
+}
+// Complex data: thread t moves rows t % 8 + 8 i (i < 4) of column t / 8, one
+// element a 16-byte access, so eight lanes share a 128-byte line.  (Element
+// loads of two coherent 8-byte halves waited once per element of a thread:
+// four round trips a tile.)
+__device__ inline const zd* tile_chunk(const zd* M, int64_t ld, int ti, int tj) {
+  const int t = threadIdx.x;
+  return M + (int64_t)(tj * TB + (t >> 3)) * ld + ti * TB + (t & 7);
 }
 __device__ inline const double* tile_chunk(const double* M, int64_t ld, int ti, int tj) {
   const int t = threadIdx.x;
@@ -300,6 +304,80 @@ __device__ inline void store_fast(const double (*S)[33], double* M, int64_t ld, 
   asm volatile("global_store_dwordx4 %0, %1, off sc1" :: "v"(p), "v"(a) : "memory");
   asm volatile("global_store_dwordx4 %0, %1, off offset:16 sc1" :: "v"(p), "v"(b) : "memory");
 }
+__device__ inline void put_chunk(zd (*S)[33], v2d a, v2d b, v2d c, v2d d) {
+  const int t = threadIdx.x;
+  const int col = t >> 3, r = t & 7;
+  S[r][col] = mkz(a.x, a.y);
+  S[r + 8][col] = mkz(b.x, b.y);
+  S[r + 16][col] = mkz(c.x, c.y);
+  S[r + 24][col] = mkz(d.x, d.y);
+}
+#define MAK_ZLOAD4(o0, o1, o2, o3, p)                                                              \
+  "global_load_dwordx4 " o0 ", " p ", off sc1\n\tglobal_load_dwordx4 " o1 ", " p ", off offset:128 sc1\n\t" \
+  "global_load_dwordx4 " o2 ", " p ", off offset:256 sc1\n\tglobal_load_dwordx4 " o3 ", " p               \
+  ", off offset:384 sc1\n\t"
+__device__ inline void load_fast1(zd (*S)[33], const zd* p) {
+  v2d a, b, c, d;
+  asm volatile(MAK_ZLOAD4("%0", "%1", "%2", "%3", "%4") "s_waitcnt vmcnt(0)"
+               : "=&v"(a), "=&v"(b), "=&v"(c), "=&v"(d) : "v"(p) : "memory");
+  put_chunk(S, a, b, c, d);
+}
+__device__ inline void load_fast2(zd (*S0)[33], const zd* p0, zd (*S1)[33], const zd* p1) {
+  v2d a, b, c, d, e, f, g, h;
+  asm volatile(MAK_ZLOAD4("%0", "%1", "%2", "%3", "%8") MAK_ZLOAD4("%4", "%5", "%6", "%7", "%9")
+               "s_waitcnt vmcnt(0)"
+               : "=&v"(a), "=&v"(b), "=&v"(c), "=&v"(d), "=&v"(e), "=&v"(f), "=&v"(g), "=&v"(h)
+               : "v"(p0), "v"(p1) : "memory");
+  put_chunk(S0, a, b, c, d);
+  put_chunk(S1, e, f, g, h);
+}
+__device__ inline void load_fast3(zd (*S0)[33], const zd* p0, zd (*S1)[33], const zd* p1, zd (*S2)[33],
+                                  const zd* p2) {
+  v2d a, b, c, d, e, f, g, h, i, j, k, l;
+  asm volatile(MAK_ZLOAD4("%0", "%1", "%2", "%3", "%12") MAK_ZLOAD4("%4", "%5", "%6", "%7", "%13")
+               MAK_ZLOAD4("%8", "%9", "%10", "%11", "%14") "s_waitcnt vmcnt(0)"
+               : "=&v"(a), "=&v"(b), "=&v"(c), "=&v"(d), "=&v"(e), "=&v"(f), "=&v"(g), "=&v"(h), "=&v"(i),
+                 "=&v"(j), "=&v"(k), "=&v"(l)
+               : "v"(p0), "v"(p1), "v"(p2) : "memory");
+  put_chunk(S0, a, b, c, d);
+  put_chunk(S1, e, f, g, h);
+  put_chunk(S2, i, j, k, l);
+}
+// real and imaginary parts of four or five tiles in flight would take the
+// registers of the task's products: two batches
+__device__ inline void load_fast4(zd (*S0)[33], const zd* p0, zd (*S1)[33], const zd* p1, zd (*S2)[33], const zd* p2,
+                                  zd (*S3)[33], const zd* p3) {
+  load_fast2(S0, p0, S1, p1);
+  load_fast2(S2, p2, S3, p3);
+}
+__device__ inline void load_fast5(zd (*S0)[33], const zd* p0, zd (*S1)[33], const zd* p1, zd (*S2)[33], const zd* p2,
+                                  zd (*S3)[33], const zd* p3, zd (*S4)[33], const zd* p4) {
+  load_fast3(S0, p0, S1, p1, S2, p2);
+  load_fast2(S3, p3, S4, p4);
+}
+#undef MAK_ZLOAD4
+__device__ inline void store4z(zd* p, const v2d& a, const v2d& b, const v2d& c, const v2d& d) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc1" :: "v"(p), "v"(a) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off offset:128 sc1" :: "v"(p), "v"(b) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off offset:256 sc1" :: "v"(p), "v"(c) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off offset:384 sc1" :: "v"(p), "v"(d) : "memory");
+}
+__device__ inline void store_fast(const zd (*S)[33], zd* M, int64_t ld, int ti, int tj) {
+  const int t = threadIdx.x;
+  const int col = t >> 3, r = t & 7;
+  auto at = [&](int i) {
+    const zd v = S[r + 8 * i][col];
+    v2d a;
+    a.x = v.x;
+    a.y = v.y;
+    return a;
+  };
+  store4z(const_cast<zd*>(tile_chunk(M, ld, ti, tj)), at(0), at(1), at(2), at(3));
+}
+__device__ inline void zero_fast(zd* M, int64_t ld, int ti, int tj) {
+  const v2d z = {0.0, 0.0};
+  store4z(const_cast<zd*>(tile_chunk(M, ld, ti, tj)), z, z, z, z);
+}
 __device__ inline void zero_fast(double* M, int64_t ld, int ti, int tj) {
   double* p = const_cast<double*>(tile_chunk(M, ld, ti, tj));
   v2d z = {0.0, 0.0};
@@ -311,10 +389,17 @@ __device__ inline void zero_fast(double* M, int64_t ld, int ti, int tj) {
 // the identity (diagonal tiles) or zero.
 template <typename T>
 __device__ inline void load_tile(T (*S)[33], const T* M, int64_t ld, int n, int ti, int tj) {
-  for (int e = threadIdx.x; e < TB * TB; e += 256) {
-    const int r = e % TB, c = e / TB;
-    const int gr = ti * TB + r, gc = tj * TB + c;
-    S[r][c] = (gr < n && gc < n) ? ld_coh(M + gr + (int64_t)gc * ld) : (gr == gc ? s_one(T()) : s_zero(T()));
+  T v[TB * TB / 256];  // all loads before the first use
+#pragma unroll
+  for (int u = 0; u < TB * TB / 256; ++u) {
+    const int e = threadIdx.x + 256 * u;
+    const int gr = ti * TB + e % TB, gc = tj * TB + e / TB;
+    v[u] = (gr < n && gc < n) ? ld_coh(M + gr + (int64_t)gc * ld) : (gr == gc ? s_one(T()) : s_zero(T()));
+  }
+#pragma unroll
+  for (int u = 0; u < TB * TB / 256; ++u) {
+    const int e = threadIdx.x + 256 * u;
+    S[e % TB][e / TB] = v[u];
   }
 }
 template <typename T>
@@ -339,47 +424,17 @@ struct TileSrc {
   int64_t ld;
   int ti, tj;
 };
-template <typename T>
-__device__ inline void load_tiles(int cnt, T (*S0)[33], TileSrc s0, T (*S1)[33], TileSrc s1, T (*S2)[33], TileSrc s2,
-                                  int n) {
-  const T* M0 = reinterpret_cast<const T*>(s0.M);
-  const T* M1 = reinterpret_cast<const T*>(s1.M);
-  const T* M2 = reinterpret_cast<const T*>(s2.M);
-  bool fast = tile_fast<T>(M0, s0.ld, n, s0.ti, s0.tj);
-  if (cnt > 1) fast = fast && tile_fast<T>(M1, s1.ld, n, s1.ti, s1.tj);
-  if (cnt > 2) fast = fast && tile_fast<T>(M2, s2.ld, n, s2.ti, s2.tj);
-  if constexpr (!ScalarTraits<T>::is_complex) {
-    if (fast) {
-      const double* p0 = tile_chunk(M0, s0.ld, s0.ti, s0.tj);
-      if (cnt == 1) {
-        load_fast1(S0, p0);
-      } else if (cnt == 2) {
-        load_fast2(S0, p0, S1, tile_chunk(M1, s1.ld, s1.ti, s1.tj));
-      } else {
-        load_fast3(S0, p0, S1, tile_chunk(M1, s1.ld, s1.ti, s1.tj), S2, tile_chunk(M2, s2.ld, s2.ti, s2.tj));
-      }
-      return;
-    }
-  }
-  load_tile<T>(S0, M0, s0.ld, n, s0.ti, s0.tj);
-  if (cnt > 1) load_tile<T>(S1, M1, s1.ld, n, s1.ti, s1.tj);
-  if (cnt > 2) load_tile<T>(S2, M2, s2.ld, n, s2.ti, s2.tj);
-}
 template <typename T> __device__ inline void put_tile(const T (*S)[33], T* M, int64_t ld, int n, int ti, int tj) {
-  if constexpr (!ScalarTraits<T>::is_complex) {
-    if (tile_fast<T>(M, ld, n, ti, tj)) {
-      store_fast(S, M, ld, ti, tj);
-      return;
-    }
+  if (tile_fast<T>(M, ld, n, ti, tj)) {
+    store_fast(S, M, ld, ti, tj);
+    return;
   }
   store_tile<T>(S, M, ld, n, ti, tj);
 }
 template <typename T> __device__ inline void clear_tile(T* M, int64_t ld, int n, int ti, int tj) {
-  if constexpr (!ScalarTraits<T>::is_complex) {
-    if (tile_fast<T>(M, ld, n, ti, tj)) {
-      zero_fast(M, ld, ti, tj);
-      return;
-    }
+  if (tile_fast<T>(M, ld, n, ti, tj)) {
+    zero_fast(M, ld, ti, tj);
+    return;
   }
   zero_tile<T>(M, ld, n, ti, tj);
 }
@@ -436,18 +491,16 @@ __device__ inline void load_n(T (*S0)[33], TileSrc s0, T (*S1)[33], TileSrc s1, 
   if constexpr (CNT > 2) fast = fast && fast_of(s2);
   if constexpr (CNT > 3) fast = fast && fast_of(s3);
   if constexpr (CNT > 4) fast = fast && fast_of(s4);
-  if constexpr (!ScalarTraits<T>::is_complex) {
-    if (fast) {
-      auto chunk = [&](const TileSrc& q) {
-        return tile_chunk(reinterpret_cast<const double*>(q.M), q.ld, q.ti, q.tj);
-      };
-      if constexpr (CNT == 1) load_fast1(S0, chunk(s0));
-      else if constexpr (CNT == 2) load_fast2(S0, chunk(s0), S1, chunk(s1));
-      else if constexpr (CNT == 3) load_fast3(S0, chunk(s0), S1, chunk(s1), S2, chunk(s2));
-      else if constexpr (CNT == 4) load_fast4(S0, chunk(s0), S1, chunk(s1), S2, chunk(s2), S3, chunk(s3));
-      else load_fast5(S0, chunk(s0), S1, chunk(s1), S2, chunk(s2), S3, chunk(s3), S4, chunk(s4));
-      return;
-    }
+  if (fast) {
+    auto chunk = [&](const TileSrc& q) {
+      return tile_chunk(reinterpret_cast<const T*>(q.M), q.ld, q.ti, q.tj);
+    };
+    if constexpr (CNT == 1) load_fast1(S0, chunk(s0));
+    else if constexpr (CNT == 2) load_fast2(S0, chunk(s0), S1, chunk(s1));
+    else if constexpr (CNT == 3) load_fast3(S0, chunk(s0), S1, chunk(s1), S2, chunk(s2));
+    else if constexpr (CNT == 4) load_fast4(S0, chunk(s0), S1, chunk(s1), S2, chunk(s2), S3, chunk(s3));
+    else load_fast5(S0, chunk(s0), S1, chunk(s1), S2, chunk(s2), S3, chunk(s3), S4, chunk(s4));
+    return;
   }
   auto slow = [&](T (*S)[33], const TileSrc& q) {
     load_tile<T>(S, reinterpret_cast<const T*>(q.M), q.ld, n, q.ti, q.tj);
