@@ -641,7 +641,29 @@ __device__ inline void y_task(const CholTileArgs& a, int K, int r, int half, T* 
   const int kmid = (kall / 2 + 15) / 16 * 16;
   const int kbeg = half == 2 ? kmid : 0;
   const int kend = half == 1 ? kmid : kall;
+  // Whole slabs are loaded without predicates: rows of B and columns of Xc
+  // beyond the matrix repeat its last one (their products are not stored), and
+  // a load is a uniform base plus a byte offset formed once per task.
+  uint32_t oa[NA], ox[NB];
+#pragma unroll
+  for (int u = 0; u < NA; ++u)
+    oa[u] = (uint32_t)sizeof(T) * ((uint32_t)(min(m0 + (tid & (BM - 1)), a.m - 1) - m0) +
+                                   (uint32_t)((tid / BM) + (256 / BM) * u) * (uint32_t)a.ldb);
+#pragma unroll
+  for (int u = 0; u < NB; ++u)
+    ox[u] = (uint32_t)sizeof(T) * ((uint32_t)(tid & 15) +
+                                   (uint32_t)(min(n0 + (tid >> 4) + 16 * u, a.n - 1) - n0) * (uint32_t)a.ldxc);
+  const bool plain = a.ldb <= (1 << 23);  // 16 columns below 4 GB
   auto fetch = [&](int k0, T (&pa)[NA], T (&px)[NB]) {
+    if (plain && k0 + BK <= kend) {
+      const char* Bk = reinterpret_cast<const char*>(B + m0 + (int64_t)k0 * a.ldb);
+      const char* Xk = reinterpret_cast<const char*>(Xc + k0 + (int64_t)n0 * a.ldxc);
+#pragma unroll
+      for (int u = 0; u < NA; ++u) pa[u] = *reinterpret_cast<const T*>(Bk + oa[u]);
+#pragma unroll
+      for (int u = 0; u < NB; ++u) px[u] = *reinterpret_cast<const T*>(Xk + ox[u]);
+      return;
+    }
 #pragma unroll
     for (int u = 0; u < NA; ++u) {
       const int gi = m0 + (tid & (BM - 1)), gk = k0 + (tid / BM) + (256 / BM) * u;
