@@ -880,9 +880,9 @@ __device__ void chol_panel(const CholTileArgs& a, T (*lds)[TB][33]) {
       }
       stamp(K, 6);
     } else {
-      // Complex data, seven tiles: publish the block, form and publish the
-      // look-ahead's R tiles (tA, tB, tC, tF), then load the next block into
-      // the X tiles and update it; the roles rotate.
+      // Complex data, seven tiles: publish the block, form the look-ahead's R
+      // tiles (tA, tB, tC, tF), load the next block into the X tiles, update it
+      // and publish R; the roles rotate.
       put_tile<T>(tA, G, a.ldg, a.n, c0, c0);
       put_tile<T>(tB, G, a.ldg, a.n, c0, c1);
       put_tile<T>(tC, G, a.ldg, a.n, c1, c1);
@@ -906,9 +906,10 @@ __device__ void chol_panel(const CholTileArgs& a, T (*lds)[TB][33]) {
       stamp(K, 6);
       if (r0 < nt) {
         {
-          int* const wp[4] = {&gs[c0 * nt + r0], &gs[c1 * nt + r0], &gs[c0 * nt + r0 + 1], &gs[c1 * nt + r0 + 1]};
-          const int wv[4] = {K, K, K, K};
-          if (!wait_all<4>(wp, wv, ctl)) return;
+          int* const wp[7] = {&gs[c0 * nt + r0], &gs[c1 * nt + r0], &gs[c0 * nt + r0 + 1], &gs[c1 * nt + r0 + 1],
+                              &gs[r0 * nt + r0], &gs[r0 * nt + r0 + 1], &gs[(r0 + 1) * nt + r0 + 1]};
+          const int wv[7] = {K, K, K, K, K, K, K};
+          if (!wait_all<7>(wp, wv, ctl)) return;
         }
         load_n<4, T>(tA, TileSrc{G, a.ldg, c0, r0}, tB, TileSrc{G, a.ldg, c1, r0}, tC,
                      TileSrc{G, a.ldg, c0, r0 + 1}, tF, TileSrc{G, a.ldg, c1, r0 + 1}, tF, TileSrc{}, a.n);
@@ -917,6 +918,10 @@ __device__ void chol_panel(const CholTileArgs& a, T (*lds)[TB][33]) {
         mm32<T>(tA, tX, true, tA, false, 1.0, false);            // R_c0,r0 = X00^H G_c0,r0
         mm32_2<T>(tF, tE, tC, tD, tF, true, false, 1.0, false);  // R_c1,r0+1
         mm32<T>(tC, tX, true, tC, false, 1.0, false);            // R_c0,r0+1
+        // the next block (K updates) into the X tiles before the R tiles' stores,
+        // which drain behind its update (loads would wait for them)
+        load_n<3, T>(tX, TileSrc{G, a.ldg, r0, r0}, tE, TileSrc{G, a.ldg, r0, r0 + 1}, tD,
+                     TileSrc{G, a.ldg, r0 + 1, r0 + 1}, tD, TileSrc{}, tD, TileSrc{}, a.n);
         put_tile<T>(tA, G, a.ldg, a.n, c0, r0);
         put_tile<T>(tB, G, a.ldg, a.n, c1, r0);
         put_tile<T>(tC, G, a.ldg, a.n, c0, r0 + 1);
@@ -925,21 +930,13 @@ __device__ void chol_panel(const CholTileArgs& a, T (*lds)[TB][33]) {
         clear_tile<T>(G, a.ldg, a.n, r0, c1);
         clear_tile<T>(G, a.ldg, a.n, r0 + 1, c0);
         clear_tile<T>(G, a.ldg, a.n, r0 + 1, c1);
-        int* rp[4] = {&gs[c0 * nt + r0], &gs[c1 * nt + r0], &gs[c0 * nt + r0 + 1], &gs[c1 * nt + r0 + 1]};
-        const int rv[4] = {K + 1, K + 1, K + 1, K + 1};
-        publish_n(4, rp, rv);
-        // the next block (K updates) into the X tiles, then pair K's update
-        {
-          int* const wp[3] = {&gs[r0 * nt + r0], &gs[r0 * nt + r0 + 1], &gs[(r0 + 1) * nt + r0 + 1]};
-          const int wv[3] = {K, K, K};
-          if (!wait_all<3>(wp, wv, ctl)) return;
-        }
-        load_n<3, T>(tX, TileSrc{G, a.ldg, r0, r0}, tE, TileSrc{G, a.ldg, r0, r0 + 1}, tD,
-                     TileSrc{G, a.ldg, r0 + 1, r0 + 1}, tD, TileSrc{}, tD, TileSrc{}, a.n);
         __syncthreads();
         mm32_2<T>(tX, tA, tA, tB, tB, true, false, -1.0, true);  // G_r0,r0 -= R_.,r0^H R_.,r0
         mm32_2<T>(tE, tA, tC, tB, tF, true, false, -1.0, true);  // G_r0,r0+1 -= R_.,r0^H R_.,r0+1
         mm32_2<T>(tD, tC, tC, tF, tF, true, false, -1.0, true);  // G_r0+1,r0+1 -= R_.,r0+1^H R_.,r0+1
+        int* rp[4] = {&gs[c0 * nt + r0], &gs[c1 * nt + r0], &gs[c0 * nt + r0 + 1], &gs[c1 * nt + r0 + 1]};
+        const int rv[4] = {K + 1, K + 1, K + 1, K + 1};
+        publish_n(4, rp, rv);
         T(*oA)[33] = tA;
         T(*oB)[33] = tB;
         T(*oC)[33] = tC;
