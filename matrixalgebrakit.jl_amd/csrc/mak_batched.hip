@@ -10,10 +10,10 @@
 // (32-column panels, compact WY, backward orgqr, positive gauge), the panel
 // steps of all problems together and every task of a whole block gated on its
 // rejection.  Measured, m log-uniform in [16, 1024], n uniform in [8, m]: 4096
-// Float64 blocks 33.6 ms on panels alone, 18.6 ms; 1024 ComplexF64 blocks 24.6
-// and 14.5 ms.  The gated launches cost 0.7 ms of that when nothing is
-// rejected; a set whose blocks are all rejected pays the attempt, up to
-// 0.3 times the panel schedule.
+// Float64 blocks 33.6 ms on panels alone, 18.5 ms; 1024 ComplexF64 blocks 24.6
+// and 14.0 ms.  The gated launches cost 0.5 ms of that when nothing is
+// rejected; a set whose blocks are nearly all rejected pays the attempt (1024
+// Float64 blocks beyond condition 1e7: 12.2 -> 14.2 ms).
 //
 // The panel schedule:
 //   for panel step s: one node launch per row-size class factors panel s of
@@ -685,7 +685,7 @@ size_t count_apply(const std::vector<BProb>& P, const std::vector<int>& idx, int
 
 // Blocks that CholeskyQR2 of the whole block takes first (positive = true,
 // whose unique R it delivers).  Below 64 rows a 64 x 64 tile is mostly padding
-// and the panel schedule has at most two steps.
+// and the panel schedule has at most two steps (1353 such blocks of 4096: 0.4 ms).
 // (Offsets within 64 columns are 32 bits in the kernels.)
 bool whole_block(const BProb& p) {
   return p.m >= kCqMinRows && p.m >= p.n && std::max({p.lda, p.ldq, p.ldr}) <= (1 << 20);
