@@ -73,7 +73,7 @@ def qr_flops(m, n, full=False, complex_=False):
 
 
 def qr_pullback_flops(m, n):
-    """Q re-formed from WY (orgqr) + Q^H X, Q M, X R^-H (3 x 2 m n^2) + R11 products / inverse."""
+    """Algorithmic count with Q formed from WY (orgqr) + Q^H X, Q M, X R^-H (3 x 2 m n^2) + R11 products / inverse."""
     return orgqr_flops(m, n, n) + 6.0 * m * n * n + 2.0 * n ** 3
 
 
