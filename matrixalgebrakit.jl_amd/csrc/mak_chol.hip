@@ -1114,12 +1114,9 @@ __global__ void __launch_bounds__(256) chol_tile_kernel(CholTileArgs a) {
   }
 }
 
-template <typename T> __global__ void chol_zero_ints_kernel(int* p, int n) {
-  for (int e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256) p[e] = 0;
-}
-
-// Y[:, c0 : n] = 0 (m rows)
-__global__ void zero_cols_kernel(double* Y, int64_t ldy, int m, int c0, int n) {
+// The version counters and Y[:, c0 : n] (m rows) to 0, before the tile kernel.
+__global__ void chol_clear_kernel(int* p, int np, double* Y, int64_t ldy, int m, int c0, int n) {
+  for (int e = blockIdx.x * 256 + threadIdx.x; e < np; e += gridDim.x * 256) p[e] = 0;
   const int64_t tot = (int64_t)m * (n - c0);
   for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < tot; e += (int64_t)gridDim.x * 256)
     Y[e % m + (c0 + e / m) * ldy] = 0.0;
@@ -1179,13 +1176,14 @@ int chol_tile_factor(T* G, int64_t ldg, int n, T* X, int64_t ldx, int* flags, in
   a.info_offset = info_offset;
   a.trace = trace;
   const int nflags = 2 * a.nt * a.nt + 64;
-  hipLaunchKernelGGL((chol_zero_ints_kernel<T>), dim3(cdiv(nflags, 256)), dim3(256), 0, s, flags, nflags);
-  if (a.ny > 0 && a.ysplit < a.nt / 2) {
-    const int c0 = 64 * a.ysplit;  // < n (every pair has a column)
+  {
+    const bool halves = a.ny > 0 && a.ysplit < a.nt / 2;
+    const int c0 = halves ? 64 * a.ysplit : n;  // < n if halves (every pair has a column)
     // complex columns as real ones of twice the length
     constexpr int w = sizeof(T) / sizeof(double);
-    hipLaunchKernelGGL(zero_cols_kernel, dim3(1024), dim3(256), 0, s, static_cast<double*>(a.Y), w * a.ldy, w * a.m,
-                       c0, n);
+    const int64_t work = std::max<int64_t>(nflags, halves ? (int64_t)w * a.m * (n - c0) : 0);
+    hipLaunchKernelGGL(chol_clear_kernel, dim3((unsigned)std::min<int64_t>(cdiv64(work, 256), 1024)), dim3(256), 0, s,
+                       flags, nflags, static_cast<double*>(a.Y), w * a.ldy, halves ? w * a.m : 1, c0, n);
   }
   // the panel workgroup plus at least one for the other tasks; up to n ~ 1024
   // the chain dominates and fewer polling workgroups contend less for the

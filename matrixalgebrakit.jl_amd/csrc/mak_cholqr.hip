@@ -813,6 +813,15 @@ __global__ void zero_ints_kernel(int* p, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;
 }
+__global__ void zero_ints2_kernel(int* p, int n, int* q, int m) {
+  const int e = threadIdx.x;
+  if (e < n) p[e] = 0;
+  if (e < m) q[e] = 0;
+}
+void zero_ints2(int* p, int n, int* q, int m, hipStream_t s) {
+  if (n > 0 || m > 0) hipLaunchKernelGGL(zero_ints2_kernel, dim3(1), dim3(64), 0, s, p, n, q, m);
+}
+
 void zero_ints(int* p, int n, hipStream_t s) {
   if (n > 0) hipLaunchKernelGGL(zero_ints_kernel, dim3(cdiv(n, 64)), dim3(64), 0, s, p, n);
 }

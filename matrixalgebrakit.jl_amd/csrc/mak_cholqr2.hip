@@ -336,7 +336,8 @@ bool cholqr2_eligible(int m, int n) { return m >= n && n >= 1 && n <= kCholTileM
 
 // Enqueues the whole-matrix CholeskyQR2 on s; Q (m x n) and R (n x n or null)
 // receive the factors when the device-side check accepts (status word at
-// cholqr2_status(ws): [0] = 1 accepted).  ws: cholqr2_workspace_bytes(m, n).
+// cholqr2_status(ws): [0] = 1 accepted; its eight words are 0 on entry).  ws:
+// cholqr2_workspace_bytes(m, n).
 template <typename T>
 void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q, int64_t ldq, T* R, int64_t ldr,
                      char* ws) {
@@ -354,7 +355,6 @@ void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q,
   int* st = reinterpret_cast<int*>(ws + L.offSt);
   const int64_t nn = (int64_t)n * n;
   const unsigned eg = (unsigned)cdiv64(nn, 256);
-  zero_ints(st, 8, s);  // st[2]: the Cholesky's info
   // pass 1: Q1 = A X1 inside the Cholesky launch, column block by column
   // block as X1 becomes final
   gram_upper<T>(A, lda, m, n, G, X, L.kcap, s);

@@ -56,6 +56,7 @@ template <typename T> void cholqr_carry_buffers(T* cw, T** Gw, T** partN, T** R1
 // Workgroups (and Gram partials) of the panel kernels for an H-row panel.
 int cholqr_gram_blocks(int H);
 void zero_ints(int* p, int n, hipStream_t s);
+void zero_ints2(int* p, int n, int* q, int m, hipStream_t s);  // n, m <= 64, one launch
 
 // Whole-matrix CholeskyQR2 for qr_compact!(positive = true) (mak_cholqr2.hip):
 // eligible for m >= n, n <= kCholTileMaxN.  cholqr2_enqueue reads A only and
