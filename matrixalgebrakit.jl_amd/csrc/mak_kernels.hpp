@@ -206,7 +206,17 @@ struct GemmArgs {
   // null, C = alpha op(A) op(B) + beta Cin (Cin m x n, ld ldcin; it may be C).
   const void* Cin;
   int64_t ldcin;
+  // gemm_dual only: a second pair of operands with the same K.
+  const void* A2;
+  int64_t lda2, strideA2;
+  const void* B2;
+  int64_t ldb2, strideB2;
 };
+
+// C = alpha (A B + A2 B2) + beta C, no transposes; one launch for real data with
+// K a multiple of 16, equal leading dimensions of A, A2 and of B, B2, and enough
+// tiles, else two products.
+template <typename T> void gemm_dual(GemmArgs g, hipStream_t s);
 
 // C = alpha op(A) op(B) + beta C on FP64 MFMA (real) or 4 real MFMAs (complex).
 template <typename T> void gemm(int opA, int opB, GemmArgs g, hipStream_t s);

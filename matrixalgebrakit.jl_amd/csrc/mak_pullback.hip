@@ -628,8 +628,14 @@ int polar_pullback_doubling(hipStream_t s, int batch, int m, int n, const T* W, 
   if (dP)
     hipLaunchKernelGGL((baxpy_kernel<T>), gnn, dim3(256), 0, s, n, n, 1.0, dPh, (int64_t)n, nn, X, (int64_t)n, nn);
   prod(OP_N, OP_N, K, Pinv, X, -1.0, 1.0);
-  gemm<T>(OP_N, OP_N, bga<T>(batch, m, n, n, W, ldw, sw, X, n, nn, dA, ldda, sda, 1.0, 1.0), s);
-  gemm<T>(OP_N, OP_N, bga<T>(batch, m, n, n, dW, lddw, sdw, Pinv, n, nn, dA, ldda, sda, 1.0, 1.0), s);
+  GemmArgs g = bga<T>(batch, m, n, n, W, ldw, sw, X, n, nn, dA, ldda, sda, 1.0, 1.0);
+  g.A2 = dW;
+  g.lda2 = lddw;
+  g.strideA2 = sdw;
+  g.B2 = Pinv;
+  g.ldb2 = n;
+  g.strideB2 = nn;
+  gemm_dual<T>(g, s);
   return 0;
 }
 
