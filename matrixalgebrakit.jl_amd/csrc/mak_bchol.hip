@@ -469,7 +469,9 @@ __global__ void bchol_init_kernel(int* state, int n, int* any, int* status, int 
 }
 
 // States of a block: 0 factored in one pass, 2 in two, 1 rejected.
-__device__ __forceinline__ bool bc_skip(const BCholProb& p, int pass) { return *p.state != (pass == 2 ? 2 : 0); }
+__device__ __forceinline__ bool bc_skip(int state, int pass) { return state != (pass == 2 ? 2 : 0); }
+// In launches that do not write the state (all but the factor and the decision).
+__device__ __forceinline__ bool bc_skip(const BCholProb& p, int pass) { return bc_skip(*p.state, pass); }
 
 // State after E of this pass; any |= rejected.  One wave per block sums the
 // squared norms of E's upper tiles, in a fixed order.  (nt^2 times their
@@ -481,7 +483,7 @@ __global__ void bchol_decide_kernel(const BCholProb* P, int n, int* any, int pas
   if (e >= n) return;
   const BCholProb p = P[e];
   const int nt = p.np / BT, st = *p.state;
-  if (!bc_skip(p, pass)) {
+  if (!bc_skip(st, pass)) {
     double s = 0.0;
     for (int t = lane; t < nt * nt; t += 64)
       if (t % nt <= t / nt) s += (t % nt < t / nt ? 2.0 : 1.0) * p.dev[t];
@@ -608,11 +610,16 @@ template <typename T>
 __global__ void __launch_bounds__(256) bchol_factor_kernel(const BCholProb* P, const BCholTask* tasks, int pass) {
   using C = BcCfg<T>;
   __shared__ T pool[C::POOL > 5 * 32 * 33 ? C::POOL : 5 * 32 * 33];
-  __shared__ int bad_s;
+  __shared__ int bad_s, state_s;
   const BCholTask t = tasks[blockIdx.x];
   if (t.prob < 0) return;
   const BCholProb p = P[t.prob];
-  if (bc_skip(p, pass)) return;
+  // The task of the block's next diagonal tile may reject the block while this
+  // one starts: one thread reads the state for all (what the task writes is of
+  // no use then, whichever value it sees).
+  if (threadIdx.x == 0) state_s = __hip_atomic_load(p.state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (bc_skip(state_s, pass)) return;
   const int k = t.a, b = t.b;
   const int64_t ld = p.np;
   T* W = reinterpret_cast<T*>(pass == 2 ? p.U : p.W);
@@ -674,7 +681,7 @@ __global__ void __launch_bounds__(256) bchol_factor_kernel(const BCholProb* P, c
               s_sub(Wbb[ri + 16 * i + (int64_t)(cj + 16 * j + 4 * u) * ld], acc.get(i, j, u));
   }
   const bool bad = bc_chol64<T>(S11, &bad_s, Wbb, ld, Xd + (int64_t)b * BT * BT);
-  if (threadIdx.x == 0 && bad) *p.state = 1;
+  if (threadIdx.x == 0 && bad) __hip_atomic_store(p.state, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Strip a (64 rows) of Q1 = A R1^{-1}; second: of Q1 <- Q1 R2^{-1}, in place.

@@ -116,3 +116,31 @@ def test_whole_blocks_conditioning(dt, with_r, dev):
         else:
             assert all(np.array_equal(a, b) for a, b in zip(first, Qh))
     plan.close()
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.complex128], ids=["f64", "c64"])
+def test_whole_blocks_rejected_in_the_middle_of_a_factor_step(dt, dev):
+    """Blocks that lose positive definiteness at each of their diagonal tiles,
+    while other tasks of the same block and other blocks are at work in the same
+    launch: they come out as a QR of the block, and their neighbours as without
+    them."""
+    good = [O.gaussian(500, 450, dt, seed=60 + i) for i in range(4)]
+    bad = []
+    for t in range(1, 7):
+        B = O.gaussian(460, 440, dt, seed=70 + t)
+        B[:, 64 * t + 3] = B[:, 64 * t - 5]
+        bad.append(B)
+    outs = []
+    for host in (good + 4 * bad, good):
+        As = [mak.colmajor(torch.from_numpy(np.asfortranarray(h)).to(dev)) for h in host]
+        plan = mak.BatchedQRPlan(As)
+        Qs, Rs = plan.execute()
+        torch.cuda.synchronize()
+        outs.append([(q.cpu().numpy(), r.cpu().numpy()) for q, r in zip(Qs, Rs)])
+        plan.close()
+    for (q0, r0), (q1, r1), h in zip(outs[0], outs[1], good):
+        assert np.array_equal(q0, q1) and np.array_equal(r0, r1)
+        check(h, q0, r0, True)
+    for h, (q, r) in zip(4 * bad, outs[0][4:]):
+        assert np.linalg.norm(h - q @ r) <= 1e-14 * np.sqrt(h.shape[1]) * np.linalg.norm(h)
+        assert np.linalg.norm(q.conj().T @ q - np.eye(q.shape[1])) <= 1e-14 * np.sqrt(q.shape[1])
