@@ -241,32 +241,106 @@ template <int K> __device__ __forceinline__ zd row_bcast(const zd& v) {
   return mkz(row_bcast<K>(v.x), row_bcast<K>(v.y));
 }
 
-// s -= conj(b_R) ws, x -= conj(b_R) wx with b_R = b of lane R of the row.  A
-// VGPR may be a DPP source from two instructions after its write.  b is the
-// step's pivot row, last written by the previous step's first update, and ws
-// depends on the reciprocal of its pivot, so no wait is needed here (one
-// s_nop per row costs a sixth of the whole factorisation); elim16_step fixes
-// b in its registers behind a wait of its own.
+// Rows R .. R + N - 1 of s and x: s -= conj(b_R) ws, x -= conj(b_R) wx with
+// b_R = b of lane R of the 16-lane row.  A VGPR may be a DPP source from two
+// instructions after its write, and what the register allocator puts between
+// two asm blocks (a copy of b, a reload) is not known to them, so each block
+// begins with the wait itself, or with two other instructions.  A wait per row
+// costs a sixth of the whole factorisation, so a block holds all rows between
+// two links of the chain of reciprocals (qr_compact! 1024 x 512 Float64: 375 us
+// without any waits, 388 with a wait per four rows, 382 so; ComplexF64 within
+// 0.5 % of each other).
+#define MAK_E_OUT(i) [s##i] "+&v"(s[R + i]), [x##i] "+&v"(x[R + i])
+#define MAK_E_LANE(i) [r##i] "n"(R + i)
+#define MAK_E_ROW(i)                                                                                    \
+  "v_fmac_f64_dpp %[s" #i "], -%[b], %[ws] row_newbcast:%c[r" #i "] row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fmac_f64_dpp %[x" #i "], -%[b], %[wx] row_newbcast:%c[r" #i "] row_mask:0xf bank_mask:0xf\n\t"
+#define MAK_E_IN [b] "v"(b), [ws] "v"(ws), [wx] "v"(wx)
+template <int R, int N> __device__ __forceinline__ void elim_block(double* s, double* x, double b, double ws, double wx) {
+  if constexpr (N == 1)
+    asm("s_nop 1\n\t" MAK_E_ROW(0)
+        : MAK_E_OUT(0)
+        : MAK_E_IN, MAK_E_LANE(0));
+  else if constexpr (N == 2)
+    asm("s_nop 1\n\t" MAK_E_ROW(0) MAK_E_ROW(1)
+        : MAK_E_OUT(0), MAK_E_OUT(1)
+        : MAK_E_IN, MAK_E_LANE(0), MAK_E_LANE(1));
+  else if constexpr (N == 3)
+    asm("s_nop 1\n\t" MAK_E_ROW(0) MAK_E_ROW(1) MAK_E_ROW(2)
+        : MAK_E_OUT(0), MAK_E_OUT(1), MAK_E_OUT(2)
+        : MAK_E_IN, MAK_E_LANE(0), MAK_E_LANE(1), MAK_E_LANE(2));
+  else if constexpr (N == 4)
+    asm("s_nop 1\n\t" MAK_E_ROW(0) MAK_E_ROW(1) MAK_E_ROW(2) MAK_E_ROW(3)
+        : MAK_E_OUT(0), MAK_E_OUT(1), MAK_E_OUT(2), MAK_E_OUT(3)
+        : MAK_E_IN, MAK_E_LANE(0), MAK_E_LANE(1), MAK_E_LANE(2), MAK_E_LANE(3));
+  else if constexpr (N == 5)
+    asm("s_nop 1\n\t" MAK_E_ROW(0) MAK_E_ROW(1) MAK_E_ROW(2) MAK_E_ROW(3) MAK_E_ROW(4)
+        : MAK_E_OUT(0), MAK_E_OUT(1), MAK_E_OUT(2), MAK_E_OUT(3), MAK_E_OUT(4)
+        : MAK_E_IN, MAK_E_LANE(0), MAK_E_LANE(1), MAK_E_LANE(2), MAK_E_LANE(3), MAK_E_LANE(4));
+  else if constexpr (N == 6)
+    asm("s_nop 1\n\t" MAK_E_ROW(0) MAK_E_ROW(1) MAK_E_ROW(2) MAK_E_ROW(3) MAK_E_ROW(4) MAK_E_ROW(5)
+        : MAK_E_OUT(0), MAK_E_OUT(1), MAK_E_OUT(2), MAK_E_OUT(3), MAK_E_OUT(4), MAK_E_OUT(5)
+        : MAK_E_IN, MAK_E_LANE(0), MAK_E_LANE(1), MAK_E_LANE(2), MAK_E_LANE(3), MAK_E_LANE(4), MAK_E_LANE(5));
+  else if constexpr (N == 7)
+    asm("s_nop 1\n\t" MAK_E_ROW(0) MAK_E_ROW(1) MAK_E_ROW(2) MAK_E_ROW(3) MAK_E_ROW(4) MAK_E_ROW(5) MAK_E_ROW(6)
+        : MAK_E_OUT(0), MAK_E_OUT(1), MAK_E_OUT(2), MAK_E_OUT(3), MAK_E_OUT(4), MAK_E_OUT(5), MAK_E_OUT(6)
+        : MAK_E_IN, MAK_E_LANE(0), MAK_E_LANE(1), MAK_E_LANE(2), MAK_E_LANE(3), MAK_E_LANE(4), MAK_E_LANE(5), MAK_E_LANE(6));
+}
+// The same for row R alone, forming ws = s[R - 1] inv and wx = x[R - 1] inv
+// first (b = s[R - 1]); s[R] may be a DPP source afterwards.
 template <int R>
-__device__ __forceinline__ void elim_row(double& s, double& x, double b, double ws, double wx) {
-  asm("v_fmac_f64_dpp %0, -%2, %3 row_newbcast:%c5 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %1, -%2, %4 row_newbcast:%c5 row_mask:0xf bank_mask:0xf"
-      : "+v"(s), "+v"(x)
-      : "v"(b), "v"(ws), "v"(wx), "n"(R));
+__device__ __forceinline__ void elim_first(double* s, double* x, double b, double inv, double& ws, double& wx) {
+  constexpr int K = R - 1;
+  asm("v_mul_f64 %[ws], %[b], %[inv]\n\tv_mul_f64 %[wx], %[xk], %[inv]\n\t" MAK_E_ROW(0) "s_nop 0"
+      : MAK_E_OUT(0), [ws] "=&v"(ws), [wx] "=&v"(wx)
+      : [b] "v"(b), [xk] "v"(x[K]), [inv] "v"(inv), MAK_E_LANE(0));
+}
+#undef MAK_E_OUT
+#undef MAK_E_ROW
+#undef MAK_E_IN
+#define MAK_E_OUT(i) \
+  [sx##i] "+&v"(s[R + i].x), [sy##i] "+&v"(s[R + i].y), [xx##i] "+&v"(x[R + i].x), [xy##i] "+&v"(x[R + i].y)
+#define MAK_E_FMAC(acc, i, part, w) \
+  "v_fmac_f64_dpp %[" acc #i "], " part ", %[" w "] row_newbcast:%c[r" #i "] row_mask:0xf bank_mask:0xf\n\t"
+#define MAK_E_ROW(i)                                                                                  \
+  MAK_E_FMAC("sx", i, "-%[bx]", "wsx") MAK_E_FMAC("sy", i, "-%[bx]", "wsy")                           \
+  MAK_E_FMAC("xx", i, "-%[bx]", "wxx") MAK_E_FMAC("xy", i, "-%[bx]", "wxy")                           \
+  MAK_E_FMAC("sx", i, "-%[by]", "wsy") MAK_E_FMAC("sy", i, "%[by]", "wsx")                            \
+  MAK_E_FMAC("xx", i, "-%[by]", "wxy") MAK_E_FMAC("xy", i, "%[by]", "wxx")
+#define MAK_E_IN \
+  [bx] "v"(b.x), [by] "v"(b.y), [wsx] "v"(ws.x), [wsy] "v"(ws.y), [wxx] "v"(wx.x), [wxy] "v"(wx.y)
+template <int R, int N>
+__device__ __forceinline__ void elim_block(zd* s, zd* x, const zd& b, const zd& ws, const zd& wx) {
+  if constexpr (N == 1)
+    asm("s_nop 1\n\t" MAK_E_ROW(0)
+        : MAK_E_OUT(0)
+        : MAK_E_IN, MAK_E_LANE(0));
+  else if constexpr (N == 2)
+    asm("s_nop 1\n\t" MAK_E_ROW(0) MAK_E_ROW(1)
+        : MAK_E_OUT(0), MAK_E_OUT(1)
+        : MAK_E_IN, MAK_E_LANE(0), MAK_E_LANE(1));
+  else if constexpr (N == 3)
+    asm("s_nop 1\n\t" MAK_E_ROW(0) MAK_E_ROW(1) MAK_E_ROW(2)
+        : MAK_E_OUT(0), MAK_E_OUT(1), MAK_E_OUT(2)
+        : MAK_E_IN, MAK_E_LANE(0), MAK_E_LANE(1), MAK_E_LANE(2));
+  else if constexpr (N == 4)
+    asm("s_nop 1\n\t" MAK_E_ROW(0) MAK_E_ROW(1) MAK_E_ROW(2) MAK_E_ROW(3)
+        : MAK_E_OUT(0), MAK_E_OUT(1), MAK_E_OUT(2), MAK_E_OUT(3)
+        : MAK_E_IN, MAK_E_LANE(0), MAK_E_LANE(1), MAK_E_LANE(2), MAK_E_LANE(3));
 }
 template <int R>
-__device__ __forceinline__ void elim_row(zd& s, zd& x, const zd& b, const zd& ws, const zd& wx) {
-  asm("v_fmac_f64_dpp %0, -%4, %6 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %1, -%4, %7 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %2, -%4, %8 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %3, -%4, %9 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %0, -%5, %7 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %1, %5, %6 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %2, -%5, %9 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %3, %5, %8 row_newbcast:%c10 row_mask:0xf bank_mask:0xf"
-      : "+v"(s.x), "+v"(s.y), "+v"(x.x), "+v"(x.y)
-      : "v"(b.x), "v"(b.y), "v"(ws.x), "v"(ws.y), "v"(wx.x), "v"(wx.y), "n"(R));
+__device__ __forceinline__ void elim_first(zd* s, zd* x, const zd& b, double inv, zd& ws, zd& wx) {
+  constexpr int K = R - 1;
+  asm("v_mul_f64 %[wsx], %[bx], %[inv]\n\tv_mul_f64 %[wsy], %[by], %[inv]\n\t"
+      "v_mul_f64 %[wxx], %[xkx], %[inv]\n\tv_mul_f64 %[wxy], %[xky], %[inv]\n\t" MAK_E_ROW(0)
+      : MAK_E_OUT(0), [wsx] "=&v"(ws.x), [wsy] "=&v"(ws.y), [wxx] "=&v"(wx.x), [wxy] "=&v"(wx.y)
+      : [bx] "v"(b.x), [by] "v"(b.y), [xkx] "v"(x[K].x), [xky] "v"(x[K].y), [inv] "v"(inv), MAK_E_LANE(0));
 }
+#undef MAK_E_OUT
+#undef MAK_E_LANE
+#undef MAK_E_ROW
+#undef MAK_E_FMAC
+#undef MAK_E_IN
 // Step K: with the pivot d = s[K] of lane K and the pivot row b = s[K],
 //   s[r] -= conj(b_r) s[K] / d,  x[r] -= conj(b_r) x[K] / d   (r > K).
 // 1 / d is v_rcp_f64's y with its third-order correction, y (1 + e + e^2) with
@@ -274,6 +348,8 @@ __device__ __forceinline__ void elim_row(zd& s, zd& x, const zd& b, const zd& ws
 // Row K + 1, which holds the next pivot, is updated first, and the next
 // pivot's reciprocal is formed between the other rows' updates (order_after
 // keeps it there), so that the serial chain runs under them.
+// dpp_source: the wait before a value that an asm block wrote becomes the DPP
+// source of a compiler's instruction (the compiler sees no write in asm).
 __device__ __forceinline__ void dpp_source(double& b) { asm("s_nop 1" : "+v"(b)); }
 __device__ __forceinline__ void dpp_source(zd& b) { asm("s_nop 1" : "+v"(b.x), "+v"(b.y)); }
 struct ElimPivot {
@@ -282,21 +358,20 @@ struct ElimPivot {
 template <typename T, int K, int R0, int R1>
 __device__ __forceinline__ void elim16_rows(T (&s)[16], T (&x)[16], const T& b, const T& ws, const T& wx) {
   if constexpr (R0 < R1) {
-    elim_row<R0>(s[R0], x[R0], b, ws, wx);
-    elim16_rows<T, K, R0 + 1, R1>(s, x, b, ws, wx);
+    constexpr int most = ScalarTraits<T>::is_complex ? 4 : 7, N = R1 - R0 < most ? R1 - R0 : most;
+    elim_block<R0, N>(s, x, b, ws, wx);
+    elim16_rows<T, K, R0 + N, R1>(s, x, b, ws, wx);
   }
 }
 template <typename T, int K>
 __device__ __forceinline__ void elim16_step(T (&s)[16], T (&x)[16], int c0, double& piv, ElimPivot& p) {
-  T b = s[K];
-  dpp_source(b);
-  T ws = s_scale(b, p.inv);
-  const T wx = s_scale(x[K], p.inv);
+  const T b = s[K];
   piv = sel(step_lane(c0) == K, p.d, piv);
   if constexpr (K < 15) {
     constexpr int n = 14 - K, R0 = K + 2, R1 = R0 + (n + 1) / 2, R2 = R1 + (16 - R1 + 2) / 3,
                   R3 = R2 + (16 - R2 + 1) / 2;
-    elim_row<K + 1>(s[K + 1], x[K + 1], b, ws, wx);
+    T ws, wx;
+    elim_first<K + 1>(s, x, b, p.inv, ws, wx);
     p.d = row_bcast<K + 1>(s_re(s[K + 1]));
     p.y = __builtin_amdgcn_rcp(p.d);
     order_after(ws, p.y);

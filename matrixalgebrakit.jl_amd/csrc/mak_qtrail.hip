@@ -83,6 +83,7 @@ __device__ __forceinline__ void gj16_rows(T (&s)[16], T (&x)[16], const T& ws, c
 }
 template <typename T, int K>
 __device__ __forceinline__ void gj16_step(T (&s)[16], T (&x)[16], int c0, int valid, T& sg) {
+  dpp_source(s[K]);
   const T p = row_bcast<K>(s[K]);
   const T sk = K < valid ? minus_sign(p) : s_zero(T());
   const T inv = s_recip(s_sub(p, sk));
