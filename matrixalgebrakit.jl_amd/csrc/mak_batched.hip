@@ -425,6 +425,8 @@ struct BatchedQrPlan {
   std::vector<Step> steps;
   std::vector<int> qOff, qCnt, qFree;  // orgqr per step (trans = 0)
   std::vector<int> cqIdx;          // status words of the CholeskyQR2 panel tasks (test hook)
+  std::vector<int> cqWhole;        // per panel task: its block's place among the whole blocks, or -1 (test hook)
+  int nwhole = 0;
   int nc = 64, gridMult = 2, cus = 256;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -1167,7 +1169,12 @@ int plan_create(BatchedQrPlan* pl, int count, const int* m, const int* n, void* 
                  apply, steps, qOff, qCnt, qFree);
   if (!upload_tasks(dcq, cq, dnode, node, drf, rf, dex, ex, dapply, apply)) return 1;
   pl->cqIdx.clear();
-  for (const CholQrTask& t : cq) pl->cqIdx.push_back((int)(t.status - stBase));
+  pl->cqWhole.clear();
+  pl->nwhole = (int)whole.size();
+  for (const CholQrTask& t : cq) {
+    pl->cqIdx.push_back((int)(t.status - stBase));
+    pl->cqWhole.push_back(t.gate != nullptr ? (int)(t.gate - wstate) : -1);
+  }
   pl->steps = steps;
   pl->qOff = qOff;
   pl->qCnt = qCnt;
@@ -1287,6 +1294,29 @@ int maktest_batched_panel_status(const mak_qr_batched_plan* plan, int* accepted,
   for (int i : p.cqIdx) {
     if (st[i] == 0) ++*accepted;
     else if (st[i] == 1) ++*rejected;
+  }
+  return 0;
+}
+
+// Test hook, as above: panels[3] = the panels whose CholeskyQR2 task accepted,
+// rejected, and did not run (their block was factored whole); whole[3] = the
+// blocks factored whole in one pass, in two, and rejected.
+int maktest_batched_routes(const mak_qr_batched_plan* plan, int* panels, int* whole) {
+  if (plan == nullptr || panels == nullptr || whole == nullptr) return -1;
+  const mak::BatchedQrPlan& p = plan->p;
+  for (int i = 0; i < 3; ++i) panels[i] = whole[i] = 0;
+  std::vector<int> state(p.nwhole), st;
+  if (p.nwhole > 0) {
+    const char* at = p.ws + p.offWholeProbs + mak::al256(sizeof(mak::BCholProb) * p.nwhole);
+    if (hipMemcpy(state.data(), at, sizeof(int) * p.nwhole, hipMemcpyDeviceToHost) != hipSuccess) return 1;
+  }
+  for (int v : state) ++whole[v == 0 ? 0 : v == 2 ? 1 : 2];
+  if (p.cqIdx.empty()) return 0;
+  st.resize((size_t)*std::max_element(p.cqIdx.begin(), p.cqIdx.end()) + 1);
+  if (hipMemcpy(st.data(), p.ws + p.offSt, sizeof(int) * st.size(), hipMemcpyDeviceToHost) != hipSuccess) return 1;
+  for (size_t t = 0; t < p.cqIdx.size(); ++t) {
+    const bool ran = p.cqWhole[t] < 0 || state[p.cqWhole[t]] == 1;
+    ++panels[!ran ? 2 : st[p.cqIdx[t]] == 0 ? 0 : 1];
   }
   return 0;
 }

@@ -961,7 +961,7 @@ __global__ void __launch_bounds__(256) qr_small_kernel(const T* A, int64_t lda, 
     As[r][c] = r < m && c < n ? A[r + (int64_t)c * lda] : s_zero(T());
   }
   if (tid == 0) bad_s = 0;
-  if (status != nullptr && tid < 8) status[tid] = 0;
+  if (status != nullptr && tid < 8) status[tid] = 0;  // [0]: 1 below if accepted
   __syncthreads();
   // pass 0: G = A^H A to S11, S12, S22; pass 1: U from E = Q1^H Q1 - I to Y11, W12, S12
   const bool quad = wm <= wn && (two || wn == 0);
@@ -1061,6 +1061,7 @@ __global__ void __launch_bounds__(256) qr_small_kernel(const T* A, int64_t lda, 
     small_householder<T>(As, reinterpret_cast<T (*)[SP]>(&tiles[0][0][0]), tau_s, A, lda, Q, ldq, R, ldr, m, n);
     return;
   }
+  if (status != nullptr && tid == 0) status[0] = 1;
   // Q = Q1 - Q1 U
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -1123,6 +1124,7 @@ struct TallArgs {
   int64_t ldr;
   void *part, *W, *X, *D;  // gridDim.x blocks of 64 x 64; 64 x 64 each
   int* ctl;                // state (1 until accepted), a ticket per launch; set by the caller to 1, 0, 0
+  int* status;             // optional: [0] = 1 when accepted
   int m, n, rps;
 };
 
@@ -1307,7 +1309,10 @@ __global__ void __launch_bounds__(256) qr_tall_kernel(const TallArgs p) {
         put_r(T1, T2, 32, 32);
       }
     }
-    if (tid == 0) p.ctl[0] = 0;
+    if (tid == 0) {
+      p.ctl[0] = 0;
+      if (p.status != nullptr) p.status[0] = 1;
+    }
   }
 }
 
@@ -1388,7 +1393,7 @@ void qr_tall_enqueue(const T* A, int64_t lda, T* Q, int64_t ldq, T* R, int64_t l
   const int rps = cdiv(cdiv(m, kTallMaxWgs), BT) * BT, wgs = cdiv(m, rps);
   T* W = scratch + kTallCtlElems;
   const TallArgs a{A, lda, Q, ldq, R, ldr, W + 3 * BT * BT, W, W + BT * BT, W + 2 * BT * BT,
-                   reinterpret_cast<int*>(scratch), m, n, rps};
+                   reinterpret_cast<int*>(scratch), status, m, n, rps};
   hipLaunchKernelGGL(qr_tall_init_kernel, dim3(1), dim3(64), 0, s, a.ctl, status, flags);
   hipLaunchKernelGGL((qr_tall_kernel<T, 0>), dim3(wgs), dim3(256), 0, s, a);
   hipLaunchKernelGGL((qr_tall_kernel<T, 1>), dim3(wgs), dim3(256), 0, s, a);

@@ -85,14 +85,15 @@ template <typename T>
 void launch_bchol(BCholPhase phase, const BCholProb* P, const BCholTask* tasks, int n, int pass, hipStream_t s);
 // qr_compact! with positive = true of one matrix, m >= 64 > n: the first int of
 // scratch is 0 afterwards if Q and R were written, else A is for the panels;
-// status, flags: eight and three words cleared, or null
+// status, flags: eight and three words cleared, or null; status[0] = 1 if
+// CholeskyQR2 was accepted
 constexpr int kTallMaxWgs = 64, kTallCtlElems = 32;
 constexpr int64_t kTallScratchElems = kTallCtlElems + (int64_t)(kTallMaxWgs + 3) * kBCholTile * kBCholTile;
 template <typename T>
 void qr_tall_enqueue(const T* A, int64_t lda, T* Q, int64_t ldq, T* R, int64_t ldr, T* scratch, int* status,
                      int* flags, int m, int n, hipStream_t s);
 // qr_compact! with positive = true of one matrix, n <= m < 64; scratch: 64 x 64;
-// status: eight words cleared, or null
+// status: eight words cleared, [0] = 1 if CholeskyQR2 was accepted, or null
 template <typename T>
 void launch_qr_small(const T* A, int64_t lda, T* Q, int64_t ldq, T* R, int64_t ldr, T* scratch, int* status, int m,
                      int n, hipStream_t s);

@@ -570,7 +570,7 @@ template <typename T> void qr_record(const char* ws, int m, int n, int full, int
   if (L.offFlags) hipMemcpy(h, ws + L.offFlags, sizeof(h), hipMemcpyDeviceToHost);
   if (L.offCq2) hipMemcpy(st, cholqr2_status<T>(const_cast<char*>(ws) + L.offCq2, m, n), sizeof(st),
                           hipMemcpyDeviceToHost);
-  out[0] = st[0];                  // 1: the whole-matrix CholeskyQR2 result was taken
+  out[0] = st[0];                  // 1: the CholeskyQR2 result of the whole matrix was taken (any size)
   out[1] = h[0] ? h[2] : -1;       // first panel handed to Householder TSQR (-1: none)
   out[2] = st[2];                  // Cholesky info of the whole-matrix path
   out[3] = L.offCq2 != 0;          // the whole-matrix path exists for this shape

@@ -57,7 +57,7 @@ int maktest_gemm_prec(void* stream, int prec, int opA, int opB, int M, int N, in
 }
 
 // Status words a qr call left in its workspace `work` (synchronous read):
-// out[0] 1 when the whole-matrix CholeskyQR2 result was taken, out[1] the
+// out[0] 1 when the CholeskyQR2 result of the whole matrix was taken, out[1] the
 // first 32-column panel handed to Householder TSQR (-1: none), out[2] the
 // whole-matrix path's Cholesky info, out[3] 1 when that path exists for the
 // shape, out[4..5] its ||Q1^H Q1 - I||_F (a double), out[6 / 7 / 8] 1 when
