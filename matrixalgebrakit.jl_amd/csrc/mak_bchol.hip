@@ -48,7 +48,6 @@ namespace {
 constexpr int BT = kBCholTile;  // 64
 constexpr double kBCholMaxE = 1e-8, kBCholMaxE2 = 0.1;
 constexpr double kTallMaxE = 1e-6;
-constexpr double kBCholLoMaxE = 1e-10;
 
 // LDS of one stage of a tile product: KB inner indices of the two operands.
 // The pitches keep the fragment reads (16 rows x 4 k of a wave) off each
@@ -65,7 +64,7 @@ template <> struct BcCfg<zd> {
   static constexpr int KB = 8, PK = 9, PR = 65;
   static constexpr int L = 64 * PK, R = 64 * PK, STAGE = L + R;
   static constexpr int OCC_GRAM = 2, OCC = 2;
-  static constexpr int POOL = 2 * STAGE + 64;  // the FP32 stages need 64 elements more
+  static constexpr int POOL = 2 * STAGE;
 };
 constexpr int KX = 16;  // inner indices of one stage of the product with a 64 x 64 inverse
 template <typename T> struct BcX;
@@ -234,136 +233,6 @@ __device__ __forceinline__ void bc_product(BcAcc<T>& acc, T* pool, const T* L, i
   __syncthreads();
 }
 
-// ---------------------------------------------------------------------------
-// L R on FP32 MFMA (operands rounded, FP32 accumulation): the correction Q1 U
-// where ||U||_F < ||E||_F <= kBCholLoMaxE.  Its error, at most about
-// n u_32 ||U||_F <= 6e-15 in the worst case of the accumulation and typically
-// sqrt(n) u_32 ||U||_F ~ 2e-16, is that of the single-matrix path's correction.
-// The whole correction launch: 5.4 -> 5.0 ms (4096 Float64 blocks), 3.5 -> 2.9 ms
-// (1024 ComplexF64); strips of 128 rows at half the stage depth took 5.4 and 3.7.
-// ---------------------------------------------------------------------------
-struct zf {
-  float x, y;
-};
-template <typename T> struct BcLo;
-template <> struct BcLo<double> {
-  using F = float;
-  static constexpr int KB = 32, PK = 33, PR = 80;
-  v4f r[2][2];
-  __device__ __forceinline__ static float to(double v) { return (float)v; }
-  __device__ __forceinline__ void zero() {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) r[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-  }
-  __device__ __forceinline__ double get(int i, int j, int u) const { return r[i][j][u]; }
-  __device__ __forceinline__ void step(const float (&a)[2], const float (&b)[2]) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) r[i][j] = mfma_f32(b[j], a[i], r[i][j]);
-  }
-};
-template <> struct BcLo<zd> {
-  using F = zf;
-  static constexpr int KB = 16, PK = 17, PR = 80;
-  v4f p[2][2], q[2][2], s[2][2];
-  __device__ __forceinline__ static zf to(zd v) { return zf{(float)v.x, (float)v.y}; }
-  __device__ __forceinline__ void zero() {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) p[i][j] = q[i][j] = s[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-  }
-  __device__ __forceinline__ zd get(int i, int j, int u) const {
-    return mkz((double)p[i][j][u] - (double)q[i][j][u],
-               (double)s[i][j][u] - (double)p[i][j][u] - (double)q[i][j][u]);
-  }
-  __device__ __forceinline__ void step(const zf (&a)[2], const zf (&b)[2]) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        p[i][j] = mfma_f32(b[j].x, a[i].x, p[i][j]);
-        q[i][j] = mfma_f32(b[j].y, a[i].y, q[i][j]);
-        s[i][j] = mfma_f32(b[j].x + b[j].y, a[i].x + a[i].y, s[i][j]);
-      }
-  }
-};
-static_assert(2 * (32 * 80 + 64 * 33) * sizeof(float) <= BcCfg<double>::POOL * sizeof(double), "FP32 stages");
-static_assert(2 * (16 * 80 + 64 * 17) * sizeof(zf) <= BcCfg<zd>::POOL * sizeof(zd), "FP32 stages");
-
-// As bc_product<T, false>; result column 16 j + 4 (lane / 16) + u of register u.
-template <typename T>
-__device__ __forceinline__ void bc_product_lo(BcLo<T>& acc, void* pool, const T* L, int64_t ldl, int nl, const T* R,
-                                              int64_t ldr, int nr, int K) {
-  using C = BcLo<T>;
-  using F = typename C::F;
-  constexpr int KB = C::KB, NQ = BT * KB / 256, SL = KB * C::PR, STAGE = SL + 64 * C::PK;
-  if (K <= 0) return;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int lr = lane & 15, lq = lane >> 4;
-  const int wm = w & 1, wn = w >> 1;
-  unsigned ol[NQ], orr[NQ];
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const int e = tid + 256 * q;
-    orr[q] = (unsigned)((e % KB + min(e / KB, nr - 1) * (int)ldr) * (int)sizeof(T));
-    ol[q] = (unsigned)((min(e % BT, nl - 1) + (e / BT) * (int)ldl) * (int)sizeof(T));
-  }
-  T vl[NQ], vr[NQ];
-  auto load = [&](int k0) {
-    const char* bl = reinterpret_cast<const char*>(L + (int64_t)k0 * ldl);
-    const char* br = reinterpret_cast<const char*>(R + k0);
-    if (k0 + KB <= K) {
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        vl[q] = *reinterpret_cast<const T*>(bl + ol[q]);
-        vr[q] = *reinterpret_cast<const T*>(br + orr[q]);
-      }
-    } else {
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        const int e = tid + 256 * q;
-        vl[q] = k0 + e / BT < K ? *reinterpret_cast<const T*>(bl + ol[q]) : s_zero(T());
-        vr[q] = k0 + e % KB < K ? *reinterpret_cast<const T*>(br + orr[q]) : s_zero(T());
-      }
-    }
-  };
-  auto store = [&](F* st) {
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      const int e = tid + 256 * q;
-      st[(e / BT) * C::PR + e % BT] = C::to(vl[q]);
-      st[SL + (e / KB) * C::PK + e % KB] = C::to(vr[q]);
-    }
-  };
-  F* st = reinterpret_cast<F*>(pool);
-  load(0);
-  store(st);
-  int cur = 0;
-  for (int k0 = 0; k0 < K; k0 += KB) {
-    const bool more = k0 + KB < K;
-    if (more) load(k0 + KB);
-    __syncthreads();
-    const F* c = st + cur * STAGE;
-#pragma unroll
-    for (int kk = 0; kk < KB; kk += 4) {
-      F a[2], b[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        a[i] = c[(kk + lq) * C::PR + wm * 32 + i * 16 + lr];
-        b[i] = c[SL + (wn * 32 + i * 16 + lr) * C::PK + kk + lq];
-      }
-      acc.step(a, b);
-    }
-    cur ^= 1;
-    if (more) store(st + cur * STAGE);
-  }
-  __syncthreads();
-}
-
 // One stage of KX inner indices held in the pool: left as [k][row], right as [col][k].
 template <typename T, bool CL>
 __device__ __forceinline__ void bcx_step(BcAcc<T>& acc, const T* left, const T* right) {
@@ -491,7 +360,6 @@ __global__ void bchol_decide_kernel(const BCholProb* P, int n, int* any, int pas
     const bool ok = s <= kBCholMaxE * kBCholMaxE;  // false for a NaN
     const int to = ok ? st : pass == 1 && s <= kBCholMaxE2 * kBCholMaxE2 ? 2 : 1;
     if (lane == 0) {
-      p.dev[0] = s;  // for the choice of the correction's precision
       *p.state = to;
       if (to == 1) *any = 1;  // every writer writes 1
     }
@@ -787,28 +655,6 @@ __global__ void __launch_bounds__(256, BcCfg<T>::OCC)
   if (t.kind == 0) {
     const int r0 = t.a * BT, rows = p.m - r0;
     T* Q = reinterpret_cast<T*>(p.Q) + r0;
-    if (p.dev[0] <= kBCholLoMaxE * kBCholLoMaxE) {
-      BcLo<T> lo;
-      for (int jb = p.np / BT - 1; jb >= 0; --jb) {
-        const int j0 = jb * BT, ldq = bc_local(p.ldq);
-        lo.zero();
-        bc_product_lo<T>(lo, pool, Q, ldq, rows, U + (int64_t)j0 * p.np, p.np, BT, min(j0 + BT, p.n));
-        T* Qj = Q + (int64_t)j0 * p.ldq;
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const int r = ri + 16 * i, c = wn * 32 + 16 * j + 4 * lq + u;
-              if (r < rows && j0 + c < p.n) {
-                T* q = Qj + r + c * ldq;
-                *q = s_sub(*q, lo.get(i, j, u));
-              }
-            }
-      }
-      return;
-    }
     for (int jb = p.np / BT - 1; jb >= 0; --jb) {
       const int j0 = jb * BT, ldq = bc_local(p.ldq);
       acc.zero();

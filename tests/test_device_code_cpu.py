@@ -57,6 +57,20 @@ def listing(tmp_path_factory):
     return out
 
 
+@pytest.fixture(scope="module")
+def listing_by_kernel(listing):
+    """The set of opcodes of each kernel, by its mangled name."""
+    out, name = {}, None
+    for line in listing:
+        head = re.fullmatch(r"[0-9a-f]+ <(\S+)>:", line)
+        if head:
+            name = head[1]
+            out.setdefault(name, set())
+        elif name is not None and line:
+            out[name].add(line.split()[0])
+    return out
+
+
 def registers(operand):
     """The VGPR numbers of an operand such as v7, -v[4:5]."""
     m = re.fullmatch(r"-?\|?v(?:(\d+)|\[(\d+):(\d+)\])\|?", operand.strip())
@@ -103,3 +117,13 @@ def test_dpp_sources_are_waited_for(listing):
     assert reads > 1000 and blocks > 1000, (reads, blocks)
     assert not close, (len(close), close[:3])
     assert not loose, (len(loose), loose[:3])
+
+
+def test_batched_blocks_stay_in_64_bits(listing_by_kernel):
+    """The batched factorisation of whole blocks is Float64 / ComplexF64
+    throughout: no kernel of it converts to 32 bits or multiplies in them."""
+    kernels = {k: v for k, v in listing_by_kernel.items() if "bchol" in k or "qr_small" in k or "qr_tall" in k}
+    assert len(kernels) >= 15, sorted(kernels)
+    for name, ops in kernels.items():
+        low = {op for op in ops if re.match(r"v_mfma_f32|v_cvt_f32_f64|v_cvt_f16|v_cvt_pk_bf16|v_fma(c|mk|ak)?_f32", op)}
+        assert not low, (name, low)
