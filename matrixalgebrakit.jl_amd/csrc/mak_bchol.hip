@@ -427,8 +427,11 @@ __global__ void __launch_bounds__(256, BcCfg<T>::OCC_GRAM)
 // 32 x 32 blocks in S[0], S[64], S[128] (rows of 33; S[32], S[96] scratch) become
 // R (W, ld) and R^{-1} (X, ld 64) with zeros below the diagonal.  True if a
 // pivot was not positive.  The blocks were written before a barrier here.
+// cond (optional): the largest ||R(:, k)||^2 ||R^{-1}(k, :)||^2, the inverse
+// square of the sine between a column and the span of the others; red: 4 in LDS.
 template <typename T>
-__device__ __forceinline__ bool bc_chol64(T (*S)[33], int* bad_s, T* W, int64_t ld, T* X) {
+__device__ __forceinline__ bool bc_chol64(T (*S)[33], int* bad_s, T* W, int64_t ld, T* X, double* cond = nullptr,
+                                          double* red = nullptr) {
   T (*S11)[33] = S;
   T (*Y11)[33] = S + 32;
   T (*S12)[33] = S + 64;  // then Y22
@@ -466,10 +469,33 @@ __device__ __forceinline__ bool bc_chol64(T (*S)[33], int* bad_s, T* W, int64_t 
     W[i + (int64_t)j * ld] = wv;
     if (i >= 32 || j < 32) X[e] = xv;
   }
+  // four threads a column
+  const int kc = threadIdx.x >> 2, kr = kc & 31, kq = 8 * (threadIdx.x & 3);
+  double cn = 0.0, rn = 0.0;
+  if (cond != nullptr) {
+    const T (*C1)[33] = kc < 32 ? S11 : W12;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) cn += s_abs2(C1[kq + i][kr]) + (kc < 32 ? 0.0 : s_abs2(S22[kq + i][kr]));
+  }
   __syncthreads();
   mm32<T>(S22, W12, false, S12, false, 1.0, false);
   mm32<T>(S22, Y11, false, S22, false, -1.0, false);
   for (int e = threadIdx.x; e < 32 * 32; e += 256) X[e % 32 + (32 + e / 32) * BT] = S22[e % 32][e / 32];
+  if (cond != nullptr) {
+    const T (*R1)[33] = kc < 32 ? Y11 : S12;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) rn += s_abs2(R1[kr][kq + i]) + (kc < 32 ? s_abs2(S22[kr][kq + i]) : 0.0);
+    cn += __shfl_xor(cn, 1);
+    rn += __shfl_xor(rn, 1);
+    cn += __shfl_xor(cn, 2);
+    rn += __shfl_xor(rn, 2);
+    double d = cn * rn;
+#pragma unroll
+    for (int h = 4; h < 64; h *= 2) d = fmax(d, __shfl_xor(d, h));
+    if (lane == 0) red[w] = d;
+    __syncthreads();
+    if (threadIdx.x == 0) *cond = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+  }
   return *bad_s != 0;
 }
 
@@ -1020,6 +1046,9 @@ struct TallArgs {
   int m, n, rps;
 };
 
+// bc_chol64's conditioning of R1, after the ints of ctl
+__device__ __forceinline__ double* tall_cond(int* ctl) { return reinterpret_cast<double*>(ctl + 4); }
+
 template <typename T, int PASS>
 __global__ void __launch_bounds__(256) qr_tall_kernel(const TallArgs p) {
   using C = BcCfg<T>;
@@ -1037,8 +1066,15 @@ __global__ void __launch_bounds__(256) qr_tall_kernel(const TallArgs p) {
   BcAcc<T> acc;
   if constexpr (PASS == 1) {
     if (p.ctl[3]) return;  // G was not positive definite
-    for (int b0 = 0; b0 < rows; b0 += BT) {
+    // Q1 = A X, then Q1 += (A - Q1 R1) X: the product alone leaves a residual of
+    // u cond(R1) (100 x 63 with two columns 1e-4 apart: 4e-13 of ||A||; with the
+    // second round 3e-16), which well-conditioned inputs do without (512 x 32: 96 us
+    // a call, 106 with it; 16384 x 32: 152 and 199)
+    const bool refine = *tall_cond(p.ctl) > kBCholRefine * kBCholRefine;
+    for (int b0 = 0, round = 0; b0 < rows;) {
       T v[2][2][4];
+      acc.zero();
+      if (round) bc_product<T, false>(acc, pool, Q + b0, p.ldq, rows - b0, W, BT, BT, n);
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -1046,7 +1082,7 @@ __global__ void __launch_bounds__(256) qr_tall_kernel(const TallArgs p) {
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const int r = b0 + ri + 16 * i, c = cj + 16 * j + 4 * u;
-            v[i][j][u] = r < rows && c < n ? A[r + (int64_t)c * p.lda] : s_zero(T());
+            v[i][j][u] = r < rows && c < n ? s_sub(A[r + (int64_t)c * p.lda], acc.get(i, j, u)) : s_zero(T());
           }
       bc_times_x<T>(acc, pool, v, X, BT);
 #pragma unroll
@@ -1056,8 +1092,14 @@ __global__ void __launch_bounds__(256) qr_tall_kernel(const TallArgs p) {
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const int r = b0 + ri + 16 * i, c = cj + 16 * j + 4 * u;
-            if (r < rows && c < n) Q[r + (int64_t)c * p.ldq] = acc.get(i, j, u);
+            if (r < rows && c < n) {
+              T* q = Q + r + (int64_t)c * p.ldq;
+              *q = round ? s_add(*q, acc.get(i, j, u)) : acc.get(i, j, u);
+            }
           }
+      __syncthreads();  // the second round reads the rows in every wave
+      if (round || !refine) b0 += BT;
+      round = !round && refine;
     }
     __syncthreads();
   }
@@ -1108,7 +1150,7 @@ __global__ void __launch_bounds__(256) qr_tall_kernel(const TallArgs p) {
     S[64 * q + r][c] = v;
   }
   if constexpr (PASS == 0) {
-    const bool bad = bc_chol64<T>(S, &bad_s, W, BT, X);
+    const bool bad = bc_chol64<T>(S, &bad_s, W, BT, X, tall_cond(p.ctl), red);
     if (tid == 0) p.ctl[3] = bad;
   } else {
     s2 = wave_sum(s2);

@@ -43,3 +43,11 @@ def test_small_near_parallel(m, n, j, dt, dev):
     for cond in (1e2, 1e3):
         A = near_parallel(m, n, j, cond, dt, 3)
         check(A, *mak.qr_compact(to_dev(A, dev)))
+
+
+@DTYPES
+@pytest.mark.parametrize("m,n,j", [(64, 33, 32), (100, 63, 32), (600, 40, 1), (600, 40, 39), (5000, 63, 62), (700, 32, 1)])
+def test_tall_near_parallel(m, n, j, dt, dev):
+    for cond in (1e2, 1e4):
+        A = near_parallel(m, n, j, cond, dt, 5)
+        check(A, *mak.qr_compact(to_dev(A, dev)))
