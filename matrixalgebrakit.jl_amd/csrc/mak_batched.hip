@@ -795,15 +795,12 @@ WholeLists whole_lists(const std::vector<BProb>& P, const std::vector<int>& idx,
   // the second pass: the same tasks, and the composition of the R factors
   // (R = R2 R1, then back to R1's place)
   const std::vector<WholeLists::Launch> first = out.launches;
-  auto again = [&](WholeLists::Launch l, BCholPhase phase) {
-    l.phase = phase;
+  auto again = [&](WholeLists::Launch l) {
     l.pass = 2;
     out.launches.push_back(l);
   };
-  for (const auto& l : first)
-    if (l.phase == BCHOL_SOLVE) again(l, BCHOL_RESOLVE);
   for (const auto& l : first) {
-    again(l, l.phase);
+    again(l);
     if (l.phase == BCHOL_SOLVE)
       for (int kind : {2, 3}) {
         r_tiles(kind);

@@ -6,12 +6,10 @@
 // E is what the condition of G left of the rounding of R1; with
 // ||E||_F <= 1e-8 (condition numbers to about 2e4) the terms of second order in
 // U are below rounding, so that the second factorisation is U itself.  With
-// ||E||_F <= 0.1 (to about 1e7) a second pass comes between: Q1 with one step
-// of refinement (its residual A - Q1 R1 would grow with the condition of R1's
-// diagonal tiles), the Cholesky factor R2 of Q1^H Q1, Q1 <- Q1 R2^{-1},
-// R1 <- R2 R1.  A block whose Gram matrix has a pivot that is not positive, or
-// whose E is larger, is rejected: left to the gated Householder launches.  A is
-// only read.
+// ||E||_F <= 0.1 (to about 1e7) a second pass comes between: the Cholesky factor
+// R2 of Q1^H Q1, Q1 <- Q1 R2^{-1}, R1 <- R2 R1.  A block whose Gram matrix has a
+// pivot that is not positive, or whose E is larger, is rejected: left to the
+// gated Householder launches.  A is only read.
 //
 // Every product runs on 64 x 64 tiles, one workgroup of four waves (32 x 32
 // each) per task, over task lists of all blocks:
@@ -21,8 +19,8 @@
 //             factor diagonal tile k+1, so that a step is one launch
 //   solve     64-row strips, block column by block column:
 //             Q1_j = (A_j - sum_i Q1_i R_ij) R_jj^{-1}.  Substitution and not
-//             a product with R1^{-1}: its residual does not grow with the
-//             condition number of R1
+//             a product with R1^{-1}, refined where R_jj is ill conditioned:
+//             its residual does not grow with the condition number of R1
 //   Gram      E, and its tiles' norms
 //   correct   Q1 - Q1 U in place, strips from the last block column to the
 //             first; the tiles of R
@@ -510,6 +508,7 @@ __global__ void __launch_bounds__(256) bchol_factor_kernel(const BCholProb* P, c
   using C = BcCfg<T>;
   __shared__ T pool[C::POOL > 5 * 32 * 33 ? C::POOL : 5 * 32 * 33];
   __shared__ int bad_s, state_s;
+  __shared__ double red[4];
   const BCholTask t = tasks[blockIdx.x];
   if (t.prob < 0) return;
   const BCholProb p = P[t.prob];
@@ -579,15 +578,20 @@ __global__ void __launch_bounds__(256) bchol_factor_kernel(const BCholProb* P, c
           S[16 * i + lr][16 * j + 4 * u + lq] =
               s_sub(Wbb[ri + 16 * i + (int64_t)(cj + 16 * j + 4 * u) * ld], acc.get(i, j, u));
   }
-  const bool bad = bc_chol64<T>(S11, &bad_s, Wbb, ld, Xd + (int64_t)b * BT * BT);
+  const bool bad = bc_chol64<T>(S11, &bad_s, Wbb, ld, Xd + (int64_t)b * BT * BT, p.dev + b * (p.np / BT + 1), red);
   if (threadIdx.x == 0 && bad) __hip_atomic_store(p.state, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Strip a (64 rows) of Q1 = A R1^{-1}; second: of Q1 <- Q1 R2^{-1}, in place.
-// REFINE: with Q1_j += (B_j - Q1_j R_jj) R_jj^{-1} for each block column.
+// Strip a (64 rows) of Q1 = A R1^{-1}, block column by block column; second: of
+// Q1 <- Q1 R2^{-1}, in place.  A block column whose diagonal tile has a column
+// closer than kBCholRefine to the span of the others (bc_chol64) gets a second
+// round, Q1_j += (A_j - sum_{i<=j} Q1_i R_ij) R_jj^{-1}: the residual of the
+// first is about u times that quotient, 5e-16 of ||A|| at 8 and 1e-14 at 1e3
+// (Householder QR 5e-16).  Of Gaussian blocks only the last tiles of nearly
+// square ones pass the limit.  R2 is near the identity and needs none.
 // Bound by the operands' path through L2 (8 flops a byte; 5.4 GB of 4096 Float64
 // blocks come from beyond it) and the chain of block columns.
-template <typename T, bool REFINE>
+template <typename T>
 __global__ void __launch_bounds__(256, BcCfg<T>::OCC)
     bchol_solve_kernel(const BCholProb* P, const BCholTask* tasks, int pass, int second) {
   using C = BcCfg<T>;
@@ -605,10 +609,10 @@ __global__ void __launch_bounds__(256, BcCfg<T>::OCC)
   const int lr = lane & 15, lq = lane >> 4, wm = w & 1, wn = w >> 1;
   const int ri = wm * 32 + lr, cj = wn * 32 + lq;
   BcAcc<T> acc;
-  for (int jb = 0; jb * BT < p.n; ++jb) {
+  for (int jb = 0, round = 0; jb * BT < p.n;) {
     const int j0 = jb * BT, lda = bc_local(second ? p.ldq : p.lda), ldq = bc_local(p.ldq);
     acc.zero();
-    bc_product<T, false>(acc, pool, Q, ldq, rows, W + (int64_t)j0 * p.np, p.np, BT, j0);
+    bc_product<T, false>(acc, pool, Q, ldq, rows, W + (int64_t)j0 * p.np, p.np, BT, min(j0 + round * BT, p.n));
     T v[2][2][4];
     const T* Aj = A + (int64_t)j0 * p.lda;
 #pragma unroll
@@ -620,38 +624,7 @@ __global__ void __launch_bounds__(256, BcCfg<T>::OCC)
           const int r = ri + 16 * i, c = cj + 16 * j + 4 * u;
           v[i][j][u] = (r < rows && j0 + c < p.n) ? s_sub(Aj[r + c * lda], acc.get(i, j, u)) : s_zero(T());
         }
-    const T* X = Xd + (int64_t)jb * BT * BT;
-    bc_times_x<T>(acc, pool, v, X, BT);
-    if constexpr (REFINE) {
-      T q[2][2][4];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int u = 0; u < 4; ++u) q[i][j][u] = acc.get(i, j, u);
-      bc_times_x<T>(acc, pool, q, W + (int64_t)j0 * (p.np + 1), p.np);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int u = 0; u < 4; ++u) v[i][j][u] = s_sub(v[i][j][u], acc.get(i, j, u));
-      bc_times_x<T>(acc, pool, v, X, BT);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int u = 0; u < 4; ++u) v[i][j][u] = s_add(q[i][j][u], acc.get(i, j, u));
-    } else {
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int u = 0; u < 4; ++u) v[i][j][u] = acc.get(i, j, u);
-    }
+    bc_times_x<T>(acc, pool, v, Xd + (int64_t)jb * BT * BT, BT);
     T* Qj = Q + (int64_t)j0 * p.ldq;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -660,9 +633,18 @@ __global__ void __launch_bounds__(256, BcCfg<T>::OCC)
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const int r = ri + 16 * i, c = cj + 16 * j + 4 * u;
-          if (r < rows && j0 + c < p.n) Qj[r + c * ldq] = v[i][j][u];
+          if (r < rows && j0 + c < p.n) {
+            T* q = Qj + r + c * ldq;
+            *q = round ? s_add(*q, acc.get(i, j, u)) : acc.get(i, j, u);
+          }
         }
-    __syncthreads();  // the next block column reads this one in every wave
+    __syncthreads();  // what follows reads this block column in every wave
+    if (round == 0 && !second && p.dev[jb * (p.np / BT + 1)] > kBCholRefine * kBCholRefine) {
+      round = 1;
+    } else {
+      round = 0;
+      ++jb;
+    }
   }
 }
 
@@ -1299,8 +1281,7 @@ void launch_bchol(BCholPhase phase, const BCholProb* P, const BCholTask* tasks, 
   switch (phase) {
     case BCHOL_GRAM1: hipLaunchKernelGGL((bchol_gram_kernel<T, false>), g, b, 0, s, P, tasks, pass); break;
     case BCHOL_FACTOR: hipLaunchKernelGGL((bchol_factor_kernel<T>), g, b, 0, s, P, tasks, pass); break;
-    case BCHOL_SOLVE: hipLaunchKernelGGL((bchol_solve_kernel<T, false>), g, b, 0, s, P, tasks, pass, pass == 2); break;
-    case BCHOL_RESOLVE: hipLaunchKernelGGL((bchol_solve_kernel<T, true>), g, b, 0, s, P, tasks, pass, 0); break;
+    case BCHOL_SOLVE: hipLaunchKernelGGL((bchol_solve_kernel<T>), g, b, 0, s, P, tasks, pass, pass == 2); break;
     case BCHOL_GRAM2: hipLaunchKernelGGL((bchol_gram_kernel<T, true>), g, b, 0, s, P, tasks, pass); break;
     case BCHOL_CORRECT:
     case BCHOL_COMPOSE: hipLaunchKernelGGL((bchol_correct_kernel<T>), g, b, 0, s, P, tasks, pass); break;

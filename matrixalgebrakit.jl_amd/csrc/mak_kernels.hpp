@@ -71,14 +71,15 @@ struct BCholProb {
   void* U;        // np x np scratch: U (upper tiles)
   void* X;        // np / 64 scratch blocks of 64 x 64: inverses of R1's diagonal tiles
   int* state;     // out: 1 if the block is left to the gated Householder launches
-  double* dev;    // (np / 64)^2 scratch: squared norms of E's tiles, (a, b) at a + b np / 64
+  double* dev;    // (np / 64)^2 scratch: squared norms of E's tiles, (a, b) at a + b np / 64; before
+                  // that (b, b) holds the conditioning of R1's diagonal tile b
   int m, n, np;   // np: n rounded up to a multiple of 64; m >= n >= 1
 };
 struct BCholTask {
   int prob;  // < 0: nothing to do
   int a, b, kind;
 };
-enum BCholPhase { BCHOL_GRAM1, BCHOL_FACTOR, BCHOL_SOLVE, BCHOL_RESOLVE, BCHOL_GRAM2, BCHOL_CORRECT, BCHOL_COMPOSE };
+enum BCholPhase { BCHOL_GRAM1, BCHOL_FACTOR, BCHOL_SOLVE, BCHOL_GRAM2, BCHOL_CORRECT, BCHOL_COMPOSE };
 void launch_bchol_init(int* state, int n, int* any, int* status, int nst, hipStream_t s);
 void launch_bchol_decide(const BCholProb* P, int n, int* any, int pass, hipStream_t s);
 template <typename T>

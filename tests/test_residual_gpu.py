@@ -51,3 +51,17 @@ def test_tall_near_parallel(m, n, j, dt, dev):
     for cond in (1e2, 1e4):
         A = near_parallel(m, n, j, cond, dt, 5)
         check(A, *mak.qr_compact(to_dev(A, dev)))
+
+
+@DTYPES
+def test_whole_blocks_near_parallel(dt, dev):
+    """Columns of one 64-column tile and of different ones; one pass and two."""
+    host = [near_parallel(m, n, j, cond, dt, 7)
+            for m, n, j in ((64, 40, 1), (100, 64, 32), (130, 128, 127), (200, 150, 140), (300, 190, 65), (400, 64, 63))
+            for cond in (1e2, 1e3, 1e5)]
+    plan = mak.BatchedQRPlan([to_dev(h, dev) for h in host])
+    Qs, Rs = plan.execute()
+    torch.cuda.synchronize()
+    for h, q, r in zip(host, Qs, Rs):
+        check(h, q, r)
+    plan.close()
