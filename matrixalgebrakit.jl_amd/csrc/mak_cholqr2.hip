@@ -258,9 +258,10 @@ __global__ void __launch_bounds__(256) sum_r_slices_kernel(const T* P, int ks, i
 // st[0] = 1 (accept) when the Cholesky succeeded (info == 0) and ||E||_F <=
 // 1e-6; st[1] = 1 when the second-order terms are needed (||E||_F > 1e-9);
 // of the accepted calls, exactly one of st[7], st[3], st[6] is 1: Q = Q1 +
-// Q1 (W2^{-1} - I) takes its correction from BF16 MFMA (st[7]: lo_ok and
+// Q1 (W2^{-1} - I) may take its correction from BF16 MFMA (st[7]: lo_ok and
 // ||E||_F <= kBf16CorrMaxE) or from FP32 MFMA (st[3]: lo_ok and ||E||_F <=
-// kLoCorrMaxE), else Q = Q1 W2^{-1} runs on FP64 MFMA (st[6]);
+// kLoCorrMaxE), else Q = Q1 W2^{-1} runs on FP64 MFMA (st[6]), as it does in any
+// case below the size where the others are faster;
 // st[4..5] = ||E||_F as a double.
 __global__ void cq2_decide_kernel(const double* part, int np, const int* cinfo, int lo_ok, int* st) {
   __shared__ double red[4];
@@ -337,10 +338,12 @@ bool cholqr2_eligible(int m, int n) { return m >= n && n >= 1 && n <= kCholTileM
 // Enqueues the whole-matrix CholeskyQR2 on s; Q (m x n) and R (n x n or null)
 // receive the factors when the device-side check accepts (status word at
 // cholqr2_status(ws): [0] = 1 accepted; its eight words are 0 on entry).  ws:
-// cholqr2_workspace_bytes(m, n).
+// cholqr2_workspace_bytes(m, n).  lo: the correction may run on BF16 / FP32
+// MFMA where that is faster (a call that documents it); else it runs on FP64
+// (8192 x 1024 Float64: 0.1 ms more).
 template <typename T>
 void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q, int64_t ldq, T* R, int64_t ldr,
-                     char* ws) {
+                     char* ws, bool lo) {
   const CQ2Layout L = cq2_layout<T>(m, n);
   T* Q1 = reinterpret_cast<T*>(ws + L.offQ1);
   T* G = reinterpret_cast<T*>(ws + L.offG);   // G1, then R1
@@ -355,6 +358,12 @@ void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q,
   int* st = reinterpret_cast<int*>(ws + L.offSt);
   const int64_t nn = (int64_t)n * n;
   const unsigned eg = (unsigned)cdiv64(nn, 256);
+  // The low-precision correction pays from about 2e9 (complex 3e9) multiply-adds;
+  // below, its packing and launches cost more than they save.  The call, us, low /
+  // FP64: Float64 100 x 64 157 / 135, 1024 x 256 257 / 235, 4096 x 512 429 / 421,
+  // 2048 x 1024 766 / 783, 8192 x 1024 1070 / 1170; ComplexF64 700 x 64 221 / 156,
+  // 1024 x 256 404 / 347, 2048 x 1024 1630 / 1540, 4096 x 1024 1710 / 1910.
+  const bool low = lo && (double)m * (double)nn >= (ScalarTraits<T>::is_complex ? 3e9 : 2e9);
   // pass 1: Q1 = A X1 inside the Cholesky launch, column block by column
   // block as X1 becomes final
   gram_upper<T>(A, lda, m, n, G, X, L.kcap, s);
@@ -366,7 +375,7 @@ void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q,
   // sweep), the decision, and W2, W2^{-1} in closed form
   const int ks2 = gram_upper_slices<T>(Q1, m, m, n, X, L.kcap, s);
   hipLaunchKernelGGL((cq2_sum_up_kernel<T>), dim3(kRedWgs), dim3(256), 0, s, X, ks2, n, E, U, part);
-  hipLaunchKernelGGL(cq2_decide_kernel, dim3(1), dim3(256), 0, s, part, kRedWgs, st + 2, 1, st);
+  hipLaunchKernelGGL(cq2_decide_kernel, dim3(1), dim3(256), 0, s, part, kRedWgs, st + 2, lo ? 1 : 0, st);
   // second order (st[1] == 1): U = up(E - U1^H U1), U2 = U U
   {
     GemmArgs g = gq<T>(n, n, n, U, n, U, n, Tm, n, 1.0, 0.0, TRI_A_LOWER | TRI_B_UPPER, st + 1, 1);
@@ -379,16 +388,16 @@ void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q,
   T* D = E;
   hipLaunchKernelGGL((cq2_w_kernel<T>), dim3(eg), dim3(256), 0, s, U, Tm, st, n, W, X, D);
   // Q = Q1 W2^{-1};  R = W2 R1 (R1 is upper with a zero strict lower part).
-  // ||E|| small: Q = Q1 + Q1 D with the correction on BF16 (st[7]) or FP32
+  // low and ||E|| small: Q = Q1 + Q1 D with the correction on BF16 (st[7]) or FP32
   // (st[3]) MFMA (complex data through its real embedding; the packed
   // operands go where the Gram slices were); else Q1 W2^{-1} on FP64
-  {
+  if (low) {
     GemmArgs g = gq<T>(m, n, n, Q1, m, D, n, Q, ldq, 1.0, 1.0, TRI_B_UPPER);
     g.Cin = Q1;
     g.ldcin = m;
     gemm_lo_reduced(g, OP_N, OP_N, st + 7, st + 3, Sl, s, ScalarTraits<T>::is_complex);
-    gemm<T>(OP_N, OP_N, gq<T>(m, n, n, Q1, m, X, n, Q, ldq, 1.0, 0.0, TRI_B_UPPER, st + 6, 1), s);
   }
+  gemm<T>(OP_N, OP_N, gq<T>(m, n, n, Q1, m, X, n, Q, ldq, 1.0, 0.0, TRI_B_UPPER, low ? st + 6 : st, 1), s);
   if (R != nullptr) {
     // complex data: R = W2 R1 = R1 + U R1 with the correction on BF16 (st[7])
     // or FP32 (st[3]) MFMA, else (st[6]) on FP64.  U R1 (upper x upper) is
@@ -396,7 +405,7 @@ void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q,
     // too.  (Real data: the split-K FP64 product below is as fast at n ~ 1e3
     // as the packing and launches of the low-precision one.)
     const int* r64 = st;
-    if constexpr (ScalarTraits<T>::is_complex) {
+    if (ScalarTraits<T>::is_complex && low) {
       GemmArgs g = gq<T>(n, n, n, U, n, G, n, R, ldr, 1.0, 1.0, TRI_B_UPPER);
       g.Cin = G;
       g.ldcin = n;
@@ -437,8 +446,8 @@ template <typename T> Cholqr2Buffers<T> cholqr2_buffers(char* ws, int m, int n) 
 template size_t cholqr2_workspace_bytes<double>(int, int);
 template size_t cholqr2_workspace_bytes<zd>(int, int);
 template void cholqr2_enqueue<double>(hipStream_t, int, int, const double*, int64_t, double*, int64_t, double*,
-                                      int64_t, char*);
-template void cholqr2_enqueue<zd>(hipStream_t, int, int, const zd*, int64_t, zd*, int64_t, zd*, int64_t, char*);
+                                      int64_t, char*, bool);
+template void cholqr2_enqueue<zd>(hipStream_t, int, int, const zd*, int64_t, zd*, int64_t, zd*, int64_t, char*, bool);
 template int* cholqr2_status<double>(char*, int, int);
 template int* cholqr2_status<zd>(char*, int, int);
 template Cholqr2Buffers<double> cholqr2_buffers<double>(char*, int, int);

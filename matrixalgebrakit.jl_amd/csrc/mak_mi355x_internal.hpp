@@ -68,7 +68,7 @@ bool cholqr2_eligible(int m, int n);
 template <typename T> size_t cholqr2_workspace_bytes(int m, int n);
 template <typename T>
 void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q, int64_t ldq, T* R, int64_t ldr,
-                     char* ws);
+                     char* ws, bool lo);
 template <typename T> int* cholqr2_status(char* ws, int m, int n);
 template <typename T> T* cholqr2_scratch(char* ws, int m, int n);
 // Workspace of a cholqr2_enqueue call that is free once its launches are

@@ -576,9 +576,11 @@ template <typename T> void qr_record(const char* ws, int m, int n, int full, int
   out[3] = L.offCq2 != 0;          // the whole-matrix path exists for this shape
   out[4] = st[4];                  // ||E||_F of the whole-matrix path (a double in out[4..5])
   out[5] = st[5];
-  out[6] = st[3];                  // 1: its final product took the FP32 correction
-  out[7] = st[6];                  // 1: its final product ran on FP64
-  out[8] = st[7];                  // 1: its final product took the BF16 correction
+  // the precision that ||E|| allows the final product (large matrices of qr_compact! with
+  // positive = true take it, the others run on FP64):
+  out[6] = st[3];                  // 1: FP32 correction
+  out[7] = st[6];                  // 1: FP64
+  out[8] = st[7];                  // 1: BF16 correction
 }
 
 template <typename T>
@@ -641,7 +643,8 @@ int qr_driver(hipStream_t s, int full, int m, int n, T* A, int64_t lda, T* Q, in
   // Householder signs of positive = false follow from its Q.  The signs are
   // those of the panel path: for a square matrix the last column's reflector
   // is the identity there, and for complex data its last panels (under
-  // kCholQrMinRows rows) take real signs, so those forms stay on it.
+  // kCholQrMinRows rows) take real signs, so those forms stay on it.  Both run
+  // on FP64 throughout, as the panels do.
   const bool signs = !positive || (full && m > n);
   T* Qd = inplace ? reinterpret_cast<T*>(ws + L.offQs) : Q;
   const int64_t ldqd = inplace ? m : ldq;
@@ -650,7 +653,7 @@ int qr_driver(hipStream_t s, int full, int m, int n, T* A, int64_t lda, T* Q, in
                      (!signs || (m > n && (!ScalarTraits<T>::is_complex || m - (n - 1) / NB * NB >= kCholQrMinRows)));
   if (whole) {
     char* cw = ws + L.offCq2;
-    cholqr2_enqueue<T>(s, m, n, A, lda, Qd, ldqd, R, ldr, cw);
+    cholqr2_enqueue<T>(s, m, n, A, lda, Qd, ldqd, R, ldr, cw, !signs);
     if (signs) qr_trailing_enqueue<T>(s, m, n, Qd, ldqd, R, ldr, full, positive, cw);
     int st = 0;
     if (hipMemcpyAsync(&st, cholqr2_status<T>(cw, m, n), sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||

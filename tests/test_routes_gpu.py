@@ -33,8 +33,9 @@ def to_dev(A, dev):
     return mak.colmajor(torch.from_numpy(np.asfortranarray(A)).to(dev))
 
 
-def run_record(A, dev, full=False, positive=True):
-    """Q, R and whether the whole matrix's CholeskyQR2 was accepted."""
+def run_record(A, dev, full=False, positive=True, words=False):
+    """Q, R and whether the whole matrix's CholeskyQR2 was accepted (words: the
+    whole record)."""
     At = to_dev(A, dev)
     m, n = At.shape
     Q, R = mak.initialize_output_qr(At, full)
@@ -51,7 +52,7 @@ def run_record(A, dev, full=False, positive=True):
     lib.maktest_qr_record.argtypes = [C.c_int, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p]
     rec = (C.c_int * 9)()
     assert lib.maktest_qr_record(dt, int(full), m, n, C.c_void_p(ws.data_ptr()), rec) == 0
-    return Q.cpu().numpy(), R.cpu().numpy(), rec[0]
+    return Q.cpu().numpy(), R.cpu().numpy(), list(rec) if words else rec[0]
 
 
 def routes(plan):
@@ -140,3 +141,23 @@ def test_panels_of_a_plan_without_the_gauge(dt, dev):
     for i in range(0, 120, 17):
         sound(host[i], Qs[i].cpu().numpy(), Rs[i].cpu().numpy())
     plan.close()
+
+
+@DTYPES
+@pytest.mark.parametrize("m,n", [(500, 100), (2100, 1024)])
+@pytest.mark.parametrize("full,positive", [(True, True), (True, False), (False, False)])
+def test_signed_and_full_run_on_fp64(m, n, full, positive, dt, dev):
+    """Only qr_compact! with positive = True may form its final correction on BF16
+    or FP32 MFMA (record: FP32, FP64, BF16 in words 6 to 8)."""
+    A = O.gaussian(m, n, dt, seed=11)
+    assert run_record(A, dev, full, positive, words=True)[2][6:9] == [0, 1, 0]
+
+
+@DTYPES
+def test_small_compact_is_the_full_factorisation(dt, dev):
+    """Below the size where the low-precision correction is faster, qr_compact! and
+    qr_full! run the same FP64 products: the same bits."""
+    for m, n in ((100, 64), (900, 200)):
+        A = to_dev(O.gaussian(m, n, dt, seed=12), dev)
+        (Qc, Rc), (Qf, Rf) = mak.qr_compact(A), mak.qr_full(A)
+        assert torch.equal(Qc, Qf[:, :n]) and torch.equal(Rc, Rf[:n])
