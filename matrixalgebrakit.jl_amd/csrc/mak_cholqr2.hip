@@ -53,6 +53,11 @@ constexpr double kLoCorrMaxE = 1e-10;
 // and in practice (errors of random sign) some thirty times less.
 constexpr double kBf16CorrMaxE = 5e-14;
 
+// Columns of R1 closer than 1 / kRefineCond to the span of the others: the
+// residual of A R1^{-1} by the computed inverse passes what Householder QR
+// leaves (about 5e-16 of ||A|| here) and grows in proportion.
+constexpr double kRefineCond = 8.0;
+
 struct CQ2Layout {
   size_t offQ1, offG, offE, offX, offU, offW, offT, offSl, offFlags, offPart, offSt, offXc, bytes;
   int ks;    // split-K slices reserved for the Gram products
@@ -326,6 +331,44 @@ __global__ void cq2_w_kernel(const T* U, const T* U2, const int* st, int n, T* W
   Wi[idx] = wi;
 }
 
+// *flag = 1 if the Cholesky succeeded and a column k of R is closer than 1 /
+// kRefineCond to the span of the others: ||R(:, k)|| ||X(k, :)|| > kRefineCond,
+// X = R^{-1}.  Sixteen columns a workgroup.
+template <typename T>
+__global__ void __launch_bounds__(256) cq2_cond_kernel(const T* R, const T* X, int n, const int* info, int* flag) {
+  __shared__ double cn[16], rn[16][17];
+  if (*info != 0) return;
+  const int k0 = blockIdx.x * 16, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int c = w; c < 16; c += 4) {
+    double s = 0.0;
+    if (k0 + c < n)
+      for (int i = lane; i <= k0 + c; i += 64) s += s_abs2(R[i + (int64_t)(k0 + c) * n]);
+    s = wave_sum(s);
+    if (lane == 0) cn[c] = s;
+  }
+  const int kk = threadIdx.x & 15, g = threadIdx.x >> 4;
+  double s = 0.0;
+  if (k0 + kk < n)
+    for (int j = k0 + g; j < n; j += 16) s += s_abs2(X[k0 + kk + (int64_t)j * n]);
+  rn[g][kk] = s;
+  __syncthreads();
+  if (threadIdx.x < 16 && k0 + kk < n) {
+    double r = 0.0;
+    for (int h = 0; h < 16; ++h) r += rn[h][kk];
+    if (cn[kk] * r > kRefineCond * kRefineCond) *flag = 1;  // every writer writes 1
+  }
+}
+
+// Y = B (m x n), when *gate == 1
+template <typename T>
+__global__ void __launch_bounds__(256) cq2_copy_kernel(const T* B, int64_t ldb, int m, T* Y, int64_t ldy, const int* gate) {
+  if (*gate != 1) return;
+  const T* b = B + (int64_t)blockIdx.y * ldb;
+  T* y = Y + (int64_t)blockIdx.y * ldy;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < m; i += gridDim.x * 256) y[i] = b[i];
+}
+
 }  // namespace
 
 template <typename T> size_t cholqr2_workspace_bytes(int m, int n) {
@@ -337,10 +380,10 @@ bool cholqr2_eligible(int m, int n) { return m >= n && n >= 1 && n <= kCholTileM
 
 // Enqueues the whole-matrix CholeskyQR2 on s; Q (m x n) and R (n x n or null)
 // receive the factors when the device-side check accepts (status word at
-// cholqr2_status(ws): [0] = 1 accepted; its eight words are 0 on entry).  ws:
+// cholqr2_status(ws): [0] = 1 accepted; its kCq2StatusWords are 0 on entry).  ws:
 // cholqr2_workspace_bytes(m, n).  lo: the correction may run on BF16 / FP32
 // MFMA where that is faster (a call that documents it); else it runs on FP64
-// (8192 x 1024 Float64: 0.1 ms more).
+// (8192 x 1024 Float64: 0.1 ms more), and Q1 is refined where R1 is ill conditioned.
 template <typename T>
 void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q, int64_t ldq, T* R, int64_t ldr,
                      char* ws, bool lo) {
@@ -370,6 +413,18 @@ void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q,
   {
     const CholRightProduct rp{A, lda, Q1, m, m, ws + L.offXc, L.ldxc};
     chol_tile_factor<T>(G, n, n, X, n, flags, st + 2, 0, s, 0, nullptr, &rp);
+  }
+  // Q1 = A X1 leaves a residual of u cond(R1), the panel path only one of its
+  // 32-column panels' conditions (600 x 160, columns 0 and 130 1e-4 apart: 1.5e-13
+  // and 7e-16 of ||A||).  So a call that the panels served before: Q1 += (A - Q1
+  // R1) X1 where R1 is ill conditioned, Q serving as scratch (2 x 2 m n^2 flops).
+  if (!lo) {
+    int* flag = st + 8;
+    hipLaunchKernelGGL((cq2_cond_kernel<T>), dim3(cdiv(n, 16)), dim3(256), 0, s, G, X, n, st + 2, flag);
+    hipLaunchKernelGGL((cq2_copy_kernel<T>), dim3(std::min(cdiv(m, 256), 16), n), dim3(256), 0, s, A, lda, m, Q, ldq,
+                       flag);
+    gemm<T>(OP_N, OP_N, gq<T>(m, n, n, Q1, m, G, n, Q, ldq, -1.0, 1.0, TRI_B_UPPER, flag, 1), s);
+    gemm<T>(OP_N, OP_N, gq<T>(m, n, n, Q, ldq, X, n, Q1, m, 1.0, 1.0, TRI_B_UPPER, flag, 1), s);
   }
   // pass 2: G2 = I + E (slices summed with U1 = up(E) and ||E||_F in one
   // sweep), the decision, and W2, W2^{-1} in closed form

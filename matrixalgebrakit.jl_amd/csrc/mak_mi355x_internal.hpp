@@ -64,6 +64,7 @@ void zero_ints2(int* p, int n, int* q, int m, hipStream_t s);  // n, m <= 64, on
 // word (cholqr2_status: [0] = 1 accepted, [2] Cholesky info, [4..5] ||E||_F
 // as a double) is valid once the stream reaches it.  cholqr2_scratch: its
 // m x n scratch (free after the call; the in-place Q mode reuses it).
+constexpr int kCq2StatusWords = 9;
 bool cholqr2_eligible(int m, int n);
 template <typename T> size_t cholqr2_workspace_bytes(int m, int n);
 template <typename T>

@@ -631,7 +631,7 @@ int qr_driver(hipStream_t s, int full, int m, int n, T* A, int64_t lda, T* Q, in
       return 1;
     if (st == 0) return hipGetLastError() == hipSuccess ? 0 : 1;
   }
-  zero_ints2(L.offCq2 ? cholqr2_status<T>(ws + L.offCq2, m, n) : nullptr, L.offCq2 ? 8 : 0,
+  zero_ints2(L.offCq2 ? cholqr2_status<T>(ws + L.offCq2, m, n) : nullptr, L.offCq2 ? kCq2StatusWords : 0,
              reinterpret_cast<int*>(ws + L.offFlags), L.offFlags ? 3 : 0, s);
   if (minmn == 0) {
     set_identity<T>(Q, ldq, m, qcols, s);

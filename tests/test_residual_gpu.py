@@ -65,3 +65,13 @@ def test_whole_blocks_near_parallel(dt, dev):
     for h, q, r in zip(host, Qs, Rs):
         check(h, q, r)
     plan.close()
+
+
+@DTYPES
+@pytest.mark.parametrize("full,positive", [(True, True), (True, False), (False, False)])
+@pytest.mark.parametrize("m,n,j", [(200, 64, 1), (200, 64, 33), (600, 160, 130), (700, 300, 299)])
+def test_signed_and_full_near_parallel(m, n, j, full, positive, dt, dev):
+    for cond in (1e2, 1e4):
+        A = near_parallel(m, n, j, cond, dt, 9)
+        f = mak.qr_full if full else mak.qr_compact
+        check(A, *f(to_dev(A, dev), mak.MI355XHouseholder(positive=positive)))
