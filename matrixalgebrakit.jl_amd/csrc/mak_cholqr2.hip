@@ -401,12 +401,12 @@ void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q,
   int* st = reinterpret_cast<int*>(ws + L.offSt);
   const int64_t nn = (int64_t)n * n;
   const unsigned eg = (unsigned)cdiv64(nn, 256);
-  // The low-precision correction pays from about 2e9 (complex 3e9) multiply-adds;
-  // below, its packing and launches cost more than they save.  The call, us, low /
-  // FP64: Float64 100 x 64 157 / 135, 1024 x 256 257 / 235, 4096 x 512 429 / 421,
-  // 2048 x 1024 766 / 783, 8192 x 1024 1070 / 1170; ComplexF64 700 x 64 221 / 156,
-  // 1024 x 256 404 / 347, 2048 x 1024 1630 / 1540, 4096 x 1024 1710 / 1910.
-  const bool low = lo && (double)m * (double)nn >= (ScalarTraits<T>::is_complex ? 3e9 : 2e9);
+  // Below about 1e9 (complex 5e8) multiply-adds the packing and launches of the
+  // low-precision correction cost more than it saves.  The call, us, low / FP64:
+  // Float64 100 x 64 157 / 135, 1024 x 256 257 / 235, 1501 x 777 630 / 634, 2048 x 1024
+  // 766 / 783, 8192 x 1024 1070 / 1170; ComplexF64 700 x 64 221 / 156, 1024 x 256 404 /
+  // 347, 3001 x 333 627 / 599, 1501 x 777 1090 / 1180, 4096 x 1024 1710 / 1910.
+  const bool low = lo && (double)m * (double)nn >= (ScalarTraits<T>::is_complex ? 5e8 : 1e9);
   // pass 1: Q1 = A X1 inside the Cholesky launch, column block by column
   // block as X1 becomes final
   gram_upper<T>(A, lda, m, n, G, X, L.kcap, s);
