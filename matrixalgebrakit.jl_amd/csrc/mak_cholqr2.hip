@@ -57,6 +57,10 @@ constexpr double kBf16CorrMaxE = 5e-14;
 // residual of A R1^{-1} by the computed inverse passes what Householder QR
 // leaves (about 5e-16 of ||A|| here) and grows in proportion.
 constexpr double kRefineCond = 8.0;
+// ... and by kHopelessCond: ||E||_F is then about u kHopelessCond^2 = 1e-4, beyond
+// what is accepted, and the call stops before Q1 is refined and its Gram matrix
+// formed (where the conditioning is looked at).
+constexpr double kHopelessCond = 1e6;
 
 struct CQ2Layout {
   size_t offQ1, offG, offE, offX, offU, offW, offT, offSl, offFlags, offPart, offSt, offXc, bytes;
@@ -184,9 +188,11 @@ __global__ void __launch_bounds__(256) sum_upper_slices_kernel(const T* P, int k
 }
 
 // The split-K slices (at most cap) of the upper Gram X^H X; returns their count.
-template <typename T> int gram_upper_slices(const T* X, int64_t ldx, int m, int n, T* slices, int cap, hipStream_t s) {
+template <typename T>
+int gram_upper_slices(const T* X, int64_t ldx, int m, int n, T* slices, int cap, hipStream_t s,
+                      const int* gate = nullptr) {
   const GramPlan p = gram_plan<T>(m, n, cap);
-  GemmArgs g = gq<T>(n, n, m, X, ldx, X, ldx, slices, n, 1.0, 0.0, 0);
+  GemmArgs g = gq<T>(n, n, m, X, ldx, X, ldx, slices, n, 1.0, 0.0, 0, gate, 0);
   g.upperC = 1;
   if (!ScalarTraits<T>::is_complex) g.tile = p.tile;
   g.kchunk = cdiv(cdiv(m, p.ks), 16) * 16;
@@ -210,8 +216,10 @@ void gram_upper(const T* X, int64_t ldx, int m, int n, T* G, T* slices, int cap,
 // tiles), and this workgroup's part of ||E||_F^2 (off-diagonal entries
 // counted twice) into part.
 template <typename T>
-__global__ void __launch_bounds__(256) cq2_sum_up_kernel(const T* P, int ks, int n, T* E, T* U, double* part) {
+__global__ void __launch_bounds__(256) cq2_sum_up_kernel(const T* P, int ks, int n, T* E, T* U, double* part,
+                                                         const int* stop) {
   __shared__ double red[4];
+  if (*stop != 0) return;
   const int64_t tot = (int64_t)n * n;
   double dev = 0.0;
   for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < tot; e += (int64_t)gridDim.x * 256) {
@@ -268,7 +276,7 @@ __global__ void __launch_bounds__(256) sum_r_slices_kernel(const T* P, int ks, i
 // kLoCorrMaxE), else Q = Q1 W2^{-1} runs on FP64 MFMA (st[6]), as it does in any
 // case below the size where the others are faster;
 // st[4..5] = ||E||_F as a double.
-__global__ void cq2_decide_kernel(const double* part, int np, const int* cinfo, int lo_ok, int* st) {
+__global__ void cq2_decide_kernel(const double* part, int np, const int* cinfo, int lo_ok, int* st, const int* stop) {
   __shared__ double red[4];
   double acc = 0.0;
   for (int i = threadIdx.x; i < np; i += 256) acc += part[i];
@@ -277,7 +285,7 @@ __global__ void cq2_decide_kernel(const double* part, int np, const int* cinfo, 
   __syncthreads();
   if (threadIdx.x == 0) {
     const double e = sqrt(red[0] + red[1] + red[2] + red[3]);
-    const bool ok = (*cinfo == 0) && (e <= 1e-6);  // false for NaN
+    const bool ok = (*cinfo == 0) && (*stop == 0) && (e <= 1e-6);  // false for NaN
     st[0] = ok ? 1 : 0;
     st[1] = (ok && e > 1e-9) ? 1 : 0;
     st[7] = (ok && lo_ok && e <= kBf16CorrMaxE) ? 1 : 0;
@@ -331,13 +339,17 @@ __global__ void cq2_w_kernel(const T* U, const T* U2, const int* st, int n, T* W
   Wi[idx] = wi;
 }
 
-// *flag = 1 if the Cholesky succeeded and a column k of R is closer than 1 /
-// kRefineCond to the span of the others: ||R(:, k)|| ||X(k, :)|| > kRefineCond,
-// X = R^{-1}.  Sixteen columns a workgroup.
+// With d the largest ||R(:, k)|| ||X(k, :)||, X = R^{-1}, the inverse sine between
+// a column and the span of the others: st[8] = 1 for kRefineCond < d <=
+// kHopelessCond, 2 beyond, and then st[9] = 1.  st[9] = 1 also for a Cholesky that
+// failed (st[2]).  Sixteen columns a workgroup.
 template <typename T>
-__global__ void __launch_bounds__(256) cq2_cond_kernel(const T* R, const T* X, int n, const int* info, int* flag) {
+__global__ void __launch_bounds__(256) cq2_cond_kernel(const T* R, const T* X, int n, int* st) {
   __shared__ double cn[16], rn[16][17];
-  if (*info != 0) return;
+  if (st[2] != 0) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) st[9] = 1;
+    return;
+  }
   const int k0 = blockIdx.x * 16, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
   for (int c = w; c < 16; c += 4) {
@@ -350,13 +362,16 @@ __global__ void __launch_bounds__(256) cq2_cond_kernel(const T* R, const T* X, i
   const int kk = threadIdx.x & 15, g = threadIdx.x >> 4;
   double s = 0.0;
   if (k0 + kk < n)
+#pragma unroll 8
     for (int j = k0 + g; j < n; j += 16) s += s_abs2(X[k0 + kk + (int64_t)j * n]);
   rn[g][kk] = s;
   __syncthreads();
   if (threadIdx.x < 16 && k0 + kk < n) {
     double r = 0.0;
     for (int h = 0; h < 16; ++h) r += rn[h][kk];
-    if (cn[kk] * r > kRefineCond * kRefineCond) *flag = 1;  // every writer writes 1
+    const double d2 = cn[kk] * r;
+    if (d2 > kRefineCond * kRefineCond) atomicMax(st + 8, d2 > kHopelessCond * kHopelessCond ? 2 : 1);
+    if (!(d2 <= kHopelessCond * kHopelessCond)) st[9] = 1;  // every writer writes 1
   }
 }
 
@@ -380,33 +395,23 @@ bool cholqr2_eligible(int m, int n) { return m >= n && n >= 1 && n <= kCholTileM
 
 // Enqueues the whole-matrix CholeskyQR2 on s; Q (m x n) and R (n x n or null)
 // receive the factors when the device-side check accepts (status word at
-// cholqr2_status(ws): [0] = 1 accepted; its kCq2StatusWords are 0 on entry).  ws:
-// cholqr2_workspace_bytes(m, n).  lo: the correction may run on BF16 / FP32
+// cholqr2_status(ws): [0] = 1 accepted; its kCq2StatusWords are 0 on entry).
+// Two calls: cholqr2_enqueue to the decision, cholqr2_finish the rest, which a
+// caller that reads the status word between them leaves out for a rejected
+// input.  ws: cholqr2_workspace_bytes(m, n).  lo: the correction may run on BF16 / FP32
 // MFMA where that is faster (a call that documents it); else it runs on FP64
 // (8192 x 1024 Float64: 0.1 ms more), and Q1 is refined where R1 is ill conditioned.
 template <typename T>
-void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q, int64_t ldq, T* R, int64_t ldr,
-                     char* ws, bool lo) {
+void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q, int64_t ldq, char* ws, bool lo) {
   const CQ2Layout L = cq2_layout<T>(m, n);
   T* Q1 = reinterpret_cast<T*>(ws + L.offQ1);
   T* G = reinterpret_cast<T*>(ws + L.offG);   // G1, then R1
   T* E = reinterpret_cast<T*>(ws + L.offE);   // G2 = I + E
-  T* X = reinterpret_cast<T*>(ws + L.offX);   // X1 = R1^{-1}, then W2^{-1}
+  T* X = reinterpret_cast<T*>(ws + L.offX);   // X1 = R1^{-1}
   T* U = reinterpret_cast<T*>(ws + L.offU);
-  T* W = reinterpret_cast<T*>(ws + L.offW);
-  T* Tm = reinterpret_cast<T*>(ws + L.offT);
-  T* Sl = reinterpret_cast<T*>(ws + L.offSl);
   int* flags = reinterpret_cast<int*>(ws + L.offFlags);
   double* part = reinterpret_cast<double*>(ws + L.offPart);
   int* st = reinterpret_cast<int*>(ws + L.offSt);
-  const int64_t nn = (int64_t)n * n;
-  const unsigned eg = (unsigned)cdiv64(nn, 256);
-  // Below about 1e9 (complex 5e8) multiply-adds the packing and launches of the
-  // low-precision correction cost more than it saves.  The call, us, low / FP64:
-  // Float64 100 x 64 157 / 135, 1024 x 256 257 / 235, 1501 x 777 630 / 634, 2048 x 1024
-  // 766 / 783, 8192 x 1024 1070 / 1170; ComplexF64 700 x 64 221 / 156, 1024 x 256 404 /
-  // 347, 3001 x 333 627 / 599, 1501 x 777 1090 / 1180, 4096 x 1024 1710 / 1910.
-  const bool low = lo && (double)m * (double)nn >= (ScalarTraits<T>::is_complex ? 5e8 : 1e9);
   // pass 1: Q1 = A X1 inside the Cholesky launch, column block by column
   // block as X1 becomes final
   gram_upper<T>(A, lda, m, n, G, X, L.kcap, s);
@@ -419,8 +424,8 @@ void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q,
   // and 7e-16 of ||A||).  So a call that the panels served before: Q1 += (A - Q1
   // R1) X1 where R1 is ill conditioned, Q serving as scratch (2 x 2 m n^2 flops).
   if (!lo) {
-    int* flag = st + 8;
-    hipLaunchKernelGGL((cq2_cond_kernel<T>), dim3(cdiv(n, 16)), dim3(256), 0, s, G, X, n, st + 2, flag);
+    const int* flag = st + 8;
+    hipLaunchKernelGGL((cq2_cond_kernel<T>), dim3(cdiv(n, 16)), dim3(256), 0, s, G, X, n, st);
     hipLaunchKernelGGL((cq2_copy_kernel<T>), dim3(std::min(cdiv(m, 256), 16), n), dim3(256), 0, s, A, lda, m, Q, ldq,
                        flag);
     gemm<T>(OP_N, OP_N, gq<T>(m, n, n, Q1, m, G, n, Q, ldq, -1.0, 1.0, TRI_B_UPPER, flag, 1), s);
@@ -428,9 +433,32 @@ void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q,
   }
   // pass 2: G2 = I + E (slices summed with U1 = up(E) and ||E||_F in one
   // sweep), the decision, and W2, W2^{-1} in closed form
-  const int ks2 = gram_upper_slices<T>(Q1, m, m, n, X, L.kcap, s);
-  hipLaunchKernelGGL((cq2_sum_up_kernel<T>), dim3(kRedWgs), dim3(256), 0, s, X, ks2, n, E, U, part);
-  hipLaunchKernelGGL(cq2_decide_kernel, dim3(1), dim3(256), 0, s, part, kRedWgs, st + 2, lo ? 1 : 0, st);
+  const int* stop = lo ? st + 2 : st + 9;
+  const int ks2 = gram_upper_slices<T>(Q1, m, m, n, X, L.kcap, s, stop);
+  hipLaunchKernelGGL((cq2_sum_up_kernel<T>), dim3(kRedWgs), dim3(256), 0, s, X, ks2, n, E, U, part, stop);
+  hipLaunchKernelGGL(cq2_decide_kernel, dim3(1), dim3(256), 0, s, part, kRedWgs, st + 2, lo ? 1 : 0, st, stop);
+}
+
+template <typename T>
+void cholqr2_finish(hipStream_t s, int m, int n, T* Q, int64_t ldq, T* R, int64_t ldr, char* ws, bool lo) {
+  const CQ2Layout L = cq2_layout<T>(m, n);
+  T* Q1 = reinterpret_cast<T*>(ws + L.offQ1);
+  T* G = reinterpret_cast<T*>(ws + L.offG);   // R1
+  T* E = reinterpret_cast<T*>(ws + L.offE);   // I + E
+  T* X = reinterpret_cast<T*>(ws + L.offX);   // W2^{-1}
+  T* U = reinterpret_cast<T*>(ws + L.offU);
+  T* W = reinterpret_cast<T*>(ws + L.offW);
+  T* Tm = reinterpret_cast<T*>(ws + L.offT);
+  T* Sl = reinterpret_cast<T*>(ws + L.offSl);
+  int* st = reinterpret_cast<int*>(ws + L.offSt);
+  const int64_t nn = (int64_t)n * n;
+  const unsigned eg = (unsigned)cdiv64(nn, 256);
+  // Below about 1e9 (complex 5e8) multiply-adds the packing and launches of the
+  // low-precision correction cost more than it saves.  The call, us, low / FP64:
+  // Float64 100 x 64 157 / 135, 1024 x 256 257 / 235, 1501 x 777 630 / 634, 2048 x 1024
+  // 766 / 783, 8192 x 1024 1070 / 1170; ComplexF64 700 x 64 221 / 156, 1024 x 256 404 /
+  // 347, 3001 x 333 627 / 599, 1501 x 777 1090 / 1180, 4096 x 1024 1710 / 1910.
+  const bool low = lo && (double)m * (double)nn >= (ScalarTraits<T>::is_complex ? 5e8 : 1e9);
   // second order (st[1] == 1): U = up(E - U1^H U1), U2 = U U
   {
     GemmArgs g = gq<T>(n, n, n, U, n, U, n, Tm, n, 1.0, 0.0, TRI_A_LOWER | TRI_B_UPPER, st + 1, 1);
@@ -500,9 +528,12 @@ template <typename T> Cholqr2Buffers<T> cholqr2_buffers(char* ws, int m, int n) 
 
 template size_t cholqr2_workspace_bytes<double>(int, int);
 template size_t cholqr2_workspace_bytes<zd>(int, int);
-template void cholqr2_enqueue<double>(hipStream_t, int, int, const double*, int64_t, double*, int64_t, double*,
-                                      int64_t, char*, bool);
-template void cholqr2_enqueue<zd>(hipStream_t, int, int, const zd*, int64_t, zd*, int64_t, zd*, int64_t, char*, bool);
+#define MAK_CQ2_INSTANTIATE(T)                                                                                  \
+  template void cholqr2_enqueue<T>(hipStream_t, int, int, const T*, int64_t, T*, int64_t, char*, bool);        \
+  template void cholqr2_finish<T>(hipStream_t, int, int, T*, int64_t, T*, int64_t, char*, bool);
+MAK_CQ2_INSTANTIATE(double)
+MAK_CQ2_INSTANTIATE(zd)
+#undef MAK_CQ2_INSTANTIATE
 template int* cholqr2_status<double>(char*, int, int);
 template int* cholqr2_status<zd>(char*, int, int);
 template Cholqr2Buffers<double> cholqr2_buffers<double>(char*, int, int);

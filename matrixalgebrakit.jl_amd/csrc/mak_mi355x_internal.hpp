@@ -58,18 +58,19 @@ int cholqr_gram_blocks(int H);
 void zero_ints(int* p, int n, hipStream_t s);
 void zero_ints2(int* p, int n, int* q, int m, hipStream_t s);  // n, m <= 64, one launch
 
-// Whole-matrix CholeskyQR2 for qr_compact!(positive = true) (mak_cholqr2.hip):
-// eligible for m >= n, n <= kCholTileMaxN.  cholqr2_enqueue reads A only and
-// writes Q / R (R may be null) when the device-side check accepts; the status
-// word (cholqr2_status: [0] = 1 accepted, [2] Cholesky info, [4..5] ||E||_F
-// as a double) is valid once the stream reaches it.  cholqr2_scratch: its
-// m x n scratch (free after the call; the in-place Q mode reuses it).
-constexpr int kCq2StatusWords = 9;
+// Whole-matrix CholeskyQR2 (mak_cholqr2.hip): eligible for m >= n, n <=
+// kCholTileMaxN.  cholqr2_enqueue and cholqr2_finish read A only and write Q / R
+// (R may be null) when the device-side check accepts; the status word
+// (cholqr2_status: [0] = 1 accepted, [2] Cholesky info, [4..5] ||E||_F as a
+// double) is valid once the stream has passed the first.  cholqr2_scratch: its
+// m x n scratch (free after the calls; the in-place Q mode reuses it).
+constexpr int kCq2StatusWords = 10;
 bool cholqr2_eligible(int m, int n);
 template <typename T> size_t cholqr2_workspace_bytes(int m, int n);
 template <typename T>
-void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q, int64_t ldq, T* R, int64_t ldr,
-                     char* ws, bool lo);
+void cholqr2_enqueue(hipStream_t s, int m, int n, const T* A, int64_t lda, T* Q, int64_t ldq, char* ws, bool lo);
+template <typename T>
+void cholqr2_finish(hipStream_t s, int m, int n, T* Q, int64_t ldq, T* R, int64_t ldr, char* ws, bool lo);
 template <typename T> int* cholqr2_status(char* ws, int m, int n);
 template <typename T> T* cholqr2_scratch(char* ws, int m, int n);
 // Workspace of a cholqr2_enqueue call that is free once its launches are
@@ -81,7 +82,7 @@ template <typename T> struct Cholqr2Buffers {
 template <typename T> Cholqr2Buffers<T> cholqr2_buffers(char* ws, int m, int n);
 
 // The Householder QR's signs and trailing columns from the CholeskyQR2
-// factors (mak_qtrail.hip), enqueued after cholqr2_enqueue with its workspace.
+// factors (mak_qtrail.hip), enqueued after cholqr2_finish with its workspace.
 template <typename T>
 void qr_trailing_enqueue(hipStream_t s, int m, int n, T* Q, int64_t ldq, T* R, int64_t ldr, int full, int positive,
                          char* cw);

@@ -653,12 +653,24 @@ int qr_driver(hipStream_t s, int full, int m, int n, T* A, int64_t lda, T* Q, in
                      (!signs || (m > n && (!ScalarTraits<T>::is_complex || m - (n - 1) / NB * NB >= kCholQrMinRows)));
   if (whole) {
     char* cw = ws + L.offCq2;
-    cholqr2_enqueue<T>(s, m, n, A, lda, Qd, ldqd, R, ldr, cw, !signs);
-    if (signs) qr_trailing_enqueue<T>(s, m, n, Qd, ldqd, R, ldr, full, positive, cw);
     int st = 0;
-    if (hipMemcpyAsync(&st, cholqr2_status<T>(cw, m, n), sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess)
-      return 1;
+    auto accepted = [&]() {
+      return hipMemcpyAsync(&st, cholqr2_status<T>(cw, m, n), sizeof(int), hipMemcpyDeviceToHost, s) == hipSuccess &&
+             hipStreamSynchronize(s) == hipSuccess;
+    };
+    cholqr2_enqueue<T>(s, m, n, A, lda, Qd, ldqd, cw, !signs);
+    // With signs the decision is read before the rest (about forty launches at n =
+    // 1024), which a rejected input then does without; the rest is not waited for.
+    if (signs) {
+      if (!accepted()) return 1;
+      if (st == 1) {
+        cholqr2_finish<T>(s, m, n, Qd, ldqd, R, ldr, cw, false);
+        qr_trailing_enqueue<T>(s, m, n, Qd, ldqd, R, ldr, full, positive, cw);
+      }
+    } else {
+      cholqr2_finish<T>(s, m, n, Qd, ldqd, R, ldr, cw, true);
+      if (!accepted()) return 1;
+    }
     if (st == 1) {
       if (inplace) copy_mat<T>(m, qcols, Qd, ldqd, Q, ldq, s);
       return hipGetLastError() == hipSuccess ? 0 : 1;

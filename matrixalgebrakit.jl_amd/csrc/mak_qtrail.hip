@@ -292,7 +292,7 @@ GemmArgs gated(int M, int N, int K, const T* A, int64_t lda, const T* B, int64_t
 
 }  // namespace
 
-// After cholqr2_enqueue (same stream, its workspace cw): Q (m x m when full,
+// After cholqr2_finish (same stream, its workspace cw): Q (m x m when full,
 // else m x n) and R (m x n when full, else n x n, or null) of the Householder
 // QR, with the positive gauge or without; runs only where the CholeskyQR2
 // result was accepted.  m > n unless positive; n >= 64 (the buffers of
