@@ -337,6 +337,11 @@ int mak_left_polar_pullback_z(void* stream, int batch, int m, int n, const void*
 typedef struct mak_qr_batched_plan mak_qr_batched_plan;
 
 int mak_qr_batched_workspace_size(int dtype, int count, const int* m, const int* n, int tune, size_t* bytes);
+/* The same for a given `positive`: a plan without the gauge has no whole blocks
+ * and needs far less.  A positive plan accepts the size for positive = 0 too;
+ * where the whole blocks' scratch does not fit, every block runs on panels. */
+int mak_qr_batched_plan_workspace_size(int dtype, int count, const int* m, const int* n, int positive, int tune,
+                                       size_t* bytes);
 int mak_qr_batched_plan_create(mak_qr_batched_plan** plan, int dtype, int count, const int* m, const int* n,
                                void* const* A, const int* lda, void* const* Q, const int* ldq, void* const* R,
                                const int* ldr, int positive, int tune, void* work, size_t work_bytes);

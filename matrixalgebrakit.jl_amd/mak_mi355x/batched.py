@@ -4,8 +4,8 @@ The reference has no batched API; a tensor-network caller loops
 ``qr_compact!`` over its blocks (src/implementations/qr.jl:110-113 per
 block).  :class:`BatchedQRPlan` runs all blocks through one captured hipGraph
 (``mak_qr_batched_plan_create`` / ``mak_qr_batched_execute``); every block
-gets exactly what ``qr_compact!(A_i, (Q_i, R_i), Householder(; positive))``
-gives it, and ``A_i`` is overwritten like the single-matrix call.
+gets what ``qr_compact!(A_i, (Q_i, R_i), Householder(; positive))`` gives it,
+and the contents of ``A_i`` are undefined afterwards.
 """
 from __future__ import annotations
 
@@ -79,8 +79,9 @@ class BatchedQRPlan:
         self._lib = lib
         dt = _DT[dtype]
         nbytes = C.c_size_t(0)
-        _status(lib.mak_qr_batched_workspace_size(dt, cnt, self._m, self._n, int(tune), C.byref(nbytes)),
-                "mak_qr_batched_workspace_size")
+        _status(lib.mak_qr_batched_plan_workspace_size(dt, cnt, self._m, self._n, int(bool(alg.positive)), int(tune),
+                                                       C.byref(nbytes)),
+                "mak_qr_batched_plan_workspace_size")
         self._ws = _workspace(dev, nbytes.value)
         torch.cuda.synchronize(dev)
         h = C.c_void_p(None)
