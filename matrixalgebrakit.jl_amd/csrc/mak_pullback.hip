@@ -525,12 +525,17 @@ __global__ void __launch_bounds__(256) bcayley_kernel(int n, T* G, T* M, const d
   M[o] = s_sub(idx % n == idx / n ? s_one(T()) : s_zero(T()), v);
 }
 
-// Largest tr(P) tr(P^{-1}) / n^2 (1 for P = c I; at least kappa(P) / n^2, and
-// kappa / n for one small eigenvalue) that takes the doubling solver: up to it
-// the steps stay below kDoublingMax and Gauss-Jordan without pivoting loses
-// nothing against Cholesky.  A tall Gaussian matrix of 2 n rows has 1.6.
-constexpr double kDoublingMaxCond = 16.0;
-constexpr int kDoublingMax = 16;
+// The quotient q = tr(P) tr(P^{-1}) / n^2 (1 for P = c I; a tall Gaussian matrix
+// of 2 n rows has 1.6) decides on the doubling solver.  P / s has its eigenvalues
+// in [1 / (n q), n], so |M| <= 1 - 2 / (n q + 1), and the stop test, n^2
+// |M|^(2^(K+1)) <= kDoublingRem, holds after at most kDoublingMax steps for n q up
+// to kDoublingMaxSpread: a batch that is taken is finished by it, at a third of
+// the products of CG and the eigendecomposition at worst.  q alone allows a
+// condition number of 16 n for one small eigenvalue and of 16 n^2 for one large
+// and one small one; error and residual there stay those of the
+// eigendecomposition (u times the condition number).
+constexpr double kDoublingMaxCond = 16.0, kDoublingMaxSpread = 16384.0;
+constexpr int kDoublingMax = 18;
 // Relative remainder |M^(2^K)|^2 after K steps, bounded by |M^(2^(K-1))|_F^4.
 constexpr double kDoublingRem = 1e-17;
 constexpr double kDoublingMinTol = 1e-15;  // requests below it keep the CG path's own test
@@ -600,7 +605,7 @@ int polar_pullback_doubling(hipStream_t s, int batch, int m, int n, const T* W, 
     return 2;
   if (hinfo != 0) return 1;
   for (int b = 0; b < batch; ++b)
-    if (!(h[b] > 0.0) || !(h[b] * h[batch + b] <= kDoublingMaxCond)) return 1;
+    if (!(h[b] > 0.0) || !(h[b] * h[batch + b] <= std::min(kDoublingMaxCond, kDoublingMaxSpread / n))) return 1;
   hipLaunchKernelGGL((bskew_scaled_kernel<T>), dim3(cdiv(n, 32), cdiv(n, 32), batch), dim3(256), 0, s, n, K,
                      dP ? (const T*)Tm : nullptr, (const double*)shift, F);
   hipLaunchKernelGGL((bcayley_kernel<T>), gnn, dim3(256), 0, s, n, N, Ma, (const double*)shift);
