@@ -66,10 +66,13 @@ int mak_qr_workspace_size(int dtype, int full, int m, int n, size_t* bytes);
  * A (m x n) is destroyed (its contents are undefined afterwards),
  * Q is m x min(m,n), R is min(m,n) x n or NULL (R not computed).
  * positive != 0 gives R a real non-negative diagonal (gauge fix).
- * The factors are FP64-accurate; on the whole-matrix CholeskyQR2 path the
- * final correction term Q1 (W2^{-1} - I), of norm ~ ||Q1^H Q1 - I||, runs on
- * BF16 (that norm <= 5e-14) or FP32 (<= 1e-10) MFMA with an error bound below
- * Q's own FP64 rounding, else on FP64.
+ * The factors are FP64-accurate; with positive != 0 the final correction term
+ * Q1 (W2^{-1} - I) of the whole-matrix CholeskyQR2 path (m n^2 >= 1e9, complex
+ * 5e8), of norm ~ ||Q1^H Q1 - I||, runs on BF16 (that norm <= 5e-14) or FP32
+ * (<= 1e-10) MFMA with an error bound below Q's own FP64 rounding, else on FP64.
+ * That path's Q1 = A R1^{-1} is formed with the computed inverse: ||A - Q R|| is up
+ * to about u cond(A) ||A|| for condition numbers to 1e5, beyond which Householder
+ * panels take over.  positive = 0 and qr_full! run on FP64 and refine Q1.
  * Replaces qr_compact!(A, QR, ::Householder) -> qr_householder!
  * (src/implementations/qr.jl:110-113, :132-188). */
 int mak_qr_compact_d(void* stream, int m, int n, double* A, int lda, double* Q, int ldq, double* R, int ldr,

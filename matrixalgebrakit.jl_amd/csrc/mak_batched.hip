@@ -10,10 +10,11 @@
 // (32-column panels, compact WY, backward orgqr, positive gauge), the panel
 // steps of all problems together and every task of a whole block gated on its
 // rejection.  Measured, m log-uniform in [16, 1024], n uniform in [8, m]: 4096
-// Float64 blocks 33.6 ms on panels alone, 18.5 ms; 1024 ComplexF64 blocks 24.6
-// and 14.0 ms.  The gated launches cost 0.5 ms of that when nothing is
-// rejected; a set whose blocks are nearly all rejected pays the attempt (1024
-// Float64 blocks beyond condition 1e7: 12.2 -> 14.2 ms).
+// Float64 blocks 33.6 ms on panels alone, 19.0 ms (20 where a block's E asks for
+// the second pass); 1024 ComplexF64 blocks 24.6 and 14.7 ms.  The gated launches
+// cost 0.6 ms of that when nothing is rejected; a set whose blocks are nearly all
+// rejected pays the attempt (condition 1e9: 1024 Float64 blocks 12.6 -> 14.1 ms,
+// 256 ComplexF64 12.9 -> 14.7 ms).
 //
 // The panel schedule:
 //   for panel step s: one node launch per row-size class factors panel s of

@@ -29,10 +29,11 @@
 // and wrote the trailing matrix once per 32 columns.
 // Tasks are listed so that a block stays on one XCD (workgroup b runs on XCD
 // b mod 8), whose L2 then serves the operands that its tiles share.
-// 4096 Float64 blocks (m log-uniform in [16, 1024], n uniform in [8, m]; 2743 of
-// them whole): Gram 3.0 ms each (51 TF/s of the padded tiles), factor 2.1, solve
-// 3.8, correct 5.0 ms; 1024 ComplexF64: 2.4, 2.5, 2.7 and 2.9 ms; the panel
-// schedule took 33.6 and 24.6 ms in all.
+// 4096 blocks (m log-uniform in [16, 1024], n uniform in [8, m]; 2743 of them
+// whole): Float64 Gram 3.1 ms each (49 TF/s of the padded tiles), factor 2.6, solve
+// 4.2, correct 5.5 ms; ComplexF64 8.7 each, 7.1, 11.0 and 13.0 ms.  All of a call,
+// Float64 33.6 ms on the panel schedule, 19.0 here; 1024 ComplexF64 blocks 24.6
+// and 14.7.
 #include <algorithm>
 
 #include "mak_common.hpp"
@@ -725,8 +726,8 @@ __global__ void __launch_bounds__(256, BcCfg<T>::OCC)
 // Products with a factor on the right belong to one wave per 16 rows and need
 // no workgroup barrier.  What bounds it: latency of the two 32 x 32 in-wave
 // Choleskys (3 us each Float64) and of the ~10 steps between barriers.
-// 57 x 33 Float64: 29.5 us, the call 31 us against 131 us as 22 launches; an
-// input of condition 1e9 128 us.
+// 57 x 33 Float64: the call 32 us against 131 us as 22 launches; with its copy of A
+// 55 against 163 us, of condition 1e9 152 against 163 us.
 // ---------------------------------------------------------------------------
 constexpr int SP = 65;  // pitch of As
 
@@ -1006,7 +1007,7 @@ __global__ void __launch_bounds__(256) qr_small_kernel(const T* A, int64_t lda, 
 
 // ---------------------------------------------------------------------------
 // One matrix with m >= 64 rows and n < 64 columns: CholeskyQR2 in three
-// launches.  Workgroup s has rows s rps ..; the last one of a launch to finish
+// launches, after a small one that clears their control words.  Workgroup s has rows s rps ..; the last one of a launch to finish
 // sums the partial Gram matrices in order and does the 64 x 64 work:
 //   0  partial A^H A;            R1 (W), R1^{-1} (X)
 //   1  Q1 = A R1^{-1}, partial Q1^H Q1;   U, D = (I + U)^{-1} - I, R = (I + U) R1

@@ -1,4 +1,5 @@
-// Whole-matrix CholeskyQR2 for qr_compact!(A, (Q, R); positive = true), m >= n
+// Whole-matrix CholeskyQR2 for qr_compact!(A, (Q, R); positive = true), m >= n,
+// and the start of qr_full! and positive = false, which mak_qtrail.hip finishes
 // (the result is the unique QR factorisation with a positive real diagonal of
 // R, the one MatrixAlgebraKit's qr_householder! + gaugefix! returns,
 // src/implementations/qr.jl:132-188, src/common/gauge.jl:16-25):
@@ -15,6 +16,8 @@
 //        1e-18 and U = U1, W2^{-1} = I - U are taken directly)
 //   Q = Q1 W2^{-1},  R = W2 R1
 //
+// For qr_full! and positive = false, Q1 is refined where R1 is ill conditioned
+// and every product runs on FP64.
 // The call is accepted on the device when the Cholesky factorisation
 // succeeded and ||E||_F <= 1e-6: then kappa(Q1) <= 1 + 1e-6 and Q is
 // orthonormal to working precision (Yamamoto, Nakatsukasa, Yanagisawa,

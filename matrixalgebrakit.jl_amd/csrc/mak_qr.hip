@@ -72,12 +72,13 @@ template <typename T> TreePlan plan_tree(int H, int nbc, size_t base) {
 constexpr int kCholQrMinRows = 64;
 // Columns from which the whole-matrix CholeskyQR2 path is tried first.
 constexpr int kCholQr2MinN = 64;
-// Rows up to which narrower matrices take the three-launch CholeskyQR2: one
+// Rows up to which narrower matrices take CholeskyQR2 in three launches: one
 // workgroup sums its partial Gram matrices, and 64 workgroups do not fill the
-// chip.  Against the panels (us a call): 1024 x 32 Float64 164 -> 93,
-// 8192 x 63 310 -> 179, 8192 x 32 177 -> 127; 32768 x 32 230 -> 216 and ComplexF64
-// 385 -> 398, 131072 x 16 383 -> 439.  An input that it rejects (||E||_F > 1e-6,
-// condition numbers from about 1e5) pays the attempt: 512 x 32 201 -> 266.
+// chip.  Against the panels (us a call, with its copy of A): 1024 x 32 Float64 164
+// -> 99, 8192 x 63 316 -> 188, 16384 x 32 196 -> 163, ComplexF64 1024 x 48 418 -> 157;
+// beyond (the call alone) 32768 x 32 230 -> 216 and ComplexF64 385 -> 398, 131072 x
+// 16 383 -> 439.  An input that it rejects (||E||_F > 1e-6, condition numbers from
+// about 1e5) pays the attempt: 512 x 32 230 -> 281.
 constexpr int kTallMaxM = 1 << 14;
 
 template <typename T> struct QrLayout {
@@ -616,8 +617,9 @@ int qr_driver(hipStream_t s, int full, int m, int n, T* A, int64_t lda, T* Q, in
   }
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &cs) != hipSuccess) cs = hipStreamCaptureStatusActive;
-  // m >= 64 > n: CholeskyQR2 in three launches, each summing its partial Gram
-  // matrices in its last workgroup (8 to 10 launches on panels)
+  // m >= 64 > n: CholeskyQR2 in three launches (and one that clears their control
+  // words), two of them summing their partial Gram matrices in the last workgroup
+  // (8 to 10 launches on panels)
   if (!full && positive && Tout == nullptr && n > 0 && n < kCholQr2MinN && m >= kCholQrMinRows && m <= kTallMaxM &&
       std::max(lda, ldq) <= (1 << 20) && (int64_t)L.wpElems >= kTallScratchElems &&
       cs == hipStreamCaptureStatusNone) {

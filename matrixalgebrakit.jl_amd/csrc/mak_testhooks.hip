@@ -61,8 +61,8 @@ int maktest_gemm_prec(void* stream, int prec, int opA, int opB, int M, int N, in
 // first 32-column panel handed to Householder TSQR (-1: none), out[2] the
 // whole-matrix path's Cholesky info, out[3] 1 when that path exists for the
 // shape, out[4..5] its ||Q1^H Q1 - I||_F (a double), out[6 / 7 / 8] 1 when
-// its final product took the FP32 correction / ran on FP64 / took the BF16
-// correction (nine ints).
+// that norm allows its final product the FP32 correction / FP64 only / the BF16
+// correction, which large matrices of qr_compact! take (nine ints).
 int maktest_qr_record(int dtype, int full, int m, int n, const void* work, int* out) {
   if (dtype == MAK_F64) mak::qr_record<double>((const char*)work, m, n, full, out);
   else mak::qr_record<mak::zd>((const char*)work, m, n, full, out);
