@@ -9,8 +9,10 @@
 // kept in g_scratch_ptr.  Every call on a GPU shares that GPU's array and
 // finds it as the previous call left it; the QR driver clears what must start
 // at zero (status words, flags) with kernels at the start of each call, as it
-// does for a caller's workspace.  Calls that overlap on one GPU (two streams,
-// two threads) race on the array: the caller serialises them.
+// does for a caller's workspace.  A call outside of a capture returns when its
+// kernels have ended, so calls one after the other may use different streams;
+// calls that overlap on one GPU (two threads, graph replays) race on the array:
+// the caller serialises them.
 #include <mutex>
 
 #include "mak_common.hpp"
@@ -62,8 +64,16 @@ int mak_qr_compact_noalloc_d(void* s, int m, int n, double* A, int lda, double* 
   if (mak::qr_workspace_bytes<double>(m, n, 0) > mak::kScratchBytes) return 7;  // beyond the static scratch
   void* ws = mak::scratch_on((hipStream_t)s);
   if (ws == nullptr) return 1;
-  return mak::qr_driver<double>((hipStream_t)s, 0, m, n, A, lda, Q, ldq, R, ldr, positive, ws, mak::kScratchBytes,
-                                nullptr);
+  const int st = mak::qr_driver<double>((hipStream_t)s, 0, m, n, A, lda, Q, ldq, R, ldr, positive, ws,
+                                        mak::kScratchBytes, nullptr);
+  // Some paths return before their kernels have ended; a next call on another
+  // stream finds the array free all the same.  (Under capture the caller orders
+  // the replays.)
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)s, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone &&
+      hipStreamSynchronize((hipStream_t)s) != hipSuccess)
+    return 1;
+  return st;
 }
 
 }  // extern "C"
